@@ -61,7 +61,8 @@ constexpr size_t kSideStreams = 4;           // hardware queues of one process
 // One launch of the LDS-resident kernel: the instances of circuits whose
 // LDS footprints are within a factor of each other.
 struct LdsClass {
-    int32_t nr = 1, nblocks = 0, n_inst = 0;
+    int32_t nr = 1, n_inst = 0;
+    bool dyn = false;                          // some source is not DC
     size_t lds = 0;
     LdsArgs args{};
 };
@@ -79,10 +80,16 @@ struct Batch {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double last_ms = 0.0;
     int32_t kernel = CS_BATCH_KERNEL_GLOBAL;   // which kernel runs this batch
-    std::vector<LdsClass> classes;             // LDS-resident kernel: one launch each
+    std::vector<LdsClass> classes;             // adjoint: one launch each
     std::vector<hipEvent_t> class_ev;
     int32_t* d_queues = nullptr;
-    LdsClass pack;                             // the packed launch of the transient
+    // the packed launch of the transient
+    PackShape pack;
+    int32_t pack_blocks = 0;
+    size_t pack_lds = 0;
+    LdsArgs pack_args{};
+    const LdsArgs* d_pack_args = nullptr;
+    std::vector<int32_t> used, c_nr;           // circuits of the batch; rows per lane by circuit id
 };
 
 }  // namespace
@@ -138,20 +145,21 @@ struct Packer {
 // keeps compact_ok = false and runs on the global-plan kernel.
 int upload_compact(cs_ctx* ctx, Circuit& C) {
     std::vector<uint16_t> blob;
-    std::vector<int32_t> colnat, diffrow, probe, dev, devrow;
+    std::vector<int32_t> lpos, colnat, diffrow, probe, dev, devrow;
     const char* why = "";
     CPlan cp{};
     if (C.cbuf) { (void)hipFree(C.cbuf); C.cbuf = nullptr; }
-    C.compact_ok = build_compact(C.plan, blob, cp, colnat, diffrow, probe, dev, devrow, &why);
+    C.compact_ok = build_compact(C.plan, blob, cp, lpos, colnat, diffrow, probe, dev, devrow, &why);
     C.compact_why = why;
     if (!C.compact_ok) return CS_OK;
     Packer pk;
-    size_t o_blob = pk.add(blob), o_cn = pk.add(colnat), o_df = pk.add(diffrow), o_pr = pk.add(probe),
+    size_t o_blob = pk.add(blob), o_lp = pk.add(lpos), o_cn = pk.add(colnat), o_df = pk.add(diffrow), o_pr = pk.add(probe),
            o_dev = pk.add(dev), o_dr = pk.add(devrow);
     HIPCHK(ctx, hipMalloc(&C.cbuf, pk.bytes.size()));
     HIPCHK(ctx, hipMemcpy(C.cbuf, pk.bytes.data(), pk.bytes.size(), hipMemcpyHostToDevice));
     char* b = (char*)C.cbuf;
     cp.blob = (const uint16_t*)(b + o_blob);
+    cp.lpos = (const int32_t*)(b + o_lp);
     cp.colnat = (const int32_t*)(b + o_cn);
     cp.diffrow = (const int32_t*)(b + o_df);
     cp.probe = (const int32_t*)(b + o_pr);
@@ -500,10 +508,10 @@ int cs_pack_plan(int32_t n_circ, const cs_netlist* const* nls, const int32_t* co
         std::string err;
         if (!nls[c] || counts[c] < 0 || build_plan(nls[c], P, err) != CS_OK) return CS_E_INVALID;
         std::vector<uint16_t> blob;
-        std::vector<int32_t> a, b, d, e, f;
+        std::vector<int32_t> a, b, d, e, f, g;
         CPlan cp{};
         const char* why = "";
-        if (!build_compact(P, blob, cp, a, b, d, e, f, &why)) return CS_E_INVALID;
+        if (!build_compact(P, blob, cp, a, b, d, e, f, g, &why)) return CS_E_INVALID;
         img[c] = 2 * (size_t)((cp.words + 7) & ~7);
         dblb[c] = 8 * (size_t)((cp.dbl + 1) & ~1);
         dbl[c] = cp.dbl;
@@ -1268,33 +1276,62 @@ int cs_tran_sens(cs_ctx* ctx, int32_t cid, const double* p, const double* u0, co
     return rc;
 }
 
-// Size classes of the LDS-resident kernel.  Circuits are sorted by LDS
-// footprint; a class takes circuits down to 3/4 of its largest footprint, so
-// small circuits are not launched with the largest circuit's LDS reservation.
-// Each class is one persistent launch with its own largest-first queue.
-static int build_lds_classes(cs_ctx* ctx, Batch& B, const std::vector<int32_t>& used,
-                             const std::vector<int32_t>& c_nr, const std::vector<size_t>& c_need,
-                             const std::function<int(void**, size_t)>& dalloc) {
-    std::vector<int32_t> cs = used;
-    std::stable_sort(cs.begin(), cs.end(), [&](int32_t a, int32_t b) { return c_need[a] > c_need[b]; });
-    std::vector<int32_t> cls_of(ctx->circuits.size(), -1);
-    std::vector<std::vector<int32_t>> members;
-    for (size_t q = 0; q < cs.size();) {
-        const size_t cap = c_need[cs[q]];
-        std::vector<int32_t> m;
-        while (q < cs.size() && 4 * c_need[cs[q]] >= 3 * cap) m.push_back(cs[q++]);
-        for (int32_t c : m) cls_of[c] = (int32_t)members.size();
-        members.push_back(m);
-    }
+static bool has_dynamic_source(const Plan& P) {
+    for (const SrcDesc& d : P.src)
+        if (d.kind != CS_WAVE_DC) return true;
+    return false;
+}
+
+// The arguments every LDS-resident launch of a batch shares.
+static int lds_base_args(cs_ctx* ctx, const Batch& B, const std::function<int(void**, size_t)>& dalloc, LdsArgs& a) {
     std::vector<CPlan> cplans(ctx->circuits.size());
     for (size_t c = 0; c < ctx->circuits.size(); c++)
         if (ctx->circuits[c] && ctx->circuits[c]->compact_ok) cplans[c] = ctx->circuits[c]->hcp;
-    void *d_cp = nullptr, *d_q = nullptr;
+    void* d_cp = nullptr;
     int rc;
-    if ((rc = dalloc(&d_cp, sizeof(CPlan) * cplans.size())) ||
-        (rc = dalloc(&d_q, sizeof(int32_t) * members.size())))
-        return rc;
+    if ((rc = dalloc(&d_cp, sizeof(CPlan) * cplans.size()))) return rc;
     HIPCHK(ctx, hipMemcpy(d_cp, cplans.data(), sizeof(CPlan) * cplans.size(), hipMemcpyHostToDevice));
+    const BatchArgs& g = B.args;
+    a = LdsArgs{};
+    a.cplans = (const CPlan*)d_cp;
+    a.plans = g.plans;
+    a.inst_cid = g.inst_cid;
+    a.p_off = g.p_off;
+    a.params = g.params;
+    a.u_off = g.u_off;
+    a.u0 = g.u0;
+    a.w_off = g.w_off;
+    a.wave = g.wave;
+    a.u_final = g.u_final;
+    a.stats = g.stats;
+    a.o = g.o;
+    return CS_OK;
+}
+
+// Size classes of the adjoint.  Circuits are sorted by LDS footprint; a class
+// takes circuits down to 3/4 of its largest footprint, so small circuits are
+// not launched with the largest circuit's LDS reservation.  Each class is one
+// persistent launch with its own largest-first queue.
+static int build_lds_classes(cs_ctx* ctx, Batch& B, const std::function<int(void**, size_t)>& dalloc) {
+    auto need = [&](int32_t c) {
+        const CPlan& cp = ctx->circuits[c]->hcp;
+        return lds_kernel_bytes((cp.dbl + 1) & ~1, cp.words_adj);
+    };
+    std::vector<int32_t> cs = B.used;
+    std::stable_sort(cs.begin(), cs.end(), [&](int32_t a, int32_t b) { return need(a) > need(b); });
+    std::vector<int32_t> cls_of(ctx->circuits.size(), -1);
+    std::vector<std::vector<int32_t>> members;
+    for (size_t q = 0; q < cs.size();) {
+        const size_t cap = need(cs[q]);
+        std::vector<int32_t> m;
+        while (q < cs.size() && 4 * need(cs[q]) >= 3 * cap) m.push_back(cs[q++]);
+        for (int32_t c : m) cls_of[c] = (int32_t)members.size();
+        members.push_back(m);
+    }
+    LdsArgs base{};
+    void* d_q = nullptr;
+    int rc;
+    if ((rc = lds_base_args(ctx, B, dalloc, base)) || (rc = dalloc(&d_q, sizeof(int32_t) * members.size()))) return rc;
     B.d_queues = (int32_t*)d_q;
     for (size_t k = 0; k < members.size(); k++) {
         LdsClass L;
@@ -1302,41 +1339,24 @@ static int build_lds_classes(cs_ctx* ctx, Batch& B, const std::vector<int32_t>& 
         for (int32_t c : members[k]) {
             const CPlan& cp = ctx->circuits[c]->hcp;
             dbl_max = std::max(dbl_max, (cp.dbl + 1) & ~1);
-            words_max = std::max(words_max, cp.words);
-            L.nr = std::max(L.nr, c_nr[c]);
+            words_max = std::max(words_max, cp.words_adj);
+            L.nr = std::max(L.nr, B.c_nr[c]);
+            L.dyn = L.dyn || has_dynamic_source(ctx->circuits[c]->plan);
         }
         std::vector<int32_t> order;
         for (int32_t i = 0; i < B.n_inst; i++)
             if (cls_of[B.cid[i]] == (int32_t)k) order.push_back(i);
-        std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
-            return c_need[B.cid[a]] > c_need[B.cid[b]];
-        });
+        std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return need(B.cid[a]) > need(B.cid[b]); });
         void* d_order = nullptr;
         if ((rc = dalloc(&d_order, sizeof(int32_t) * order.size()))) return rc;
         HIPCHK(ctx, hipMemcpy(d_order, order.data(), sizeof(int32_t) * order.size(), hipMemcpyHostToDevice));
         L.n_inst = (int32_t)order.size();
         L.lds = lds_kernel_bytes(dbl_max, words_max);
-        const int per_cu = lds_max_blocks(L.nr, L.lds);
-        if (per_cu <= 0) return fail(ctx, CS_E_RANGE, "LDS-resident kernel does not fit on a CU");
-        L.nblocks = (int32_t)std::min<int64_t>(L.n_inst, (int64_t)per_cu * std::max(ctx->n_cu, 1));
-        LdsArgs& a = L.args;
-        const BatchArgs& g = B.args;
-        a.cplans = (const CPlan*)d_cp;
-        a.plans = g.plans;
-        a.inst_cid = g.inst_cid;
-        a.p_off = g.p_off;
-        a.params = g.params;
-        a.u_off = g.u_off;
-        a.u0 = g.u0;
-        a.w_off = g.w_off;
-        a.wave = g.wave;
-        a.u_final = g.u_final;
-        a.stats = g.stats;
-        a.order = (const int32_t*)d_order;
-        a.queue = B.d_queues + k;
-        a.n_inst = L.n_inst;
-        a.dbl_max = dbl_max;
-        a.o = g.o;
+        L.args = base;
+        L.args.order = (const int32_t*)d_order;
+        L.args.queue = B.d_queues + k;
+        L.args.n_inst = L.n_inst;
+        L.args.dbl_max = dbl_max;
         B.classes.push_back(L);
     }
     while (ctx->side.size() < kSideStreams) {
@@ -1362,11 +1382,13 @@ static int build_lds_classes(cs_ctx* ctx, Batch& B, const std::vector<int32_t>& 
 // circuit that fit, it keeps the one that fills the most wavefronts.  Large
 // circuits are LDS-bound (a few instances beside their image) and small ones
 // slot-bound, so mixing them lets every instance of a batch like the ring
-// Monte Carlo be resident at once.  Returns CS_E_RANGE when a circuit does
-// not fit even one wavefront beside its image.
-static int build_pack(cs_ctx* ctx, Batch& B, const std::vector<int32_t>& used,
-                      const std::vector<int32_t>& c_nr,
-                      const std::function<int(void**, size_t)>& dalloc) {
+// Monte Carlo be resident at once.  A batch that does not fill the device is
+// spread over its CUs instead: a chunk takes no more instances than there
+// would be per CU, since wavefronts on one CU share its LDS and issue ports
+// (60 rings over 500 ps: 8 CUs at 8 wavefronts each before).  Returns
+// CS_E_RANGE when a circuit does not fit even one wavefront beside its image.
+static int build_pack(cs_ctx* ctx, Batch& B, const std::function<int(void**, size_t)>& dalloc) {
+    const std::vector<int32_t>&used = B.used, &c_nr = B.c_nr;
     const size_t nc = ctx->circuits.size();
     std::vector<int32_t> cs = used;
     std::stable_sort(cs.begin(), cs.end(), [&](int32_t a, int32_t b) {
@@ -1374,20 +1396,27 @@ static int build_pack(cs_ctx* ctx, Batch& B, const std::vector<int32_t>& used,
         return x.dbl != y.dbl ? x.dbl > y.dbl : x.n > y.n;
     });
     std::vector<size_t> img(nc, 0), dblb(nc, 0);
-    int32_t nr = 1;
+    PackShape& ks = B.pack;
+    ks = PackShape{};
+    ks.dyn = false;
     for (int32_t c : cs) {
         const CPlan& cp = ctx->circuits[c]->hcp;
         img[c] = 2 * (size_t)((cp.words + 7) & ~7);
         dblb[c] = 8 * (size_t)((cp.dbl + 1) & ~1);
         if (img[c] + dblb[c] > kPackLds) return CS_E_RANGE;
-        nr = std::max(nr, c_nr[c]);
+        ks.nr = std::max(ks.nr, c_nr[c]);
+        ks.dyn = ks.dyn || has_dynamic_source(ctx->circuits[c]->plan);
     }
+    const int64_t n_cu = std::max(ctx->n_cu, 1);
+    ks.waves = (int32_t)std::min<int64_t>(kPackWaves, (B.n_inst + n_cu - 1) / n_cu);
+    // four wavefronts per SIMD only where the batch has more than two
+    ks.occ = ks.nr <= 2 && B.n_inst > kPackWaves * n_cu ? 4 : 2;
     std::vector<std::vector<int32_t>> per(nc);
     for (int32_t i = 0; i < B.n_inst; i++) per[B.cid[i]].push_back(i);
     std::vector<size_t> rem(nc, 0), next(nc, 0);
     for (int32_t c : cs) rem[c] = per[c].size();
     size_t need = 0;
-    const std::vector<std::vector<PackSeg>> chunks = pack_chunks(cs, img, dblb, rem, kPackWaves, kPackSegs, kPackLds, &need);
+    const std::vector<std::vector<PackSeg>> chunks = pack_chunks(cs, img, dblb, rem, ks.waves, kPackSegs, kPackLds, &need);
     if (chunks.empty() && B.n_inst > 0) return CS_E_RANGE;
     // When the chunks outnumber the resident workgroups by E, the E extra
     // chunks start when the first workgroups finish.  The chunks come largest
@@ -1396,15 +1425,14 @@ static int build_pack(cs_ctx* ctx, Batch& B, const std::vector<int32_t>& used,
     // E smallest (descending): the workgroups that finish first take a second
     // small chunk, the largest of those first, instead of a large chunk being
     // followed by a small one.
-    LdsClass& Lc = B.pack;
-    const int per_cu = pack_max_blocks(nr, need);
+    const int per_cu = pack_max_blocks(ks, need);
     if (per_cu <= 0) return fail(ctx, CS_E_RANGE, "packed LDS kernel does not fit on a CU");
     const size_t C = chunks.size();
-    Lc.nblocks = (int32_t)std::min<int64_t>((int64_t)C, (int64_t)per_cu * std::max(ctx->n_cu, 1));
+    B.pack_blocks = (int32_t)std::min<int64_t>((int64_t)C, per_cu * n_cu);
     std::vector<size_t> qorder(C);
     for (size_t i = 0; i < C; i++) qorder[i] = i;
     {
-        const size_t E = C - (size_t)Lc.nblocks;
+        const size_t E = C - (size_t)B.pack_blocks;
         if (E > 0 && 2 * E <= C) {
             qorder.clear();
             for (size_t i = 0; i < E; i++) qorder.push_back(C - 1 - i);
@@ -1438,20 +1466,19 @@ static int build_pack(cs_ctx* ctx, Batch& B, const std::vector<int32_t>& used,
         chunk_seg.push_back((int32_t)(segs.size() / 2));
     }
     if ((int32_t)order.size() != B.n_inst) return fail(ctx, CS_E_INVALID, "packing lost instances");
-    void *d_order, *d_segs, *d_cseg, *d_q;
+    void *d_order, *d_segs, *d_cseg, *d_q, *d_args;
     int rc;
     if ((rc = dalloc(&d_order, sizeof(int32_t) * order.size())) ||
         (rc = dalloc(&d_segs, sizeof(int4) * segs.size())) ||
-        (rc = dalloc(&d_cseg, sizeof(int32_t) * chunk_seg.size())) || (rc = dalloc(&d_q, sizeof(int32_t))))
+        (rc = dalloc(&d_cseg, sizeof(int32_t) * chunk_seg.size())) || (rc = dalloc(&d_q, sizeof(int32_t))) ||
+        (rc = dalloc(&d_args, sizeof(LdsArgs))))
         return rc;
-    Lc.nr = nr;
-    Lc.lds = need;
-    Lc.n_inst = B.n_inst;
+    B.pack_lds = need;
     HIPCHK(ctx, hipMemcpy(d_order, order.data(), sizeof(int32_t) * order.size(), hipMemcpyHostToDevice));
     HIPCHK(ctx, hipMemcpy(d_segs, segs.data(), sizeof(int4) * segs.size(), hipMemcpyHostToDevice));
     HIPCHK(ctx, hipMemcpy(d_cseg, chunk_seg.data(), sizeof(int32_t) * chunk_seg.size(), hipMemcpyHostToDevice));
-    LdsArgs& a = Lc.args;
-    a = B.classes.empty() ? LdsArgs{} : B.classes[0].args;
+    LdsArgs& a = B.pack_args;
+    if ((rc = lds_base_args(ctx, B, dalloc, a))) return rc;
     a.order = (const int32_t*)d_order;
     a.queue = (int32_t*)d_q;
     a.n_inst = B.n_inst;
@@ -1459,6 +1486,8 @@ static int build_pack(cs_ctx* ctx, Batch& B, const std::vector<int32_t>& used,
     a.segs = (const int4*)d_segs;
     a.chunk_seg = (const int32_t*)d_cseg;
     a.n_chunks = (int32_t)C;
+    HIPCHK(ctx, hipMemcpy(d_args, &a, sizeof(LdsArgs), hipMemcpyHostToDevice));
+    B.d_pack_args = (const LdsArgs*)d_args;
     return CS_OK;
 }
 
@@ -1511,7 +1540,6 @@ int cs_batch_create(cs_ctx* ctx, int32_t n_inst, const int32_t* inst_cid, const 
     }
     std::string lds_why;
     std::vector<int32_t> c_nr(ctx->circuits.size(), 0);
-    std::vector<size_t> c_need(ctx->circuits.size(), 0);
     bool lds_fits = true;
     for (int32_t c : used) {
         const Circuit& C = *ctx->circuits[c];
@@ -1531,7 +1559,6 @@ int cs_batch_create(cs_ctx* ctx, int32_t n_inst, const int32_t* inst_cid, const 
             break;
         }
         c_nr[c] = nr;
-        c_need[c] = need;
     }
     if (want == CS_BATCH_KERNEL_LDS && !lds_fits)
         return fail(ctx, CS_E_RANGE, "LDS-resident batch kernel: " + lds_why);
@@ -1611,8 +1638,9 @@ int cs_batch_create(cs_ctx* ctx, int32_t n_inst, const int32_t* inst_cid, const 
         A.clin = (double*)d_c;
         A.linbuf = (double*)d_l;
     } else {
-        if ((rc = build_lds_classes(ctx, *B, used, c_nr, c_need, dalloc)) != CS_OK) return rc;
-        if ((rc = build_pack(ctx, *B, used, c_nr, dalloc)) != CS_OK)
+        B->used = used;
+        B->c_nr = c_nr;
+        if ((rc = build_pack(ctx, *B, dalloc)) != CS_OK)
             return rc == CS_E_RANGE ? fail(ctx, rc, "a circuit does not fit the packed LDS kernel") : rc;
     }
     HIPCHK(ctx, hipEventCreate(&B->ev0));
@@ -1638,10 +1666,9 @@ int cs_batch_run(cs_ctx* ctx, int32_t bid, double* kernel_ms) {
         HIPCHK(ctx, launch_tran_batch(B->nr, B->args, B->nblocks, B->lds, s));
         HIPCHK(ctx, hipEventRecord(B->ev1, s));
     } else {
-        const LdsClass& L = B->pack;
-        HIPCHK(ctx, hipMemsetAsync(L.args.queue, 0, sizeof(int32_t), s));
+        HIPCHK(ctx, hipMemsetAsync(B->pack_args.queue, 0, sizeof(int32_t), s));
         HIPCHK(ctx, hipEventRecord(B->ev0, s));
-        HIPCHK(ctx, launch_tran_pack(L.nr, L.args, L.nblocks, L.lds, s));
+        HIPCHK(ctx, launch_tran_pack(B->pack, B->d_pack_args, B->pack_blocks, B->pack_lds, s));
         HIPCHK(ctx, hipEventRecord(B->ev1, s));
     }
     HIPCHK(ctx, hipEventSynchronize(B->ev1));
@@ -2133,6 +2160,13 @@ int cs_adjoint_batch(cs_ctx* ctx, int32_t n_inst, const int32_t* inst_cid, const
         allocs.push_back(*q);
         return CS_OK;
     };
+    auto balloc = [&](void** q, size_t bytes) -> int {   // lives with the batch
+        hipError_t e = hipMalloc(q, std::max<size_t>(bytes, 16));
+        if (e != hipSuccess) return fail(ctx, CS_E_OOM, "adjoint allocation failed");
+        B->allocs.push_back(*q);
+        return CS_OK;
+    };
+    if ((rc = build_lds_classes(ctx, *B, balloc)) != CS_OK) return rc;
     const int64_t cap = ao->max_steps;
     const int64_t K = ao->ckpt_every;
     const int64_t ckcap = cap / K + 1;
@@ -2153,7 +2187,7 @@ int cs_adjoint_batch(cs_ctx* ctx, int32_t n_inst, const int32_t* inst_cid, const
     std::vector<int> nblk(ncls);
     for (size_t k = 0; k < ncls; k++) {
         const LdsClass& L = B->classes[k];
-        const int per_cu = adj_lds_max_blocks(L.nr, L.lds);
+        const int per_cu = adj_lds_max_blocks(L.nr, L.dyn, L.lds);
         if (per_cu <= 0) return fail(ctx, CS_E_RANGE, "adjoint kernels do not fit on a CU");
         nblk[k] = (int)std::min<int64_t>(L.n_inst, (int64_t)per_cu * std::max(ctx->n_cu, 1));
         void* d_seg;
@@ -2175,6 +2209,10 @@ int cs_adjoint_batch(cs_ctx* ctx, int32_t n_inst, const int32_t* inst_cid, const
         a.seg = (double*)d_seg;
         a.queue2 = (int32_t*)d_q2 + k;
     }
+    void* d_args;
+    if ((rc = dalloc(&d_args, sizeof(AdjLdsArgs) * ncls))) return rc;
+    HIPCHK(ctx, hipMemcpy(d_args, args.data(), sizeof(AdjLdsArgs) * ncls, hipMemcpyHostToDevice));
+    const AdjLdsArgs* da = (const AdjLdsArgs*)d_args;
     hipStream_t s = ctx->stream;
     HIPCHK(ctx, hipMemsetAsync(B->d_queues, 0, sizeof(int32_t) * ncls, s));
     HIPCHK(ctx, hipMemsetAsync(d_q2, 0, sizeof(int32_t) * ncls, s));
@@ -2183,8 +2221,8 @@ int cs_adjoint_batch(cs_ctx* ctx, int32_t n_inst, const int32_t* inst_cid, const
     for (size_t k = 0; k < ns; k++) HIPCHK(ctx, hipStreamWaitEvent(ctx->side[k], B->ev0, 0));
     for (size_t k = 0; k < ncls; k++) {
         const LdsClass& L = B->classes[k];
-        HIPCHK(ctx, launch_adj_lds(L.nr, false, args[k], nblk[k], L.lds, ctx->side[k % ns]));
-        HIPCHK(ctx, launch_adj_lds(L.nr, true, args[k], nblk[k], L.lds, ctx->side[k % ns]));
+        HIPCHK(ctx, launch_adj_lds(L.nr, L.dyn, false, da + k, nblk[k], L.lds, ctx->side[k % ns]));
+        HIPCHK(ctx, launch_adj_lds(L.nr, L.dyn, true, da + k, nblk[k], L.lds, ctx->side[k % ns]));
     }
     for (size_t k = 0; k < ns; k++) {
         HIPCHK(ctx, hipEventRecord(B->class_ev[k], ctx->side[k]));

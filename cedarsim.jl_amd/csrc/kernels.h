@@ -196,18 +196,21 @@ size_t batch_lds_bytes(const BatchArgs& a);
 int batch_max_blocks(int nr, size_t lds);   // resident workgroups per CU
 hipError_t launch_tran_batch(int nr, const BatchArgs& a, int nblocks, size_t lds, hipStream_t s);
 
-// LDS-resident batched transient: LDS bytes of a class, resident workgroups
-// per CU, launch (nr = rows per lane: 1, 2 or 4; devices per lane = 2*nr)
+// LDS bytes of one instance beside its image
 size_t lds_kernel_bytes(int32_t dbl_max, int32_t words_max);
-int lds_max_blocks(int nr, size_t lds);
-hipError_t launch_tran_lds(int nr, const LdsArgs& a, int nblocks, size_t lds, hipStream_t s);
-// packed launch: workgroups of kPackWaves wavefronts, each workgroup runs one
-// chunk at a time: up to kPackSegs runs of same-circuit instances, each run
-// sharing one plan image in LDS
+// packed launch: workgroups of up to kPackWaves wavefronts, each workgroup
+// runs one chunk at a time: up to kPackSegs runs of same-circuit instances,
+// each run sharing one plan image in LDS
 constexpr int kPackWaves = 8;
 constexpr int kPackSegs = 4;
-int pack_max_blocks(int nr, size_t lds);
-hipError_t launch_tran_pack(int nr, const LdsArgs& a, int nblocks, size_t lds, hipStream_t s);
+struct PackShape {
+    int32_t nr = 1;       // rows per lane: 1, 2 or 4 (devices per lane = 2*nr)
+    int32_t waves = 1;    // wavefronts per workgroup
+    int32_t occ = 2;      // wavefronts per SIMD the kernel's registers allow: 2 or 4
+    bool dyn = true;      // some source is not DC
+};
+int pack_max_blocks(const PackShape& k, size_t lds);   // resident workgroups per CU
+hipError_t launch_tran_pack(const PackShape& k, const LdsArgs* d_args, int nblocks, size_t lds, hipStream_t s);
 // one recorded Newton iteration of the LDS-resident instance code (pivot order)
 hipError_t launch_lds_probe(int nr, const CPlan* cp, const DPlan* P, const double* p, const double* u_piv,
                             const double* qx_piv, double a0, double t, int mode, double* f_asm,
@@ -215,8 +218,8 @@ hipError_t launch_lds_probe(int nr, const CPlan* cp, const DPlan* P, const doubl
 
 // LDS-resident adjoint: resident workgroups per CU (min over both kernels),
 // launch of the recording forward or the reverse kernel
-int adj_lds_max_blocks(int nr, size_t lds);
-hipError_t launch_adj_lds(int nr, bool reverse, const AdjLdsArgs& a, int nblocks, size_t lds,
+int adj_lds_max_blocks(int nr, bool dyn, size_t lds);
+hipError_t launch_adj_lds(int nr, bool dyn, bool reverse, const AdjLdsArgs* d_args, int nblocks, size_t lds,
                           hipStream_t s);
 
 // BSIM-CMG: sizes of the generated structs, host helpers, launch

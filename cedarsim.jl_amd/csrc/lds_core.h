@@ -1,429 +1,780 @@
 // lds_core.h — building blocks of the LDS-resident batched kernels
 // (tran_lds.hip: transient; adj_lds.hip: adjoint).
 //
-// One 64-lane wavefront (one workgroup) owns one circuit instance.  The
-// circuit's 16-bit plan image (compact.h) and the instance's numbers live in
-// LDS; a Newton iteration touches only LDS and registers:
+// One 64-lane wavefront owns one circuit instance.  The circuit's 16-bit
+// plan image (compact.h) and the instance's numbers live in LDS; a Newton
+// iteration touches only LDS and registers:
 //
-//   eval      lane m evaluates MOSFETs m, m+64, ...: terminals (pivot
-//             columns), beta = kp*W/L and type*Vth stay in registers;
+//   eval      lane m evaluates MOSFETs m, m+64, ...: terminals (offsets of
+//             u), beta = kp*W/L and type*Vth stay in registers;
 //             (id, dI/dVd, dI/dVg) go to the stamp buffer;
-//   assemble  lane k owns pivot rows k, k+64, ...: F entries gathered from
-//             fixed contributor lists (no atomics, fixed summation order),
-//             residual -> x;
-//   A levels  LU tasks and forward-substitution tasks, one barrier per level;
-//   B levels  backward substitution, one barrier per level;
+//   assemble  one lane per matrix entry: F from fixed records (no atomics,
+//             fixed summation order); one lane per pivot row: -residual -> x;
+//   steps     the solve program: LU with the forward substitution folded in,
+//             then the backward substitution, up to 64 records at a time;
 //   update    u[k] += x[k] (pivot order: no permutation), WRMS norm by a
 //             cross-lane reduction.
 //
+// What bounds it: one iteration is a chain of about 30 dependent LDS round
+// trips of one wavefront (a read 60 cycles, a read after a write 113, a taken
+// branch about 28), so it is latency-bound until 16 wavefronts share a CU;
+// then the LDS pipe is (87 % busy on the 4096-ring batch).  Hence records
+// whose operands are direct byte offsets (two reads deep where row
+// descriptors, pointers and index pairs took five), the next step's record
+// requested before the current step computes, and few register spills: with
+// the plan header's 44 words in scalar registers the packed kernel spilled
+// 233 scalar and 146 vector registers (now 99 and 7), and reloaded them
+// inside the iteration.  Instructions per iteration, averaged over that
+// batch, before and after: vector 1895 -> 995, scalar 1087 -> 470, LDS 359 ->
+// 218.
+//
 // Step control, predictor, local-error test and output interpolation follow
-// rules.h exactly as the global-plan kernel (tran_device.h) does; history
-// (u and charges of the last three accepted points) lives in the registers
-// of the lane that owns the row/column.
+// rules.h as the global-plan kernel (tran_device.h) does; history (u and
+// charges of the last three accepted points) lives in the registers of the
+// lane that owns the row/column.
 #pragma once
 #include "compact.h"
 #include "dcop_rules.h"
 #include "device.h"
 #include "kernels.h"
 
+// Multiplications and additions are fused only where the source says fma: the
+// adjoint's reverse kernel must repeat the forward kernel's bits, and the
+// compiler's own choice may differ from kernel to kernel.
+#pragma clang fp contract(off)
+
 namespace cedar {
 namespace lds {
 
 constexpr int W = 64;
 
-// Cold, register-hungry math (waveforms with fmod/sin/exp, pow in the step
-// factors) stays out of line so it does not raise the register count of the
-// Newton loop; it runs once per step.
-static __device__ __noinline__ double cold_source(int kind, const double* d, int len, double dc, double t,
-                                           int mode) {
-    return source_value(kind, d, len, dc, t, mode);
-}
-static __device__ __noinline__ double cold_next_bp(int kind, const double* d, int len, double t) {
-    return wave_next_bp(kind, d, len, t);
-}
-static __device__ __noinline__ double cold_reject(double err, int k) { return reject_factor(err, k); }
-static __device__ __noinline__ double cold_accept(double err, int k) { return accept_factor(err, k); }
-
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & (W - 1)); }
 
-// Stamp reference r = (slot << 1) | negate: the sign goes straight into the
-// sign bit (negation is exactly a sign flip).
-__device__ __forceinline__ double sv(const double* st, uint32_t r) {
-    const double v = st[r >> 1];
-    return __longlong_as_double(__double_as_longlong(v) ^ ((long long)(r & 1u) << 63));
+// 1/a: the hardware estimate and two Newton corrections (error below one
+// ulp); an infinite estimate (a = 0 or subnormal) stands as it is.
+__device__ __forceinline__ double recip(double a) {
+    const double r0 = __builtin_amdgcn_rcp(a);
+    double r = r0;
+    double e = __builtin_fma(-a, r, 1.0);
+    r = __builtin_fma(r, e, r);
+    e = __builtin_fma(-a, r, 1.0);
+    r = __builtin_fma(r, e, r);
+    return __builtin_isinf(r0) ? r0 : r;
 }
 
-// Sum of the stamp references refs[q, qe) onto s, in order, two references
-// per step so that both loads are in flight together.
-__device__ __forceinline__ double ref_sum(double s, const double* st, const uint16_t* refs, int q, int qe) {
-    for (; q + 1 < qe; q += 2) {
-        const double t0 = sv(st, refs[q]), t1 = sv(st, refs[q + 1]);
-        s += t0;
-        s += t1;
+// a / b for step control: the quotient by recip, corrected once by its
+// residual.
+__device__ __forceinline__ double quot(double a, double b) {
+    const double r = recip(b), q = a * r;
+    return __builtin_fma(__builtin_fma(-q, b, a), r, q);
+}
+
+// s^(-1/(2(k+1))), k = 1 or 2, for s within [1e-6, 1e8]: the step factor's
+// root of the error err = sqrt(s), by a single-precision estimate and two
+// Newton steps on z^-(2(k+1)) = s.
+__device__ __forceinline__ double inv_root(double s, int k) {
+    const float p = k == 1 ? -0.25f : -1.0f / 6.0f;
+    double z = (double)__builtin_amdgcn_exp2f(p * __builtin_amdgcn_logf((float)s));
+    const double w = k == 1 ? 0.25 : 1.0 / 6.0;
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const double z2 = z * z, zp = k == 1 ? z2 * z2 : z2 * z2 * z2;
+        z = __builtin_fma(z * w, __builtin_fma(-s, zp, 1.0), z);
     }
-    if (q < qe) s += sv(st, refs[q]);
-    return s;
+    return z;
+}
+
+// reject_factor and accept_factor of rules.h from the mean square of the
+// error: outside err in [0.09, 729] (k = 2) or [0.2, 81] (k = 1) their clamps
+// decide.
+__device__ __forceinline__ double step_reject(double s, int k) {
+    if (!(s < 1e8)) return 0.1;
+    const double f = 0.9 * inv_root(s, k);
+    return f < 0.1 ? 0.1 : f;
+}
+__device__ __forceinline__ double step_accept(double s, int k) {
+    if (!(s > 1e-6)) return 2.0;
+    const double f = 0.9 * inv_root(s, k);
+    return f > 2.0 ? 2.0 : f;
 }
 
 // Value of lane src (uniform) for the whole wavefront.
-__device__ __forceinline__ double bcast(double v, int src) {
-    const long long b = __double_as_longlong(v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(b & 0xffffffffll), src);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), src);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
+__device__ __forceinline__ double bcast(double v, int src) { return readlane_f64(v, src); }
 
 // Sum over the wavefront in a fixed order (wave_reduce): every lane ends
 // with the same value, the same on every run.
 __device__ __forceinline__ double wave_sum(double v) { return wave_reduce(v, OpSum()); }
-
-// s plus the stamp references refs[q0, q1), summed by the whole wavefront:
-// lane l adds references q0 + l, q0 + l + 64, ... in order, then one
-// wave_sum of the lanes' partial sums.
-__device__ __forceinline__ double wave_ref_sum(double s, const double* st, const uint16_t* refs, int q0, int q1) {
-    double p = 0.0;
-    for (int q = q0 + lane_id(); q < q1; q += W) p += sv(st, refs[q]);
-    return s + wave_sum(p);
+// two of them, their steps interleaved
+__device__ __forceinline__ void wave_sum2(double& a, double& b) {
+    a += dpp_f64<0xB1>(a);   b += dpp_f64<0xB1>(b);
+    a += dpp_f64<0x4E>(a);   b += dpp_f64<0x4E>(b);
+    a += dpp_f64<0x141>(a);  b += dpp_f64<0x141>(b);
+    a += dpp_f64<0x140>(a);  b += dpp_f64<0x140>(b);
+    a = (readlane_f64(a, 0) + readlane_f64(a, 16)) + (readlane_f64(a, 32) + readlane_f64(a, 48));
+    b = (readlane_f64(b, 0) + readlane_f64(b, 16)) + (readlane_f64(b, 32) + readlane_f64(b, 48));
 }
 
 // Synchronisation of the instance's own wavefront.  An instance is owned by
 // one wavefront, so its phases need only wavefront-scope ordering of LDS
 // accesses (other wavefronts of the workgroup own other instances): a fence
 // that keeps the compiler from moving memory accesses across, and the
-// wavefront barrier.
+// wavefront barrier.  The LDS serves one wavefront's accesses in order.
 __device__ __forceinline__ void lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+template <int K>
+struct Count { static constexpr int value = K; };
+
+// Row of slot r of lane tid: lanes past the last row hold a copy of it.
+__device__ __forceinline__ int row_of(int tid, int r, int n) { return tid + W * r < n ? tid + W * r : n - 1; }
+
 // Per-lane MOSFET constants of NM device slots.
 template <int NM>
 struct DevRegs {
     double beta[NM], tpvth[NM];
-    uint32_t dg[NM], sx[NM];   // d | g << 16;  s | (type > 0) << 16
+    uint32_t dg[NM], sx[NM];   // byte offsets of u: d | g << 16;  s | (type < 0) << 31
 };
 
+// The instance's region and the circuit's image.
 struct View {
-    double *F, *G, *C, *st, *u, *x, *inv, *wd;
+    char* R;
     const uint16_t* B;
+    __device__ __forceinline__ double& at(uint32_t off) const { return *reinterpret_cast<double*>(R + off); }
+    // stamp reference: the sign goes straight into the sign bit
+    __device__ __forceinline__ double ref(uint32_t r) const {
+        const double v = at(r & 0xFFF8u);
+        return __longlong_as_double(__double_as_longlong(v) ^ ((long long)r << 63));
+    }
+    __device__ __forceinline__ double2 gc(uint32_t l16) const { return *reinterpret_cast<const double2*>(R + l16); }
 };
 
-// The plan header is uniform: keep it in scalar registers (a vector load
-// followed by readfirstlane, since the compiler cannot prove the header is
-// never written and so will not use scalar loads itself).
-__device__ __forceinline__ CPlan load_header(const CPlan* __restrict__ cp) {
-    CPlan c;
-    const CPlan cv = *cp;
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(&cv);
-    uint32_t* dst = reinterpret_cast<uint32_t*>(&c);
-#pragma unroll
-    for (int w = 0; w < (int)(sizeof(CPlan) / 4); w++) dst[w] = __builtin_amdgcn_readfirstlane(src[w]);
-    return c;
+// Uniform tables (the plan headers, the launch's arguments and options) are
+// read through the scalar cache where they are used.  fresh() makes the
+// compiler forget what it read through a pointer, so that a phase's fields
+// occupy scalar registers only within the phase: carried across the whole
+// transient they exceed the 102 there are.
+template <class T>
+using ConstPtr = const __attribute__((address_space(4))) T*;
+template <class T>
+__device__ __forceinline__ ConstPtr<T> as_const(const T* p) {
+    return (ConstPtr<T>)p;
+}
+template <class T>
+__device__ __forceinline__ ConstPtr<T> fresh(ConstPtr<T> p) {
+    asm volatile("" : "+s"(p));
+    return p;
+}
+// The same for a lane's own values: what is derived from them (addresses,
+// lane masks) is recomputed where it is used instead of being kept.
+__device__ __forceinline__ int fresh_lane(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+typedef ConstPtr<CPlan> Hdr;
+
+// What one Newton iteration reads of the plan header, loaded together at the
+// start of a step's iterations.
+struct Hot {
+    int n, nm, ns, b_x, b_u, b_st;
+    int o_ea, n_ea, o_eb, n_eb, o_ec, n_ec, o_ed, n_ed, o_ez, n_ez;
+    int o_rr, o_lcol, o_items, n_items, o_refs, wide, wide_ed, b_trash;
+    int o_steps, n_lu, n_steps, o_rec, o_upd;
+    const double* mos_m;
+};
+__device__ __forceinline__ Hot load_hot(Hdr c) {
+    c = fresh(c);
+    Hot h;
+    h.n = c->n; h.nm = c->n_mos; h.ns = c->n_src; h.b_x = c->b_x; h.b_u = c->b_u; h.b_st = c->b_st;
+    h.o_ea = c->o_ea; h.n_ea = c->n_ea; h.o_eb = c->o_eb; h.n_eb = c->n_eb; h.o_ec = c->o_ec; h.n_ec = c->n_ec;
+    h.o_ed = c->o_ed; h.n_ed = c->n_ed; h.o_ez = c->o_ez; h.n_ez = c->n_ez;
+    h.o_rr = c->o_rr; h.o_lcol = c->o_lcol; h.o_items = c->o_items; h.n_items = c->n_items; h.o_refs = c->o_refs;
+    h.wide = c->wide_rows; h.wide_ed = c->wide_ed; h.b_trash = c->b_trash;
+    h.o_steps = c->o_steps; h.n_lu = c->n_lu; h.n_steps = c->n_steps; h.o_rec = c->o_rec; h.o_upd = c->o_upd;
+    h.mos_m = c->mos_m;
+    return h;
 }
 
-// Copy the plan image into LDS (words is a multiple of 8, the image 16-byte
-// aligned in both places) with threads t0, t0 + nt, ...  The caller
+// Copy the first `words` uint16 of a plan image (a multiple of 8, the image
+// 16-byte aligned in both places) with threads t0, t0 + nt, ...  The caller
 // synchronises.
-__device__ __forceinline__ void copy_image(const CPlan& c, uint16_t* blob, int t0, int nt) {
-    const uint4* src = reinterpret_cast<const uint4*>(c.blob);
+__device__ __forceinline__ void copy_image(const uint16_t* image, int words, uint16_t* blob, int t0, int nt) {
+    const uint4* src = reinterpret_cast<const uint4*>(image);
     uint4* dst = reinterpret_cast<uint4*>(blob);
-    for (int q = t0; q < c.words / 8; q += nt) dst[q] = src[q];
+#pragma nounroll
+    for (int q = t0; q < words / 8; q += nt) dst[q] = src[q];
 }
 
-__device__ __forceinline__ View make_view(double* lds, const uint16_t* blob, const CPlan& c) {
-    View v;
-    v.F = lds;
-    v.G = v.F + c.nnz;
-    v.C = v.G + c.nlin;
-    v.st = v.C + c.nlin;
-    v.u = v.st + c.stamp_n;
-    v.x = v.u + c.n;
-    v.inv = v.x + c.n;
-    v.wd = v.inv + c.n;
-    v.B = blob;
-    return v;
+// Square-law MOSFET stamps (sqlaw_core of rules.h without branches: in
+// saturation vx is vov, in cutoff vov is 0).
+__device__ __forceinline__ void mos_eval(bool pmos, double beta, double tpvth, double gmin, double vd, double vg,
+                                         double vs, double& id, double& dd, double& dg) {
+    const double vdif = vd - vs;
+    const double vds = pmos ? -vdif : vdif;
+    const bool fwd = vds >= 0.0;
+    const double vgx = vg - (fwd ? vs : vd);
+    const double vo = (pmos ? -vgx : vgx) - tpvth;
+    const double vov = vo > 0.0 ? vo : 0.0;
+    const double va = fabs(vds);
+    const double vx = va < vov ? va : vov;
+    const double cur = beta * (__builtin_fma(-0.5, vx, vov) * vx);
+    const double gm = beta * vx, gds = beta * (vov - vx);
+    id = __builtin_fma(gmin, vdif, (pmos == fwd) ? -cur : cur);
+    dd = (fwd ? gds : gm + gds) + gmin;
+    dg = fwd ? gm : -gm;
 }
 
-template <int NM>
-__device__ __forceinline__ void eval_mos(const CPlan& c, const View& v, const DevRegs<NM>& dr,
-                                         double gmin) {
-    const int nm = c.n_mos;
+// ILP: device slots in pairs, so that two evaluations are in flight
+// together; lanes past the last device hold a copy of it and store the same
+// stamps.
+template <int NM, bool ILP>
+__device__ __forceinline__ void eval_mos(const Hot& h, const View& v, const DevRegs<NM>& dr, double gmin) {
+    const int nm = h.nm, st = h.b_st;
+    if constexpr (!ILP) {
 #pragma unroll
-    for (int j = 0; j < NM; j++) {
-        const int m = lane_id() + W * j;
-        if (m < nm) {
-            const uint32_t d = dr.dg[j] & 0xFFFF, g = dr.dg[j] >> 16, s = dr.sx[j] & 0xFFFF;
-            const double vd = d != CP_GROUND ? v.u[d] : 0.0;
-            const double vg = g != CP_GROUND ? v.u[g] : 0.0;
-            const double vs = s != CP_GROUND ? v.u[s] : 0.0;
-            const double tp = (dr.sx[j] >> 16) ? 1.0 : -1.0;
-            double id, dd, dgv, ds;
-            sqlaw_core(tp, dr.beta[j], dr.tpvth[j], gmin, vd, vg, vs, id, dd, dgv, ds);
-            if (c.mos_m) {   // uniform: only circuits with m-factors read them
-                const double mm = c.mos_m[m];
-                id *= mm; dd *= mm; dgv *= mm;
+        for (int j = 0; j < NM; j++) {
+            const int m = fresh_lane(lane_id()) + W * j;
+            if (m < nm) {
+                double id, dd, dg;
+                const uint32_t t = (uint32_t)fresh_lane((int)dr.dg[j]), u = (uint32_t)fresh_lane((int)dr.sx[j]);
+                mos_eval((int32_t)u < 0, dr.beta[j], dr.tpvth[j], gmin, v.at(t & 0xFFFF), v.at(t >> 16),
+                         v.at(u & 0xFFFF), id, dd, dg);
+                if (h.mos_m) {
+                    const double mm = h.mos_m[m];
+                    id *= mm; dd *= mm; dg *= mm;
+                }
+                v.at(st + 8 * m) = id;
+                v.at(st + 8 * (nm + m)) = dd;
+                v.at(st + 8 * (2 * nm + m)) = dg;
             }
-            v.st[m] = id;
-            v.st[nm + m] = dd;
-            v.st[2 * nm + m] = dgv;
+        }
+        return;
+    }
+    auto slots = [&](auto count, int j0) {
+        constexpr int K = decltype(count)::value;
+        double id[K], dd[K], dg[K];
+#pragma unroll
+        for (int i = 0; i < K; i++) {
+            const uint32_t t = (uint32_t)fresh_lane((int)dr.dg[j0 + i]), u = (uint32_t)fresh_lane((int)dr.sx[j0 + i]);
+            mos_eval((int32_t)u < 0, dr.beta[j0 + i], dr.tpvth[j0 + i], gmin, v.at(t & 0xFFFF), v.at(t >> 16),
+                     v.at(u & 0xFFFF), id[i], dd[i], dg[i]);
+        }
+        const int tid = fresh_lane(lane_id());
+#pragma unroll
+        for (int i = 0; i < K; i++) {
+            const int m = tid + W * (j0 + i) < nm ? tid + W * (j0 + i) : nm - 1;
+            if (h.mos_m) {   // uniform: only circuits with m-factors read them
+                const double mm = h.mos_m[m];
+                id[i] *= mm; dd[i] *= mm; dg[i] *= mm;
+            }
+            v.at(st + 8 * m) = id[i];
+            v.at(st + 8 * (nm + m)) = dd[i];
+            v.at(st + 8 * (2 * nm + m)) = dg[i];
+        }
+    };
+#pragma unroll
+    for (int j0 = 0; j0 < NM; j0 += 2) {
+        if (W * j0 >= nm) break;   // uniform
+        if (W * (j0 + 1) < nm) slots(Count<2>(), j0);
+        else slots(Count<1>(), j0);
+    }
+}
+
+// fmod(t, per), exactly: the remainder by fma is exact and the quotient off
+// by one at most while t / per is below 2^52; larger ratios are first reduced
+// modulo multiples of per.
+__device__ __forceinline__ double fmod_exact(double t, double per) {
+    double a = fabs(t);
+    const double p = fabs(per);
+    if (!(p > 0.0) || !(a < INFINITY)) return __builtin_nan("");
+    if (!(p < INFINITY)) return t;
+    auto part = [](double x, double m) {
+        double r = __builtin_fma(-floor(x / m), m, x);
+        if (r < 0.0) r += m;
+        return r >= m ? r - m : r;
+    };
+    while (!(a < p * 0x1p52)) {
+        int ea, ep;
+        (void)frexp(a, &ea);
+        (void)frexp(p, &ep);
+        a = part(a, ldexp(p, ea - ep - 41));
+    }
+    return copysign(part(a, p), t);
+}
+
+// Taylor coefficients of sine (odd, 1/17! first) and cosine (even, 1/16!
+// first), in memory: as literals they would be held in registers across the
+// whole transient.
+static __device__ const double kSinCos[2][8] = {
+    {1.0 / 355687428096000.0, -1.0 / 1307674368000.0, 1.0 / 6227020800.0, -1.0 / 39916800.0, 1.0 / 362880.0,
+     -1.0 / 5040.0, 1.0 / 120.0, -1.0 / 6.0},
+    {1.0 / 20922789888000.0, -1.0 / 87178291200.0, 1.0 / 479001600.0, -1.0 / 3628800.0, 1.0 / 40320.0,
+     -1.0 / 720.0, 1.0 / 24.0, -0.5}};
+
+// sin_deg of rules.h: reduced to [-45, 45] degrees without rounding, then the
+// Taylor sum of sine or cosine (next terms below 1e-18).
+__device__ __forceinline__ double sin_degrees(double x) {
+    const double r = fmod_exact(x, 360.0);
+    const double q = rint(r / 90.0);
+    const double y = __builtin_fma(-90.0, q, r) * (3.14159265358979323846 / 180.0);
+    const double z = y * y;
+    const int k = (int)q & 3;
+    const double* t = kSinCos[k & 1];
+    double s = t[0];
+#pragma nounroll
+    for (int j = 1; j < 8; j++) s = __builtin_fma(s, z, t[j]);
+    s = k & 1 ? __builtin_fma(s, z, 1.0) : __builtin_fma(s * z, y, y);
+    return k & 2 ? -s : s;
+}
+
+// source_value of rules.h without calls: every operation inline, so that the
+// transient loop keeps its registers across it.
+__device__ __forceinline__ double source_at(int kind, const double* d, int len, double dc, double t, int mode) {
+    if (mode == CS_MODE_DCOP) {
+        if (dc == dc) return dc;
+        t = 0.0;
+    }
+    if (kind == CS_WAVE_DC) return d[0];
+    if (kind == CS_WAVE_PULSE) {
+        const double c0 = d[2], c1 = d[2] + d[3], c2 = d[2] + d[3] + d[5];
+        const double c3 = d[2] + d[3] + d[5] + d[4];
+        return pulse_at(d[0], d[1], c0, c1, c2, c3, fmod_exact(t, d[6]));
+    }
+    if (kind == CS_WAVE_PWL) return pwl_at(d, len / 2, t);
+    // CS_WAVE_SIN: vo va freq td theta phase ncycles
+    double ang = d[5], amp = d[1];
+    if (d[3] < t && t < d[6] / d[2]) {
+        ang = 360.0 * d[2] * (t - d[3]) + d[5];
+        if (d[4] != 0.0) amp *= exp(-(t - d[3]) * d[4]);
+    }
+    return d[0] + amp * sin_degrees(ang);
+}
+
+// wave_next_bp of rules.h, the corners of a pulse one at a time
+__device__ __forceinline__ double next_bp(int kind, const double* d, int len, double t) {
+    const double thr = t + 8.0 * 2.220446049250313e-16 * fabs(t) + 1e-300;
+    double best = INFINITY;
+    if (kind == CS_WAVE_PULSE) {
+        const double per = d[6];
+        const bool once = __builtin_isinf(per);
+        const double m = once ? 0.0 : floor(t / per);
+#pragma nounroll
+        for (int j = 0; j < 4; j++) {
+            double c = d[2];
+            if (j > 0) c += d[3];
+            if (j > 1) c += d[5];
+            if (j > 2) c += d[4];
+            if (once) {
+                if (c > thr && c < best) best = c;
+            } else if (c < per) {
+#pragma nounroll
+                for (int r = -1; r <= 1; r++) {
+                    const double b = (m + r) * per + c;
+                    if (b > thr && b < best) best = b;
+                }
+            }
+        }
+    } else if (kind == CS_WAVE_PWL) {
+#pragma nounroll
+        for (int j = 0; j < len / 2; j++) {
+            const double b = d[2 * j];
+            if (b > thr && b < best) best = b;
+        }
+    } else if (kind == CS_WAVE_SIN) {
+        if (d[3] > thr) best = d[3];
+    }
+    return best;
+}
+
+// DYN = false: every source of the circuit is a DC one; the waveform code is
+// left out, and with it the registers it holds across the transient.
+template <bool DYN>
+__device__ __forceinline__ void eval_sources(Hdr c, const View& v, double t, int mode) {
+    c = fresh(c);
+    const int ns = c->n_src;
+#pragma nounroll
+    for (int s = lane_id(); s < ns; s += W) {
+        const uint16_t* d = v.B + c->o_src + 4 * s;
+        const double* wd = &v.at(d[1]);
+        double val;
+        if constexpr (DYN) {
+            val = source_at(d[0], wd, d[2], wd[d[2]], t, mode);
+        } else {
+            const double dc = wd[d[2]];
+            val = mode == CS_MODE_DCOP && dc == dc ? dc : wd[0];
+        }
+        v.at(d[3]) = c->src_m ? val * c->src_m[s] : val;
+    }
+}
+
+// Partial sums of one wavefront item: references and linear entries by
+// lane, the row's charge term by its owner lane.
+template <int NR>
+__device__ __forceinline__ double item_part(const Hot& h, const View& v, double a0, const double (&qx)[NR], uint4 p) {
+    const int tid = fresh_lane(lane_id());
+    const uint16_t* refs = v.B + h.o_refs;
+    const int q1 = p.y & 0xFFFF, l1 = p.z & 0xFFFF, k = p.z >> 16;
+    const bool row = (p.w & 0xFFFF) != 0;
+    double s = 0.0;
+#pragma nounroll
+    for (int q = (int)(p.x >> 16) + tid; q < q1; q += 2 * W) {
+        const int q2 = q + W;
+        const double s0 = v.ref(refs[q]), s1 = v.ref(refs[q2 < q1 ? q2 : q]);
+        s += q2 < q1 ? s0 + s1 : s0;
+    }
+#pragma nounroll
+    for (int l = (int)(p.y >> 16) + tid; l < l1; l += W) {
+        const double2 g = v.gc(16 * l);
+        const double j = __builtin_fma(a0, g.y, g.x);
+        s = row ? __builtin_fma(j, v.at((v.B + h.o_lcol)[l]), s) : s + j;
+    }
+    if (row) {
+#pragma unroll
+        for (int r = 0; r < NR; r++)
+            if (k == tid + W * r) s += qx[r];
+    }
+    return s;
+}
+
+// F = G + a0*C + nonlinear stamps (and the inverse of the diagonals the
+// factorization does not update); x = -residual, qx added per row.
+// The records of a class's first rounds and of the rows are read together,
+// then their operands, then everything is stored: two LDS latencies where a
+// loop per class took two each.  Lanes past a class's end read its last
+// record and store the same value to the same place, which costs the LDS
+// latency nothing (measured), where masking them off costs two branches a
+// store.  ILP = false is the form for a CU full of wavefronts, where the LDS
+// pipe bounds instead (87 % busy on the 4096-ring batch) and every lane
+// masked off saves its cycles: one record at a time, lanes past the end off.  Entries with many references and the residuals of long rows (the
+// supply node: one reference per device on it) are summed by the whole
+// wavefront, two sums at a time, in a fixed order, so that runs are
+// bit-identical.
+template <int NR, bool ILP>
+__device__ __forceinline__ void assemble(const Hot& h, const View& v, double a0, const double (&qx)[NR]) {
+    constexpr int EA = ILP ? 2 * NR : 0, ED = ILP ? NR : 0, EB = ILP ? 1 : 0;
+    const uint16_t* B = v.B;
+    const int tid = fresh_lane(lane_id());
+    const uint2* ra = reinterpret_cast<const uint2*>(B + h.o_ea);
+    const uint2* rb = reinterpret_cast<const uint2*>(B + h.o_eb);
+    const uint4* rd = reinterpret_cast<const uint4*>(B + h.o_ed);
+    const uint4* rr = reinterpret_cast<const uint4*>(B + h.o_rr);
+    auto last = [&](int i, int n) { return i < n ? i : n - 1; };
+    // -residual of the row of record p, without the sums of a long row
+    auto row = [&](const uint4& p, double q) {
+        const double2 g = v.gc(16 * (p.x & 0xFFFF));
+        double f = __builtin_fma(__builtin_fma(a0, g.y, g.x), v.at(p.y & 0xFFFF),
+                                 q + (v.ref(p.y >> 16) + v.ref(p.z & 0xFFFF)));
+        if (h.wide) {
+            f += v.ref(p.z >> 16) + (v.ref(p.w & 0xFFFF) + v.ref(p.w >> 16));
+            const uint32_t nl = p.x >> 16;
+            if (nl != 0xFFFF) {
+#pragma nounroll
+                for (uint32_t l = (p.x & 0xFFFF) + 1, le = l + nl; l + 1 < le; l++) {
+                    const double2 g = v.gc(16 * l);
+                    f = __builtin_fma(__builtin_fma(a0, g.y, g.x), v.at((B + h.o_lcol)[l]), f);
+                }
+            }
+        }
+        return -f;
+    };
+    if constexpr (ILP) {
+        uint2 pa[EA];
+        uint4 pd[ED], pr[NR];
+#pragma unroll
+        for (int r = 0; r < EA; r++) pa[r] = ra[last(tid + W * r, h.n_ea)];
+#pragma unroll
+        for (int r = 0; r < ED; r++) pd[r] = rd[last(tid + W * r, h.n_ed)];
+        const uint2 pb = rb[last(tid, h.n_eb)];
+#pragma unroll
+        for (int r = 0; r < NR; r++) pr[r] = rr[last(tid + W * r, h.n)];
+        double fa[EA], fd[ED], id[ED], fx[NR], fb;
+#pragma unroll
+        for (int r = 0; r < EA; r++) fa[r] = v.ref(pa[r].x >> 16) + v.ref(pa[r].y & 0xFFFF);
+#pragma unroll
+        for (int r = 0; r < ED; r++) {
+            const double2 g = v.gc(pd[r].x >> 16);
+            fd[r] = __builtin_fma(a0, g.y, g.x) + (v.ref(pd[r].y & 0xFFFF) + v.ref(pd[r].y >> 16));
+        }
+        if (h.wide_ed) {
+#pragma unroll
+            for (int r = 0; r < ED; r++) fd[r] += v.ref(pd[r].z >> 16) + v.ref(pd[r].w & 0xFFFF);
+        }
+        {
+            const double2 g = v.gc(pb.x >> 16);
+            fb = __builtin_fma(a0, g.y, g.x) + (v.ref(pb.y & 0xFFFF) + v.ref(pb.y >> 16));
+        }
+#pragma unroll
+        for (int r = 0; r < NR; r++) fx[r] = row(pr[r], qx[r]);
+#pragma unroll
+        for (int r = 0; r < ED; r++) id[r] = recip(fd[r]);
+        const int lane = fresh_lane(tid);
+#pragma unroll
+        for (int r = 0; r < EA; r++)
+            v.at(pa[r].x & 0xFFFF) = fa[r];
+#pragma unroll
+        for (int r = 0; r < ED; r++)
+        {
+            v.at(pd[r].x & 0xFFFF) = fd[r];
+            v.at(pd[r].z & 0xFFFF) = id[r];
+        }
+        v.at(pb.x & 0xFFFF) = fb;
+#pragma unroll
+        for (int r = 0; r < NR; r++)
+            v.at((pr[r].x >> 16) != 0xFFFF ? h.b_x + 8 * last(lane + W * r, h.n) : h.b_trash) = fx[r];
+    } else {
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            const int k = tid + W * r;
+            if (k < h.n) {
+                const uint4 p = rr[k];
+                const double f = row(p, qx[r]);
+                if ((p.x >> 16) != 0xFFFF) v.at(h.b_x + 8 * k) = f;
+            }
+        }
+    }
+    // the entries left
+#pragma nounroll
+    for (int i = tid + W * EA; i < h.n_ea; i += 2 * W) {
+        const uint2 p = ra[i], q = ra[i + W < h.n_ea ? i + W : i];
+        const double p0 = v.ref(p.x >> 16) + v.ref(p.y & 0xFFFF), q0 = v.ref(q.x >> 16) + v.ref(q.y & 0xFFFF);
+        v.at(p.x & 0xFFFF) = p0;
+        v.at(q.x & 0xFFFF) = q0;
+    }
+#pragma nounroll
+    for (int i = tid + W * ED; i < h.n_ed; i += W) {
+        const uint4 p = rd[i];
+        const double2 g = v.gc(p.x >> 16);
+        double s = __builtin_fma(a0, g.y, g.x) + (v.ref(p.y & 0xFFFF) + v.ref(p.y >> 16));
+        if (h.wide_ed) s += v.ref(p.z >> 16) + v.ref(p.w & 0xFFFF);
+        v.at(p.x & 0xFFFF) = s;
+        v.at(p.z & 0xFFFF) = recip(s);
+    }
+#pragma nounroll
+    for (int i = tid + W * EB; i < h.n_eb; i += W) {
+        const uint2 p = rb[i];
+        const double2 g = v.gc(p.x >> 16);
+        v.at(p.x & 0xFFFF) = __builtin_fma(a0, g.y, g.x) + (v.ref(p.y & 0xFFFF) + v.ref(p.y >> 16));
+    }
+#pragma nounroll
+    for (int i = tid; i < h.n_ec; i += W) {
+        const uint4 p = reinterpret_cast<const uint4*>(B + h.o_ec)[i];
+        const double2 g = v.gc(p.x >> 16);
+        const double s = (v.ref(p.y & 0xFFFF) + v.ref(p.y >> 16)) + (v.ref(p.z & 0xFFFF) + v.ref(p.z >> 16));
+        v.at(p.x & 0xFFFF) = __builtin_fma(a0, g.y, g.x) + (s + (v.ref(p.w & 0xFFFF) + v.ref(p.w >> 16)));
+    }
+#pragma nounroll
+    for (int i = tid; i < h.n_ez; i += W) v.at((B + h.o_ez)[i]) = 0.0;
+    // wavefront sums
+    const uint4* items = reinterpret_cast<const uint4*>(B + h.o_items);
+#pragma nounroll
+    for (int i = 0; i < h.n_items; i += 2) {
+        const uint4 p = items[i], q = items[i + 1];
+        double s = item_part<NR>(h, v, a0, qx, p), t = item_part<NR>(h, v, a0, qx, q);
+        wave_sum2(s, t);
+        if (tid == 0) {
+            v.at(p.x & 0xFFFF) = p.w & 0xFFFF ? -s : s;
+            v.at(q.x & 0xFFFF) = q.w & 0xFFFF ? -t : t;
         }
     }
 }
 
-__device__ __forceinline__ void eval_sources(const CPlan& c, const View& v, double t, int mode) {
-    for (int s = lane_id(); s < c.n_src; s += W) {
-        const uint16_t* d = v.B + c.o_src + 4 * s;
-        const int kind = d[0], off = d[1], len = d[2];
-        const double* wd = v.wd + off;
-        const double val = cold_source(kind, wd, len, wd[len], t, mode);
-        v.st[3 * c.n_mos + s] = c.src_m ? val * c.src_m[s] : val;
-    }
-}
-
-// F = G + a0*C + nonlinear stamps; x = -residual (qx added per row).  With
-// pin, rows that carry charge become u_k = pin_k.  Returns max |residual|.
-// A lane assembles its own rows; long rows (flag in the diagonal field) are
-// assembled afterwards by the whole wavefront: short entries one lane each,
-// heavy entries, the linear products and the residual's reference list as
-// wavefront sums of 64 terms at a time (a fixed summation order, so runs are
-// bit-identical; it differs from the one-lane order only by rounding).
+// Rows that carry charge pinned: F's row k becomes the unit row, x[k] =
+// pin - u[k] (consistent initialisation; runs after the assembly).
 template <int NR>
-__device__ __forceinline__ double assemble(const CPlan& c, const View& v, double a0,
-                                           const double (&qx)[NR], bool pin,
+__device__ __forceinline__ void apply_pins(Hdr c, const View& v, const DPlan* __restrict__ P,
                                            const double (&pinv)[NR], const uint32_t (&flag)[NR]) {
-    const uint16_t* B = v.B;
-    double lmax = 0.0;
+    c = fresh(c);
+    lds_sync();
 #pragma unroll
     for (int r = 0; r < NR; r++) {
         const int k = lane_id() + W * r;
-        if (k < c.n) {
-            const uint4 rd = reinterpret_cast<const uint4*>(B + c.o_rdesc)[k];
-            if (rd.y & 0x8000) continue;   // a long row
-            const int e0 = rd.x & 0xFFFF, e1 = rd.x >> 16, dg = rd.y & 0x7FFF;
-            double res;
-            if (pin && (flag[r] & 1)) {
-                for (int e = e0; e < e1; e++) v.F[e] = (e == dg) ? 1.0 : 0.0;
-                res = v.u[k] - pinv[r];
-            } else {
-                int q = rd.y >> 16;
-                for (int e = e0; e < e1; e++) {
-                    const int qe = B[c.o_jptr + e + 1];
-                    v.F[e] = ref_sum(0.0, v.st, B + c.o_jref, q, qe);
-                    q = qe;
-                }
-                double acc = 0.0;
-                const int l0 = rd.z & 0xFFFF, l1 = rd.z >> 16;
-                for (int l = l0; l < l1; l++) {
-                    const double jl = v.G[l] + a0 * v.C[l];
-                    v.F[B[c.o_lpos + l]] += jl;
-                    acc += jl * v.u[B[c.o_lcol + l]];
-                }
-                acc += qx[r];
-                res = ref_sum(acc, v.st, B + c.o_rref, rd.w & 0xFFFF, rd.w >> 16);
-            }
-            v.x[k] = -res;
-            const double a = fabs(res);
-            if (a != a || a > lmax) lmax = a;
+        if (k < c->n && (flag[r] & 1)) {
+            const int dg = P->diag[k];
+#pragma nounroll
+            for (int e = P->rowptr[k]; e < P->rowptr[k + 1]; e++) v.at(c->b_F + 8 * e) = e == dg ? 1.0 : 0.0;
+            v.at(c->b_inv + 8 * k) = 1.0;
+            v.at(c->b_x + 8 * k) = pinv[r] - v.at(c->b_u + 8 * k);
         }
     }
-    for (int i = 0; i < c.n_lrows; i++) {
-        const uint2 lr = reinterpret_cast<const uint2*>(B + c.o_lrows)[i];
-        const int k = lr.x & 0xFFFF, hb = lr.x >> 16, he = lr.y & 0xFFFF;
-        const uint4 rd = reinterpret_cast<const uint4*>(B + c.o_rdesc)[k];
-        const int e0 = rd.x & 0xFFFF, e1 = rd.x >> 16, dg = rd.y & 0x7FFF;
-        // the owner lane's per-row registers
-        const int owner = k % W, rk = k / W;
-        double qxo = 0.0, pio = 0.0;
-        uint32_t flo = 0;
+}
+
+// Largest |residual|, NaN-propagating; x holds the negated residuals.
+template <int NR>
+__device__ __forceinline__ double residual_max(Hdr c, const View& v) {
+    double m = 0.0;
 #pragma unroll
-        for (int r = 0; r < NR; r++)
-            if (r == rk) {
-                qxo = qx[r];
-                pio = pinv[r];
-                flo = flag[r];
-            }
-        qxo = bcast(qxo, owner);
-        pio = bcast(pio, owner);
-        flo = (uint32_t)__builtin_amdgcn_readlane((int)flo, owner);
-        double res;
-        if (pin && (flo & 1)) {
-            for (int e = e0 + lane_id(); e < e1; e += W) v.F[e] = (e == dg) ? 1.0 : 0.0;
-            res = v.u[k] - pio;
-        } else {
-            for (int e = e0 + lane_id(); e < e1; e += W) {
-                const int q0 = B[c.o_jptr + e], q1 = B[c.o_jptr + e + 1];
-                if (q1 - q0 > kHeavyRefs) continue;
-                v.F[e] = ref_sum(0.0, v.st, B + c.o_jref, q0, q1);
-            }
-            for (int h = hb; h < he; h++) {
-                const int e = B[c.o_heavy + h];
-                const double s = wave_ref_sum(0.0, v.st, B + c.o_jref, B[c.o_jptr + e], B[c.o_jptr + e + 1]);
-                if (lane_id() == 0) v.F[e] = s;
+    for (int r = 0; r < NR; r++) {
+        const int k = lane_id() + W * r;
+        if (k < c->n) {
+            const double a = fabs(v.at(c->b_x + 8 * k));
+            if (a != a || a > m) m = a;
+        }
+    }
+    return wave_reduce(m, OpMax());
+}
+
+// One long record by the whole wavefront: lane l subtracts products ub + l,
+// ub + l + 64, ... in order, then one wave_sum of the lanes' partial sums.
+__device__ __forceinline__ void long_task(const View& v, const uint16_t* upd, uint32_t w0, uint32_t w1, bool dia) {
+    const uint32_t* up = reinterpret_cast<const uint32_t*>(upd);
+    const int tid = fresh_lane(lane_id());
+    const int ue = w1 >> 16;
+    const double x0 = v.at(w0 & 0xFFFF), sc = v.at(w0 >> 16);
+    double s = 0.0;
+#pragma nounroll
+    for (int q = (int)(w1 & 0xFFFF) + tid; q < ue; q += 2 * W) {
+        const int q2 = q + W;
+        const uint32_t a = up[q], b = up[q2 < ue ? q2 : q];
+        const double fa = v.at(a & 0xFFFF), xa = v.at(a >> 16), fb = v.at(b & 0xFFFF), xb = v.at(b >> 16);
+        s = __builtin_fma(fa, xa, s);
+        if (q2 < ue) s = __builtin_fma(fb, xb, s);
+    }
+    s = x0 - wave_sum(s);
+    const double t = dia ? recip(s) : s * sc;
+    if (tid == 0) {
+        v.at(w0 & 0xFFFF) = dia ? s : t;
+        if (dia) v.at(w0 >> 16) = t;
+    }
+}
+
+// One record of a step of products or scalings, for the lanes that have one.
+__device__ __forceinline__ void masked_step(const View& v, uint32_t kind, const uint4& w) {
+    if (kind == SP_SCALE) {
+        const double r0 = v.at(w.x & 0xFFFF) * v.at(w.x >> 16), r1 = v.at(w.y & 0xFFFF) * v.at(w.y >> 16);
+        const double r2 = v.at(w.z & 0xFFFF) * v.at(w.z >> 16), r3 = v.at(w.w & 0xFFFF) * v.at(w.w >> 16);
+        v.at(w.x & 0xFFFF) = r0;
+        v.at(w.y & 0xFFFF) = r1;
+        v.at(w.z & 0xFFFF) = r2;
+        v.at(w.w & 0xFFFF) = r3;
+        return;
+    }
+    double r = __builtin_fma(-v.at(w.y & 0xFFFF), v.at(w.y >> 16), v.at(w.x & 0xFFFF));
+    if (kind != SP_MUL1)
+        r = __builtin_fma(-v.at(w.w & 0xFFFF), v.at(w.w >> 16),
+                          __builtin_fma(-v.at(w.z & 0xFFFF), v.at(w.z >> 16), r));
+    if (kind == SP_DIA3) {
+        v.at(w.x & 0xFFFF) = r;
+        v.at(w.x >> 16) = recip(r);
+    } else {
+        v.at(w.x & 0xFFFF) = r * v.at(w.x >> 16);
+    }
+}
+
+// Run ns steps of the solve program (descriptors at steps).  The descriptors
+// come one per lane, 63 steps and the following one at a time, and each
+// step's through a lane read; the next step's record is requested before this
+// step's operands, so that its latency lies under this step, and all operands
+// of a record before any is used.  Lanes past the count run the step's last
+// record again and store the same values: with the store masked, a step of
+// one product took 350 cycles for 120 (measured alone, one wavefront).  ILP =
+// false masks them off, for a CU whose LDS pipe is full.
+template <bool ILP>
+__device__ __forceinline__ void run_steps(const View& v, const uint16_t* steps, int ns, const uint16_t* recs,
+                                          const uint16_t* upd) {
+    const uint32_t* sd = reinterpret_cast<const uint32_t*>(steps);
+    const uint4* rec = reinterpret_cast<const uint4*>(recs);
+    const int tid = fresh_lane(lane_id());
+    auto fetch = [&](uint32_t d) {
+        const int c1 = (int)(d >> 16) & 63;
+        if constexpr (ILP) return rec[(d & 0xFFFF) + (tid < c1 ? tid : c1)];
+        uint4 w = make_uint4(0, 0, 0, 0);
+        if (tid <= c1) w = rec[(d & 0xFFFF) + tid];
+        return w;
+    };
+#pragma nounroll
+    for (int s0 = 0; s0 < ns; s0 += W - 1) {
+        const int m = ns - s0 < W - 1 ? ns - s0 : W - 1;
+        const int dv = (int)sd[s0 + (tid < m ? tid : m)];
+        uint32_t dn = (uint32_t)__builtin_amdgcn_readlane(dv, 0);
+        uint4 next = fetch(dn);
+#pragma nounroll
+        for (int q = 1; q <= m; q++) {
+            const uint32_t d = dn;
+            const uint4 w = next;
+            dn = (uint32_t)__builtin_amdgcn_readlane(dv, q);
+            next = fetch(dn);
+            const uint32_t kind = d >> 22;
+            if (!ILP && kind <= SP_DIA3) {
+                if (tid <= ((int)(d >> 16) & 63)) masked_step(v, kind, w);
+            } else if (kind == SP_MUL1) {
+                const double x = v.at(w.x & 0xFFFF), a0 = v.at(w.y & 0xFFFF), b0 = v.at(w.y >> 16), k = v.at(w.x >> 16);
+                const double r = __builtin_fma(-a0, b0, x) * k;
+                lds_sync();
+                v.at(w.x & 0xFFFF) = r;
+            } else if (kind == SP_MUL3) {
+                const double x = v.at(w.x & 0xFFFF), a0 = v.at(w.y & 0xFFFF), b0 = v.at(w.y >> 16);
+                const double a1 = v.at(w.z & 0xFFFF), b1 = v.at(w.z >> 16), a2 = v.at(w.w & 0xFFFF), b2 = v.at(w.w >> 16);
+                const double k = v.at(w.x >> 16);
+                const double r = __builtin_fma(-a2, b2, __builtin_fma(-a1, b1, __builtin_fma(-a0, b0, x))) * k;
+                lds_sync();
+                v.at(w.x & 0xFFFF) = r;
+            } else if (kind == SP_SCALE) {
+                const double r0 = v.at(w.x & 0xFFFF) * v.at(w.x >> 16), r1 = v.at(w.y & 0xFFFF) * v.at(w.y >> 16);
+                const double r2 = v.at(w.z & 0xFFFF) * v.at(w.z >> 16), r3 = v.at(w.w & 0xFFFF) * v.at(w.w >> 16);
+                lds_sync();
+                v.at(w.x & 0xFFFF) = r0;
+                v.at(w.y & 0xFFFF) = r1;
+                v.at(w.z & 0xFFFF) = r2;
+                v.at(w.w & 0xFFFF) = r3;
+            } else if (kind == SP_DIA3) {
+                const double x = v.at(w.x & 0xFFFF), a0 = v.at(w.y & 0xFFFF), b0 = v.at(w.y >> 16);
+                const double a1 = v.at(w.z & 0xFFFF), b1 = v.at(w.z >> 16), a2 = v.at(w.w & 0xFFFF), b2 = v.at(w.w >> 16);
+                const double r = __builtin_fma(-a2, b2, __builtin_fma(-a1, b1, __builtin_fma(-a0, b0, x)));
+                const double ri = recip(r);
+                lds_sync();
+                v.at(w.x & 0xFFFF) = r;
+                v.at(w.x >> 16) = ri;
+            } else {
+                const int c1 = (int)(d >> 16) & 63;
+#pragma nounroll
+                for (int i = 0; i <= c1; i++)
+                    long_task(v, upd, (uint32_t)__builtin_amdgcn_readlane((int)w.x, i),
+                              (uint32_t)__builtin_amdgcn_readlane((int)w.y, i), kind == SP_LDIA);
             }
             lds_sync();
-            // linear entries: F updates in parallel (distinct entries), the
-            // residual's products summed by the wavefront
-            double p = 0.0;
-            const int l0 = rd.z & 0xFFFF, l1 = rd.z >> 16;
-            for (int l = l0 + lane_id(); l < l1; l += W) {
-                const double jl = v.G[l] + a0 * v.C[l];
-                v.F[B[c.o_lpos + l]] += jl;
-                p += jl * v.u[B[c.o_lcol + l]];
-            }
-            double acc = wave_sum(p);
-            acc += qxo;
-            res = wave_ref_sum(acc, v.st, B + c.o_rref, rd.w & 0xFFFF, rd.w >> 16);
-        }
-        if (lane_id() == 0) {
-            v.x[k] = -res;
-            const double a = fabs(res);
-            if (a != a || a > lmax) lmax = a;
         }
     }
-    return lmax;
 }
 
-// One X task: x[k] -= sum F[a] x[b]; scaled by inv[k] when fl & 1.  Long
-// tasks (fl & 2) are skipped here and run by x_task_long.
-// acc minus the products Fa[a] Fb[b] over the packed pairs up[w..we) (a in
-// the low 16 bits, b in the high), subtracted in order; the loads of four
-// pairs are issued before their products
-__device__ __forceinline__ double upd_sum(double acc, const uint32_t* up, int w, int we, const double* Fa,
-                                          const double* Fb) {
-    for (; w + 3 < we; w += 4) {
-        uint32_t ab[4];
-        double fa[4], fb[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) ab[u] = up[w + u];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            fa[u] = Fa[ab[u] & 0xFFFF];
-            fb[u] = Fb[ab[u] >> 16];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) acc -= fa[u] * fb[u];
-    }
-    for (; w < we; w++) {
-        const uint32_t ab = up[w];
-        acc -= Fa[ab & 0xFFFF] * Fb[ab >> 16];
-    }
-    return acc;
+// LU with the forward substitution of x folded in.
+template <bool ILP>
+__device__ __forceinline__ void factor(const Hot& h, const View& v) {
+    run_steps<ILP>(v, v.B + h.o_steps, h.n_lu, v.B + h.o_rec, v.B + h.o_upd);
 }
 
-__device__ __forceinline__ void x_task(const uint2* xt, const uint32_t* up, int q, const View& v) {
-    const uint2 t = xt[q];
-    if ((t.y >> 16) & 2) return;
-    const int k = t.x & 0xFFFF, ub = t.x >> 16, ue = t.y & 0xFFFF;
-    const double sc = (t.y >> 16) & 1 ? v.inv[k] : 1.0;
-    const double acc = upd_sum(v.x[k], up, ub, ue, v.F, v.x);
-    v.x[k] = (t.y >> 16) & 1 ? acc * sc : acc;
-}
-
-// A long X task by the whole wavefront: x[k] minus the products F[a] x[b];
-// lane l sums products ub + l, ub + l + 64, ... in order, then one wave_sum
-// of the lanes' partial sums.
-__device__ __forceinline__ void x_task_long(const uint2 t, const uint32_t* up, const View& v) {
-    const int k = t.x & 0xFFFF, ub = t.x >> 16, ue = t.y & 0xFFFF;
-    double p = 0.0;
-    for (int w = ub + lane_id(); w < ue; w += W) {
-        const uint32_t ab = up[w];
-        p += v.F[ab & 0xFFFF] * v.x[ab >> 16];
-    }
-    const double acc = v.x[k] - wave_sum(p);
-    if (lane_id() == 0) v.x[k] = (t.y >> 16) & 1 ? acc * v.inv[k] : acc;
-}
-
-// The long tasks of a level sit at the end of its range [xb, xe); a level
-// that has them carries bit 15 in its end index.
-__device__ __forceinline__ void x_long_tasks(const uint2* xt, const uint32_t* up, int xb, int xe_flag,
-                                             const View& v) {
-    if (!(xe_flag & 0x8000)) return;
-    for (int q = (xe_flag & 0x7FFF) - 1; q >= xb; q--) {
-        const uint2 t = xt[q];
-        if (!((t.y >> 16) & 2)) break;
-        x_task_long(t, up, v);
-    }
-}
-
-// X-task levels given by (begin, end) descriptors.
-__device__ __forceinline__ void x_levels(const CPlan& c, const View& v, int o_desc, int nlev) {
-    const uint16_t* B = v.B;
-    const uint2* xt = reinterpret_cast<const uint2*>(B + c.o_xtask);
-    const uint32_t* up = reinterpret_cast<const uint32_t*>(B + c.o_upd);
-    for (int l = 0; l < nlev; l++) {
-        const uint32_t bd = reinterpret_cast<const uint32_t*>(B + o_desc)[l];
-        const int xb = bd & 0xFFFF, xe = bd >> 16, nx = (xe & 0x7FFF) - xb;
-        for (int q = lane_id(); q < nx; q += W) x_task(xt, up, xb + q, v);
-        x_long_tasks(xt, up, xb, xe, v);
-        lds_sync();
-    }
-}
-
-// LU, with the forward substitution folded in when FWD (A levels).
-template <bool FWD>
-__device__ __forceinline__ void factor(const CPlan& c, const View& v) {
-    const uint16_t* B = v.B;
-    const uint2* ft = reinterpret_cast<const uint2*>(B + c.o_ftask);
-    const uint2* xt = reinterpret_cast<const uint2*>(B + c.o_xtask);
-    const uint32_t* up = reinterpret_cast<const uint32_t*>(B + c.o_upd);
-    double* F = v.F;
-    double* inv = v.inv;
-    for (int l = 0; l < c.nA; l++) {
-        const uint2 ad = reinterpret_cast<const uint2*>(B + c.o_adesc)[l];
-        const int fb = ad.x & 0xFFFF, nf = (ad.x >> 16) - fb;
-        const int xb = ad.y & 0xFFFF, nx = FWD ? (int)((ad.y >> 16) & 0x7FFF) - xb : 0;
-        for (int q = lane_id(); q < nf + nx; q += W) {
-            if (q < nf) {
-                const uint2 t = ft[fb + q];
-                const int e = t.x & 0xFFFF, ub = t.x >> 16, ue = t.y & 0xFFFF;
-                const uint32_t ctl = t.y >> 16;
-                // the scale is loaded with the operands (its pivot is from an
-                // earlier level), not after the updates
-                const double sc = ctl < CP_PLAIN_U ? inv[ctl] : 1.0;
-                const double acc = upd_sum(F[e], up, ub, ue, F, F);
-                if (ctl < CP_PLAIN_U) {
-                    F[e] = acc * sc;
-                } else {
-                    F[e] = acc;
-                    if (ctl & CP_DIAG) inv[ctl & 0x7FFF] = 1.0 / acc;
-                }
-            } else {
-                x_task(xt, up, xb + q - nf, v);
-            }
-        }
-        if (FWD) x_long_tasks(xt, up, xb, (int)(ad.y >> 16), v);
-        lds_sync();
-    }
-}
-
-// Newton step: LU + forward (A levels), then backward (B levels).
-__device__ __forceinline__ void factor_solve(const CPlan& c, const View& v) {
-    factor<true>(c, v);
-    x_levels(c, v, c.o_bdesc, c.nB);
+// Newton step: LU + forward, then backward.
+template <bool ILP>
+__device__ __forceinline__ void factor_solve(const Hot& h, const View& v) {
+    run_steps<ILP>(v, v.B + h.o_steps, h.n_steps, v.B + h.o_rec, v.B + h.o_upd);
 }
 
 // J^T x = b on the factors in F (U^T then L^T); b and the result in x.
-__device__ __forceinline__ void solve_transposed(const CPlan& c, const View& v) {
-    x_levels(c, v, c.o_tudesc, c.nTU);
-    x_levels(c, v, c.o_tldesc, c.nTL);
+__device__ __forceinline__ void solve_transposed(Hdr c, const View& v) {
+    c = fresh(c);
+    run_steps<true>(v, v.B + c->o_tsteps, c->n_tsteps, v.B + c->o_rec, v.B + c->o_upd);
 }
 
 // charge of pivot row k: sum over its linear entries C * u
-__device__ __forceinline__ double row_charge(const CPlan& c, const View& v, int k) {
-    const uint16_t* B = v.B;
-    const uint32_t lz = reinterpret_cast<const uint32_t*>(B + c.o_rdesc)[4 * k + 2];
-    double acc = 0.0;
-    for (int l = lz & 0xFFFF; l < (int)(lz >> 16); l++) acc += v.C[l] * v.u[B[c.o_lcol + l]];
+__device__ __forceinline__ double row_charge(Hdr c, const View& v, int k) {
+    const uint4 p = reinterpret_cast<const uint4*>(v.B + c->o_rr)[k];
+    const uint32_t l0 = p.x & 0xFFFF;
+    const uint32_t nl = (p.x >> 16) == 0xFFFF ? p.y >> 16 : p.x >> 16;   // a long row's count: its first reference
+    double acc = v.gc(16 * l0).y * v.at(p.y & 0xFFFF);
+#pragma nounroll
+    for (uint32_t l = l0 + 1; l < l0 + nl; l++) acc = __builtin_fma(v.gc(16 * l).y, v.at((v.B + c->o_lcol)[l]), acc);
     return acc;
 }
 
-// (C^T y)[j] for column j: sum over the linear entries of column j
-__device__ __forceinline__ double col_charge_t(const CPlan& c, const View& v, const double* y, int j) {
+// (C^T x)[j] for column j: sum over the linear entries of column j
+__device__ __forceinline__ double col_charge_t(Hdr c, const View& v, int j) {
     const uint16_t* B = v.B;
-    const uint32_t cz = reinterpret_cast<const uint32_t*>(B + c.o_cdesc)[j];
+    const uint32_t cz = reinterpret_cast<const uint32_t*>(B + c->o_cdesc)[j];
     double acc = 0.0;
-    for (int q = cz & 0xFFFF; q < (int)(cz >> 16); q++) acc += v.C[B[c.o_lcl + q]] * y[B[c.o_lrow + q]];
+#pragma nounroll
+    for (int q = cz & 0xFFFF; q < (int)(cz >> 16); q++)
+        acc = __builtin_fma(v.gc(16 * (uint32_t)B[c->o_lcl + q]).y, v.at(c->b_x + 8 * B[c->o_lrow + q]), acc);
     return acc;
 }
 
@@ -440,90 +791,101 @@ __device__ __forceinline__ double lin_value(const DPlan* __restrict__ P, const d
     return (ref & 1) ? -val : val;
 }
 
-// Instance set-up: linear stamps G, C and source data into LDS, device
-// constants into registers.  The caller synchronises.
+// Instance set-up: linear stamps G, C, constants and source data into LDS,
+// device constants into registers.  The caller synchronises.
 template <int NM>
-__device__ __forceinline__ void setup_instance(const CPlan& c, const DPlan* __restrict__ P,
-                                               const double* __restrict__ p, const View& v,
-                                               DevRegs<NM>& dr) {
-    const uint16_t* B = v.B;
-    const int tid = lane_id();
-    for (int l = tid; l < c.nlin; l += W) {
-        const int e = B[c.o_lpos + l];
+__device__ __forceinline__ void setup_instance(Hdr c, const DPlan* __restrict__ P, const double* __restrict__ p,
+                                               const View& v, DevRegs<NM>& dr) {
+    c = fresh(c);
+    const int tid = lane_id(), nlin = c->nlin;
+    // the F position of a linear entry, from the global plan's patterns: the
+    // entries with a G or C contribution, in F order
+    const int32_t* lp = c->lpos;
+#pragma nounroll
+    for (int l = tid; l < nlin; l += W) {
+        const int e = lp[l];
         double g = 0.0, cc = 0.0;
+#pragma nounroll
         for (int q = P->g_ptr[e]; q < P->g_ptr[e + 1]; q++) g += lin_value(P, p, P->g_ref[q]);
+#pragma nounroll
         for (int q = P->c_ptr[e]; q < P->c_ptr[e + 1]; q++) cc += lin_value(P, p, P->c_ref[q]);
-        v.G[l] = g;
-        v.C[l] = cc;
+        v.at(16 * l) = g;
+        v.at(16 * l + 8) = cc;
     }
-    for (int s = tid; s < c.n_src; s += W) {
+    if (tid == 0) {
+        v.at(16 * nlin) = v.at(16 * nlin + 8) = 0.0;
+        v.at(c->b_zero) = 0.0;
+        v.at(c->b_one) = 1.0;
+        v.at(c->b_trash) = 0.0;
+    }
+#pragma nounroll
+    for (int s = tid; s < c->n_src; s += W) {
         const int4 d = P->src[s];
-        const int off = B[c.o_src + 4 * s + 1];
-        for (int j = 0; j < d.z; j++) v.wd[off + j] = p[d.y + j];
-        v.wd[off + d.z] = p[d.w];
+        double* wd = &v.at(v.B[c->o_src + 4 * s + 1]);
+#pragma nounroll
+        for (int j = 0; j < d.z; j++) wd[j] = p[d.y + j];
+        wd[d.z] = p[d.w];
     }
 #pragma unroll
     for (int j = 0; j < NM; j++) {
-        const int m = tid + W * j;
+        const int m = tid + W * j < c->n_mos ? tid + W * j : c->n_mos - 1;   // past the last: a copy of it
         dr.beta[j] = 0.0;
         dr.tpvth[j] = 0.0;
-        dr.dg[j] = 0;
-        dr.sx[j] = 0;
-        if (m < c.n_mos) {
-            const int4 dv = reinterpret_cast<const int4*>(c.dev)[m];
-            const double tp = (double)dv.w;
+        dr.dg[j] = (uint32_t)c->b_zero * 0x10001u;
+        dr.sx[j] = (uint32_t)c->b_zero;
+        if (m >= 0) {
+            const int4 dv = reinterpret_cast<const int4*>(c->dev)[m];
             dr.beta[j] = p[P->p_mos_kp + m] * p[P->p_mos_w + m] / p[P->p_mos_l + m];
-            dr.tpvth[j] = tp * p[P->p_mos_vth + m];
+            dr.tpvth[j] = (double)dv.w * p[P->p_mos_vth + m];
             dr.dg[j] = (uint32_t)dv.x | ((uint32_t)dv.y << 16);
-            dr.sx[j] = (uint32_t)dv.z | ((dv.w > 0 ? 1u : 0u) << 16);
+            dr.sx[j] = (uint32_t)dv.z | (dv.w > 0 ? 0u : 0x80000000u);
         }
     }
 }
 
 // Newton iterations of one BDF step from the predictor already in u:
 // eval -> assemble -> LU + solves -> u += x, until WRMS(x) <= tol.
-template <int NR, int NM>
-__device__ __forceinline__ bool newton(const CPlan& c, const View& v, const DevRegs<NM>& dr,
-                                       double gmin, double a0, const double (&qx)[NR],
-                                       const double (&pinv)[NR], const uint32_t (&flag)[NR],
-                                       int maxit, double tol, double reltol, double abstol,
+template <int NR, int NM, bool ILP>
+__device__ __forceinline__ bool newton(Hdr c, const View& v, const DevRegs<NM>& dr, double gmin, double a0,
+                                       const double (&qx)[NR], int maxit, double tol, double reltol, double abstol,
                                        long long& nit) {
-    const int tid = lane_id();
+    const Hot h = load_hot(c);
+    const int n = h.n, bx = h.b_x, bu = h.b_u;
+    const double lim = tol * tol * n;   // WRMS <= tol
+#pragma nounroll
     for (int it = 0; it < maxit; it++) {
-        eval_mos<NM>(c, v, dr, gmin);
+        eval_mos<NM, ILP>(h, v, dr, gmin);
         lds_sync();
-        assemble<NR>(c, v, a0, qx, false, pinv, flag);
+        assemble<NR, ILP>(h, v, a0, qx);
         lds_sync();
-        factor_solve(c, v);
+        factor_solve<ILP>(h, v);
         nit++;
         double ss = 0.0;
+        const int tid = fresh_lane(lane_id());
+        double un[NR];
 #pragma unroll
         for (int r = 0; r < NR; r++) {
-            const int kk = tid + W * r;
-            if (kk < c.n) {
-                const double d = v.x[kk];
-                const double ui = v.u[kk] + d;
-                v.u[kk] = ui;
-                const double q = d / (reltol * fabs(ui) + abstol);
-                ss += q * q;
-            }
+            const int k8 = 8 * row_of(tid, r, n);
+            const double d = v.at(bx + k8);
+            un[r] = v.at(bu + k8) + d;
+            const double q = d * recip(__builtin_fma(reltol, fabs(un[r]), abstol));
+            ss = tid + W * r < n ? __builtin_fma(q, q, ss) : ss;
         }
-        const double nr = sqrt(block_reduce<W>(ss, nullptr, OpSum()) / c.n);
         lds_sync();
-        if (!(nr == nr)) return false;
-        if (nr <= tol) return true;
+#pragma unroll
+        for (int r = 0; r < NR; r++) v.at(bu + 8 * row_of(tid, r, n)) = un[r];
+        ss = wave_sum(ss);
+        lds_sync();
+        if (!(ss == ss)) return false;
+        if (ss <= lim) return true;
     }
     return false;
 }
 
 // Start of DC trajectory j in u (pivot order; the draw is by natural index).
-// Inlined: built as an out-of-line call (its only call sites are on the DC
-// path), the packed kernel returned corrupted step counters and step sizes
-// for UIC runs that never take that call, while the same source with the
-// call inlined matches the oracle; the out-of-line cold_* helpers above take
-// only values and are unaffected.
-__device__ __forceinline__ void dc_set_start(const CPlan& c, double* u, int j) {
-    for (int k = lane_id(); k < c.n; k += W) u[k] = dc_start(j, c.colnat[k]);
+__device__ __forceinline__ void dc_set_start(Hdr c, const View& v, int j) {
+#pragma nounroll
+    for (int k = lane_id(); k < c->n; k += W) v.at(c->b_u + 8 * k) = dc_start(j, c->colnat[k]);
 }
 
 // Consistent initial point: (UIC) the charge rows pinned to u0 and the
@@ -536,26 +898,28 @@ __device__ __forceinline__ void dc_set_start(const CPlan& c, double* u, int j) {
 //   phase -1   pinned (UIC, or after the DC point), at most 50 iterations;
 //   phase 0-9  trajectory j from its own start, at most 200 iterations;
 //   phase 10   the gmin ladder from trajectory 0's start, stage by stage.
-template <int NR, int NM>
-__device__ __forceinline__ bool init_point(const CPlan& c, const View& v, const DevRegs<NM>& dr,
-                                           double gmin, bool uic, double (&pinv)[NR],
-                                           const uint32_t (&flag)[NR], double t0,
-                                           double dc_abstol, long long& nit) {
+template <int NR, int NM, bool DYN>
+__device__ __forceinline__ bool init_point(Hdr c, const View& v, const DPlan* __restrict__ P, const DevRegs<NM>& dr,
+                                           double gmin, bool uic, double (&pinv)[NR], const uint32_t (&flag)[NR],
+                                           double t0, double dc_abstol, long long& nit) {
     const int tid = lane_id();
     double qx0[NR];
 #pragma unroll
     for (int r = 0; r < NR; r++) qx0[r] = 0.0;
-    eval_sources(c, v, t0, uic ? CS_MODE_TRAN : CS_MODE_DCOP);
+    eval_sources<DYN>(c, v, t0, uic ? CS_MODE_TRAN : CS_MODE_DCOP);
     int phase = uic ? -1 : 0, stage = 0, it = 0;
     bool pin = uic;
     double g = gmin;
-    if (!uic) dc_set_start(c, v.u, 0);
+    if (!uic) dc_set_start(c, v, 0);
     lds_sync();
     for (;;) {
-        eval_mos<NM>(c, v, dr, g);
+        const Hot h = load_hot(c);
+        eval_mos<NM, false>(h, v, dr, g);
         lds_sync();
-        const double lm = assemble<NR>(c, v, 0.0, qx0, pin, pinv, flag);
-        const double fn = block_reduce<W>(lm, nullptr, OpMax());
+        assemble<NR, false>(h, v, 0.0, qx0);
+        if (pin) apply_pins<NR>(c, v, P, pinv, flag);
+        lds_sync();
+        const double fn = residual_max<NR>(c, v);
         lds_sync();
         if (fn <= dc_abstol) {
             bool dc_done = phase >= 0 && phase < kDcTrajectories;
@@ -572,9 +936,9 @@ __device__ __forceinline__ bool init_point(const CPlan& c, const View& v, const 
 #pragma unroll
             for (int r = 0; r < NR; r++) {
                 const int k = tid + W * r;
-                pinv[r] = k < c.n ? v.u[k] : 0.0;
+                pinv[r] = k < c->n ? v.at(c->b_u + 8 * k) : 0.0;
             }
-            eval_sources(c, v, t0, CS_MODE_TRAN);
+            eval_sources<DYN>(c, v, t0, CS_MODE_TRAN);
             phase = -1;
             pin = true;
             g = gmin;
@@ -586,10 +950,8 @@ __device__ __forceinline__ bool init_point(const CPlan& c, const View& v, const 
         if (!(fn == fn) || __builtin_isinf(fn) || it >= maxit) {
             if (phase < 0 || phase >= kDcTrajectories) return false;
             phase++;
-            if (phase < kDcTrajectories) {
-                dc_set_start(c, v.u, phase);
-            } else {                                         // the gmin ladder
-                dc_set_start(c, v.u, 0);
+            dc_set_start(c, v, phase < kDcTrajectories ? phase : 0);
+            if (phase >= kDcTrajectories) {                  // the gmin ladder
                 stage = 0;
                 g = dc_gmin_stage(0, gmin);
             }
@@ -597,11 +959,11 @@ __device__ __forceinline__ bool init_point(const CPlan& c, const View& v, const 
             lds_sync();
             continue;
         }
-        factor_solve(c, v);
+        factor_solve<false>(h, v);
 #pragma unroll
         for (int r = 0; r < NR; r++) {
             const int k = tid + W * r;
-            if (k < c.n) v.u[k] += v.x[k];
+            if (k < c->n) v.at(c->b_u + 8 * k) += v.at(c->b_x + 8 * k);
         }
         nit++;
         it++;
@@ -609,82 +971,116 @@ __device__ __forceinline__ bool init_point(const CPlan& c, const View& v, const 
     }
 }
 
+// bdf_coeffs, pred_weights and lte_coeff of rules.h with quot() for the
+// divisions
+__device__ __forceinline__ void step_bdf(int k, double tn, double T0, double T1, double& a0, double& a1, double& a2) {
+    const double r0 = quot(1.0, tn - T0);
+    a0 = r0;
+    a1 = -r0;
+    a2 = 0.0;
+    if (k != 1) {
+        a0 = r0 + quot(1.0, tn - T1);
+        a1 = quot(tn - T1, (T0 - tn) * (T0 - T1));
+        a2 = quot(tn - T0, (T1 - tn) * (T1 - T0));
+    }
+}
+__device__ __forceinline__ void step_pred(int np, double tn, double T0, double T1, double T2, double& l0, double& l1,
+                                          double& l2) {
+    l0 = 1.0;
+    l1 = l2 = 0.0;
+    if (np == 2) {
+        const double s = quot(tn - T0, T0 - T1);
+        l0 = 1.0 + s;
+        l1 = -s;
+    } else if (np == 3) {
+        l0 = quot((tn - T1) * (tn - T2), (T0 - T1) * (T0 - T2));
+        l1 = quot((tn - T0) * (tn - T2), (T1 - T0) * (T1 - T2));
+        l2 = quot((tn - T0) * (tn - T1), (T2 - T0) * (T2 - T1));
+    }
+}
+__device__ __forceinline__ double step_lte(int k, double tn, double T0, double T1, double T2, double a0, double a1,
+                                           double a2) {
+    const double d1 = T0 - tn, d2 = T1 - tn;
+    if (k == 1) return quot(a1 * d1 * d1, a0 * (tn - T0) * (tn - T1));
+    return quot(a1 * d1 * d1 * d1 + a2 * d2 * d2 * d2, a0 * (tn - T0) * (tn - T1) * (tn - T2));
+}
+
 // Recording policy of run_lds that records nothing.
 struct NoRec {
     template <int NR>
-    __device__ __forceinline__ bool on_accept(const CPlan&, const View&, double, double, int,
+    __device__ __forceinline__ bool on_accept(Hdr, const View&, double, double, int,
                                               long long, const double (&)[NR], const double (&)[NR],
                                               const double (&)[NR]) {
         return true;
     }
 };
 
-// One instance's whole transient.  Rec::on_accept is called for the initial
-// point (m = 0) and after every accepted step m with the new state in u and
-// the history registers; returning false stops the run with CS_E_RANGE.
-template <int NR, class Rec>
-__device__ void run_lds(Rec& rec, const CPlan& c, const DPlan* __restrict__ P,
-                        const double* __restrict__ p, const double* __restrict__ u0,
-                        double* __restrict__ wave, double* __restrict__ ufin,
-                        cs_tran_stats* __restrict__ stp, const cs_tran_opts& o, const View& v) {
+// One instance's whole transient (the step loop of rules.h).  Rec::on_accept
+// is called for the initial point (m = 0) and after every accepted step m
+// with the new state in u and the history registers; returning false stops
+// the run with CS_E_RANGE.
+template <int NR, bool DYN, bool ILP, class Rec>
+__device__ __forceinline__ void run_lds(Rec& rec, Hdr c, ConstPtr<LdsArgs> A, const DPlan* __restrict__ P, int inst,
+                                        const View& v) {
     constexpr int NM = 2 * NR;
     const int tid = lane_id();
-    const int n = c.n;
-    const uint16_t* B = v.B;
-    const StepDefaults sd = step_defaults(o);
+    const int n = c->n, bu = c->b_u;
     const uint64_t clk0 = wall_clock64();
-    const bool uic = (o.init == CS_INIT_UIC) && u0 != nullptr;
+    const double* const p = A->params + A->p_off[inst];
+    const double* const u0 = A->u0 ? A->u0 + A->u_off[inst] : nullptr;
+    const bool uic = A->o.init == CS_INIT_UIC && u0 != nullptr;
 
     DevRegs<NM> dr;
     setup_instance<NM>(c, P, p, v, dr);
     const double gmin = p[P->p_gmin];
     double Uh0[NR], Uh1[NR], Uh2[NR], Qh0[NR], Qh1[NR], up[NR], qx[NR], pinv[NR];
     uint32_t flag[NR];
-    int32_t cn[NR];
 #pragma unroll
     for (int r = 0; r < NR; r++) {
         const int k = tid + W * r;
         Uh0[r] = Uh1[r] = Uh2[r] = Qh0[r] = Qh1[r] = up[r] = qx[r] = pinv[r] = 0.0;
         flag[r] = 0;
-        cn[r] = 0;
         if (k < n) {
-            cn[r] = c.colnat[k];
-            flag[r] = c.diffrow[k] ? 1u : 0u;
-            pinv[r] = uic ? u0[cn[r]] : 0.0;
-            v.u[k] = pinv[r];
+            flag[r] = c->diffrow[k] ? 1u : 0u;
+            pinv[r] = uic ? u0[c->colnat[k]] : 0.0;
+            v.at(bu + 8 * k) = pinv[r];
         }
     }
     lds_sync();
 
     long long steps = 0, rej = 0, nit = 0;
-    int rc = init_point<NR, NM>(c, v, dr, gmin, uic, pinv, flag, o.t_start, o.dc_abstol, nit)
+    int rc = init_point<NR, NM, DYN>(c, v, P, dr, gmin, uic, pinv, flag, A->o.t_start, A->o.dc_abstol, nit)
                  ? CS_OK : CS_E_NOCONV;
 
-    double t = o.t_start;
+    A = fresh(A);
+    const double t_start = A->o.t_start;
+    double t = t_start;
     if (rc == CS_OK) {
         lds_sync();
 #pragma unroll
         for (int r = 0; r < NR; r++) {
-            const int k = tid + W * r;
-            if (k < n) {
-                Uh0[r] = v.u[k];
-                Qh0[r] = row_charge(c, v, k);
-            }
+            const int k = row_of(tid, r, n);
+            Uh0[r] = v.at(bu + 8 * k);
+            Qh0[r] = row_charge(c, v, k);
         }
-        if (!rec.template on_accept<NR>(c, v, o.t_start, o.t_start, 0, 0, Uh0, Uh1, Uh2)) rc = CS_E_RANGE;
-        double T0 = o.t_start, T1 = 0.0, T2 = 0.0;
+        if (!rec.template on_accept<NR>(c, v, t_start, t_start, 0, 0, Uh0, Uh1, Uh2)) rc = CS_E_RANGE;
+        double T0 = t_start, T1 = 0.0, T2 = 0.0;
         int npts = 1;
-        double h = sd.dt_init;
+        // step_defaults of rules.h
+        const double span = A->o.t_stop - t_start;
+        double h = A->o.dt_init > 0 ? A->o.dt_init : span * 1e-9;
+        const double dt_min = A->o.dt_min > 0 ? A->o.dt_min : span * 1e-15;
+        double* const wave = A->wave ? A->wave + A->w_off[inst] : nullptr;
         int kout = 0;
         const int n_probe = P->n_probe;
         int32_t ps[NR];
 #pragma unroll
         for (int r = 0; r < NR; r++) {
             const int k = tid + W * r;
-            ps[r] = (wave && k < n) ? c.probe[k] : -1;
+            ps[r] = (wave && k < n) ? c->probe[k] : -1;
         }
         if (wave) {
-            while (kout < o.n_out && o.t_start + kout * o.dt_out <= o.t_start + 1e-9 * o.dt_out) {
+            while (kout < A->o.n_out && t_start + kout * A->o.dt_out <= t_start + 1e-9 * A->o.dt_out) {
 #pragma unroll
                 for (int r = 0; r < NR; r++)
                     if (ps[r] >= 0) wave[(size_t)kout * n_probe + ps[r]] = Uh0[r];
@@ -694,89 +1090,96 @@ __device__ void run_lds(Rec& rec, const CPlan& c, const DPlan* __restrict__ P,
         // with only DC sources there is no breakpoint and, in transient mode,
         // no source value that changes with t: the per-step breakpoint
         // search is skipped and the sources are evaluated at the first step
-        int dyn = 0;
-        for (int s = tid; s < c.n_src; s += W)
-            if (B[c.o_src + 4 * s] != CS_WAVE_DC) dyn = 1;
-        const bool dyn_src = block_reduce<W>((double)dyn, nullptr, OpMax()) > 0.0;
+        bool dyn_src = false;
+        if constexpr (DYN) {
+            int dyn = 0;
+#pragma nounroll
+            for (int s = tid; s < c->n_src; s += W)
+                if (v.B[c->o_src + 4 * s] != CS_WAVE_DC) dyn = 1;
+            dyn_src = wave_reduce((double)dyn, OpMax()) > 0.0;
+        }
         bool src_set = false;
         lds_sync();
-        while (rc == CS_OK && t < o.t_stop) {
-            if (steps + rej >= o.max_steps) { rc = CS_E_MAXSTEPS; break; }
-            double tb = o.t_stop;
+        for (;;) {
+            lds_sync();
+            A = fresh(A);
+            const double t_stop = A->o.t_stop;
+            if (!(rc == CS_OK && t < t_stop)) break;
+            if (steps + rej >= A->o.max_steps) { rc = CS_E_MAXSTEPS; break; }
+            double tb = t_stop;
             bool srcbp = false;
-            if (dyn_src) {
-                double lb = INFINITY;
-                for (int s = tid; s < c.n_src; s += W) {
-                    const uint16_t* d = B + c.o_src + 4 * s;
-                    const double b = cold_next_bp(d[0], v.wd + d[1], d[2], t);
-                    if (b < lb) lb = b;
+            if constexpr (DYN) {
+                if (dyn_src) {
+                    double lb = INFINITY;
+#pragma nounroll
+                    for (int s = tid; s < c->n_src; s += W) {
+                        const uint16_t* d = v.B + c->o_src + 4 * s;
+                        const double b = next_bp(d[0], &v.at(d[1]), d[2], t);
+                        if (b < lb) lb = b;
+                    }
+                    tb = wave_reduce(lb, OpMin());
+                    srcbp = tb < t_stop;
+                    if (!srcbp) tb = t_stop;
                 }
-                tb = block_reduce<W>(lb, nullptr, OpMin());
-                srcbp = tb < o.t_stop;
-                if (!srcbp) tb = o.t_stop;
             }
-            double hh = h < sd.dt_max ? h : sd.dt_max;
+            const double dt_max = A->o.dt_max > 0 ? A->o.dt_max : quot(t_stop - t_start, 10.0);
+            double hh = h < dt_max ? h : dt_max;
             int hit;
             const double tn = clip_step(t, hh, tb, hit);
-            const int k = bdf_order(npts, o.max_order);
+            const int k = bdf_order(npts, A->o.max_order);
             double a0, a1, a2, w0, w1, w2;
-            bdf_coeffs(k, tn, T0, T1, a0, a1, a2);
+            step_bdf(k, tn, T0, T1, a0, a1, a2);
             const int np = npts < k + 1 ? npts : k + 1;
-            pred_weights(np, tn, T0, T1, T2, w0, w1, w2);
+            step_pred(np, tn, T0, T1, T2, w0, w1, w2);
+            const int lane = fresh_lane(tid);
 #pragma unroll
             for (int r = 0; r < NR; r++) {
-                const int kk = tid + W * r;
-                if (kk < n) {
-                    double val = Uh0[r];
-                    if (np == 2) val = w0 * Uh0[r] + w1 * Uh1[r];
-                    else if (np == 3) val = w0 * Uh0[r] + w1 * Uh1[r] + w2 * Uh2[r];
-                    up[r] = val;
-                    v.u[kk] = val;
-                    qx[r] = a1 * Qh0[r] + (k == 2 ? a2 * Qh1[r] : 0.0);
-                }
+                double val = Uh0[r];
+                if (np == 2) val = __builtin_fma(w0, Uh0[r], w1 * Uh1[r]);
+                else if (np == 3) val = __builtin_fma(w0, Uh0[r], __builtin_fma(w1, Uh1[r], w2 * Uh2[r]));
+                up[r] = val;
+                v.at(bu + 8 * row_of(lane, r, n)) = val;
+                qx[r] = __builtin_fma(a1, Qh0[r], k == 2 ? a2 * Qh1[r] : 0.0);
             }
-            if (dyn_src || !src_set) eval_sources(c, v, tn, CS_MODE_TRAN);
+            if (dyn_src || !src_set) eval_sources<DYN>(c, v, tn, CS_MODE_TRAN);
             src_set = true;
             lds_sync();
-            if (!newton<NR, NM>(c, v, dr, gmin, a0, qx, pinv, flag, o.newton_maxit, o.newton_tol,
-                                o.reltol, o.abstol, nit)) {
+            if (!newton<NR, NM, ILP>(c, v, dr, gmin, a0, qx, A->o.newton_maxit, A->o.newton_tol, A->o.reltol,
+                                A->o.abstol, nit)) {
                 rej++;
                 h = 0.25 * hh;
-                if (h < sd.dt_min) { rc = CS_E_DTMIN; break; }
+                if (h < dt_min) { rc = CS_E_DTMIN; break; }
                 continue;
             }
+            A = fresh(A);
             double fac = 2.0;
             if (npts >= 2) {
-                const double cl = lte_coeff(k, tn, T0, T1, T2, a0, a1, a2);
+                const double cl = step_lte(k, tn, T0, T1, T2, a0, a1, a2);
                 double ss = 0.0;
+                const int lane = fresh_lane(tid);
 #pragma unroll
                 for (int r = 0; r < NR; r++) {
-                    const int kk = tid + W * r;
-                    if (kk < n) {
-                        const double ui = v.u[kk];
-                        const double est = cl * (ui - up[r]);
-                        const double m = fabs(ui) > fabs(Uh0[r]) ? fabs(ui) : fabs(Uh0[r]);
-                        const double q = est / (o.reltol * m + o.abstol);
-                        ss += q * q;
-                    }
+                    const double ui = v.at(bu + 8 * row_of(lane, r, n));
+                    const double est = cl * (ui - up[r]);
+                    const double m = fabs(ui) > fabs(Uh0[r]) ? fabs(ui) : fabs(Uh0[r]);
+                    const double q = est * recip(__builtin_fma(A->o.reltol, m, A->o.abstol));
+                    ss = lane + W * r < n ? __builtin_fma(q, q, ss) : ss;
                 }
-                const double err = sqrt(block_reduce<W>(ss, nullptr, OpSum()) / n);
-                if (!(err <= 1.0)) {
+                const double err2 = quot(wave_sum(ss), (double)n);
+                if (!(err2 <= 1.0)) {
                     rej++;
-                    h = hh * cold_reject(err, k);
-                    if (h < sd.dt_min) { rc = CS_E_DTMIN; break; }
+                    h = hh * step_reject(err2, k);
+                    if (h < dt_min) { rc = CS_E_DTMIN; break; }
                     continue;
                 }
-                fac = cold_accept(err, k);
+                fac = step_accept(err2, k);
             }
             // accept
 #pragma unroll
             for (int r = 0; r < NR; r++) {
-                const int kk = tid + W * r;
-                if (kk < n) {
-                    Uh2[r] = Uh1[r]; Uh1[r] = Uh0[r]; Uh0[r] = v.u[kk];
-                    Qh1[r] = Qh0[r]; Qh0[r] = row_charge(c, v, kk);
-                }
+                const int kk = row_of(fresh_lane(tid), r, n);
+                Uh2[r] = Uh1[r]; Uh1[r] = Uh0[r]; Uh0[r] = v.at(bu + 8 * kk);
+                Qh1[r] = Qh0[r]; Qh0[r] = row_charge(c, v, kk);
             }
             if (!rec.template on_accept<NR>(c, v, tn, T0, npts, steps + 1, Uh0, Uh1, Uh2)) {
                 rc = CS_E_RANGE;
@@ -786,23 +1189,15 @@ __device__ void run_lds(Rec& rec, const CPlan& c, const DPlan* __restrict__ P,
             if (npts < 3) npts++;
             steps++;
             if (wave) {
-                while (kout < o.n_out) {
-                    const double tq = o.t_start + kout * o.dt_out;
-                    if (tq > tn + 1e-9 * o.dt_out) break;
-                    double l0, l1, l2 = 0.0;
-                    if (npts >= 3) {
-                        l0 = (tq - T1) * (tq - T2) / ((T0 - T1) * (T0 - T2));
-                        l1 = (tq - T0) * (tq - T2) / ((T1 - T0) * (T1 - T2));
-                        l2 = (tq - T0) * (tq - T1) / ((T2 - T0) * (T2 - T1));
-                    } else {
-                        const double s = (tq - T1) / (T0 - T1);
-                        l0 = s;
-                        l1 = 1.0 - s;
-                    }
+                while (kout < A->o.n_out) {
+                    const double tq = t_start + kout * A->o.dt_out;
+                    if (tq > tn + 1e-9 * A->o.dt_out) break;
+                    double l0, l1, l2;
+                    step_pred(npts, tq, T0, T1, T2, l0, l1, l2);
 #pragma unroll
                     for (int r = 0; r < NR; r++)
                         if (ps[r] >= 0)
-                            wave[(size_t)kout * n_probe + ps[r]] = l0 * Uh0[r] + l1 * Uh1[r] + l2 * Uh2[r];
+                            wave[(size_t)kout * n_probe + ps[r]] = __builtin_fma(l0, Uh0[r], __builtin_fma(l1, Uh1[r], l2 * Uh2[r]));
                     kout++;
                 }
             }
@@ -811,16 +1206,20 @@ __device__ void run_lds(Rec& rec, const CPlan& c, const DPlan* __restrict__ P,
             if (hit && srcbp) {
                 npts = 1;
                 h = 0.1 * h;
-                if (h < sd.dt_min) h = sd.dt_min;
+                if (h < dt_min) h = dt_min;
             }
         }
     }
+    A = fresh(A);
+    c = fresh(c);
+    double* const ufin = A->u_final + A->u_off[inst];
 #pragma unroll
     for (int r = 0; r < NR; r++) {
         const int k = tid + W * r;
-        if (k < n) ufin[cn[r]] = (rc == CS_OK || steps > 0) ? Uh0[r] : v.u[k];
+        if (k < n) ufin[c->colnat[k]] = (rc == CS_OK || steps > 0) ? Uh0[r] : v.at(bu + 8 * k);
     }
     if (tid == 0) {
+        cs_tran_stats* const stp = A->stats + inst;
         stp->steps = steps;
         stp->rejected = rej;
         stp->newton_iters = nit;

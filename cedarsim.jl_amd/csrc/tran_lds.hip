@@ -8,9 +8,6 @@
 // LDS region beside its circuit's image.  Mixing a large circuit's instances
 // with a small circuit's fills both the wavefront slots and the LDS of a
 // workgroup, so that every instance of a batch can be resident at once.
-//
-// k_tran_lds: one wavefront per workgroup and instance (used with size
-// classes; the adjoint's forward pass has the same shape).
 #include "lds_core.h"
 
 namespace cedar {
@@ -19,86 +16,62 @@ namespace {
 
 using namespace lds;
 
-template <int NR>
-__global__ __launch_bounds__(W) void k_tran_lds(LdsArgs A) {
-    extern __shared__ double lds_mem[];
-    uint16_t* blob = reinterpret_cast<uint16_t*>(lds_mem + A.dbl_max);
-    int cur = -1;
-    for (;;) {
-        int qi = 0;
-        if (threadIdx.x == 0) qi = atomicAdd(A.queue, 1);
-        qi = __builtin_amdgcn_readfirstlane(__shfl(qi, 0, W));
-        if (qi >= A.n_inst) break;
-        const int inst = __builtin_amdgcn_readfirstlane(A.order[qi]);
-        const int cid = __builtin_amdgcn_readfirstlane(A.inst_cid[inst]);
-        const CPlan c = load_header(A.cplans + cid);
-        if (cid != cur) {
-            copy_image(c, blob, lane_id(), W);
-            cur = cid;
-            lds_sync();
-        }
-        const View v = make_view(lds_mem, blob, c);
-        NoRec rec;
-        run_lds<NR>(rec, c, A.plans + cid, A.params + A.p_off[inst],
-                    A.u0 ? A.u0 + A.u_off[inst] : nullptr,
-                    A.wave ? A.wave + A.w_off[inst] : nullptr, A.u_final + A.u_off[inst],
-                    A.stats + inst, A.o, v);
-    }
-}
-
-// Four wavefronts per SIMD (128 VGPRs): two workgroups of eight per CU, so
-// that every instance of a 4096-instance batch is resident at once; what the
-// register limit spills is step-control state outside the level loops.
-template <int NR>
-__global__ __launch_bounds__(W* kPackWaves) __attribute__((amdgpu_waves_per_eu(4, 4)))
-void k_tran_pack(LdsArgs A) {
+// Measured against the descriptor-driven form of this kernel (two-level index
+// lists per row and task, plan header in scalar registers, eight instances
+// per workgroup whatever the batch): 4096 rings of 11 to 101 stages over
+// 0.5 ns 394 -> 218 ms; 60 of them 309 -> 116 ms; one 33-stage ring 229 ->
+// 101 ms; 1001 inverters over 2 ns from their DC points 16.5 -> 11.0 ms.
+//
+// OCC wavefronts per SIMD.  OCC = 4 (128 VGPRs): two workgroups of eight per
+// CU, so that every instance of a 4096-instance batch is resident at once.
+// OCC = 2 (256 VGPRs) for batches that fill no more, and for circuits of
+// more than 128 rows (NR = 4), which are LDS-bound below that.  DYN: some
+// circuit has a source that is not DC.
+template <int NR, bool DYN, int OCC>
+__global__ __launch_bounds__(W* kPackWaves) __attribute__((amdgpu_waves_per_eu(OCC)))
+void k_tran_pack(const LdsArgs* args) {
+    constexpr bool ILP = NR <= 2 && OCC == 2;
     extern __shared__ double lds_mem[];
     __shared__ int s_chunk;
+    ConstPtr<LdsArgs> A = as_const(args);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     uint16_t* blob = reinterpret_cast<uint16_t*>(lds_mem);
     for (;;) {
-        if (threadIdx.x == 0) s_chunk = atomicAdd(A.queue, 1);
+        A = fresh(A);
+        if (threadIdx.x == 0) s_chunk = atomicAdd(A->queue, 1);
         __syncthreads();
         const int ch = __builtin_amdgcn_readfirstlane(s_chunk);
         __syncthreads();
-        if (ch >= A.n_chunks) break;
-        const int s0 = __builtin_amdgcn_readfirstlane(A.chunk_seg[ch]);
-        const int s1 = __builtin_amdgcn_readfirstlane(A.chunk_seg[ch + 1]);
+        if (ch >= A->n_chunks) break;
+        const int s0 = __builtin_amdgcn_readfirstlane(A->chunk_seg[ch]);
+        const int s1 = __builtin_amdgcn_readfirstlane(A->chunk_seg[ch + 1]);
         // every segment's plan image, at its own offset (multiples of 8 words)
         int seg = -1;
         for (int j = s0; j < s1; j++) {
-            const int4 sa = A.segs[2 * j], sb = A.segs[2 * j + 1];
-            const CPlan* cp = A.cplans + __builtin_amdgcn_readfirstlane(sa.x);
-            const uint4* src = reinterpret_cast<const uint4*>(cp->blob);
-            const int n16 = __builtin_amdgcn_readfirstlane(cp->words) / 8;
-            uint4* dst = reinterpret_cast<uint4*>(blob + __builtin_amdgcn_readfirstlane(sb.x));
-            for (int q = (int)threadIdx.x; q < n16; q += W * kPackWaves) dst[q] = src[q];
+            const int4 sa = A->segs[2 * j], sb = A->segs[2 * j + 1];
+            Hdr c = as_const(A->cplans + __builtin_amdgcn_readfirstlane(sa.x));
+            copy_image(c->blob, c->words, blob + __builtin_amdgcn_readfirstlane(sb.x), (int)threadIdx.x,
+                       (int)blockDim.x);
             const int w0 = __builtin_amdgcn_readfirstlane(sb.w), cnt = __builtin_amdgcn_readfirstlane(sa.z);
             if (wave >= w0 && wave < w0 + cnt) seg = j;
         }
         __syncthreads();
         if (seg >= 0) {
-            const int4 sa = A.segs[2 * seg], sb = A.segs[2 * seg + 1];
+            const int4 sa = A->segs[2 * seg], sb = A->segs[2 * seg + 1];
             const int cid = __builtin_amdgcn_readfirstlane(sa.x);
             const int k = wave - __builtin_amdgcn_readfirstlane(sb.w);
-            const int inst = __builtin_amdgcn_readfirstlane(A.order[__builtin_amdgcn_readfirstlane(sa.y) + k]);
+            const int inst = __builtin_amdgcn_readfirstlane(A->order[__builtin_amdgcn_readfirstlane(sa.y) + k]);
             // the circuit's own rows per lane (at most NR)
             const int nr = __builtin_amdgcn_readfirstlane(sa.w);
-            const CPlan c = load_header(A.cplans + cid);
             double* region = lds_mem + __builtin_amdgcn_readfirstlane(sb.y) +
                              (size_t)k * __builtin_amdgcn_readfirstlane(sb.z);
-            const View v = make_view(region, blob + __builtin_amdgcn_readfirstlane(sb.x), c);
+            const View v{reinterpret_cast<char*>(region), blob + __builtin_amdgcn_readfirstlane(sb.x)};
+            Hdr c = as_const(A->cplans + cid);
+            const DPlan* P = A->plans + cid;
             NoRec rec;
-            const double* pi = A.params + A.p_off[inst];
-            const double* u0 = A.u0 ? A.u0 + A.u_off[inst] : nullptr;
-            double* wv = A.wave ? A.wave + A.w_off[inst] : nullptr;
-            if (NR > 1 && nr == 1)
-                run_lds<1>(rec, c, A.plans + cid, pi, u0, wv, A.u_final + A.u_off[inst], A.stats + inst, A.o, v);
-            else if (NR > 2 && nr == 2)
-                run_lds<(NR > 2 ? 2 : NR)>(rec, c, A.plans + cid, pi, u0, wv, A.u_final + A.u_off[inst],
-                                           A.stats + inst, A.o, v);
-            else
-                run_lds<NR>(rec, c, A.plans + cid, pi, u0, wv, A.u_final + A.u_off[inst], A.stats + inst, A.o, v);
+            if (NR > 1 && nr == 1) run_lds<1, DYN, ILP>(rec, c, A, P, inst, v);
+            else if (NR > 2 && nr == 2) run_lds<(NR > 2 ? 2 : NR), DYN, ILP>(rec, c, A, P, inst, v);
+            else run_lds<NR, DYN, ILP>(rec, c, A, P, inst, v);
         }
         __syncthreads();
     }
@@ -117,36 +90,35 @@ __global__ __launch_bounds__(W) void k_lds_probe(const CPlan* cp, const DPlan* P
     constexpr int NM = 2 * NR;
     extern __shared__ double lds_mem[];
     uint16_t* blob = reinterpret_cast<uint16_t*>(lds_mem);
-    const CPlan c = load_header(cp);
-    copy_image(c, blob, lane_id(), W);
+    Hdr c = as_const(cp);
+    const int words = c->words, n = c->n, nnz = c->nnz;
+    copy_image(c->blob, words, blob, lane_id(), W);
     lds_sync();
-    const View v = make_view(lds_mem + c.words / 4, blob, c);
+    const View v{reinterpret_cast<char*>(lds_mem + words / 4), blob};
     DevRegs<NM> dr;
     setup_instance<NM>(c, P, p, v, dr);
-    double qx[NR], pinv[NR];
-    uint32_t flag[NR];
+    double qx[NR];
 #pragma unroll
     for (int r = 0; r < NR; r++) {
-        const int k = lane_id() + W * r;
-        qx[r] = k < c.n ? qx_piv[k] : 0.0;
-        pinv[r] = 0.0;
-        flag[r] = 0;
-        if (k < c.n) v.u[k] = u_piv[k];
+        const int k = row_of(lane_id(), r, n);
+        qx[r] = qx_piv[k];
+        v.at(c->b_u + 8 * k) = u_piv[k];
     }
     lds_sync();
-    eval_sources(c, v, t, mode);
+    eval_sources<true>(c, v, t, mode);
     lds_sync();
-    eval_mos<NM>(c, v, dr, p[P->p_gmin]);
+    const Hot h = load_hot(c);
+    eval_mos<NM, true>(h, v, dr, p[P->p_gmin]);
     lds_sync();
-    assemble<NR>(c, v, a0, qx, false, pinv, flag);
+    assemble<NR, true>(h, v, a0, qx);
     lds_sync();
-    for (int e = lane_id(); e < c.nnz; e += W) f_asm[e] = v.F[e];
-    for (int k = lane_id(); k < c.n; k += W) res_piv[k] = -v.x[k];
+    for (int e = lane_id(); e < nnz; e += W) f_asm[e] = v.at(c->b_F + 8 * e);
+    for (int k = lane_id(); k < n; k += W) res_piv[k] = -v.at(c->b_x + 8 * k);
     lds_sync();
-    factor_solve(c, v);
+    factor_solve<true>(h, v);
     lds_sync();
-    for (int e = lane_id(); e < c.nnz; e += W) f_lu[e] = v.F[e];
-    for (int k = lane_id(); k < c.n; k += W) dx_piv[k] = v.x[k];
+    for (int e = lane_id(); e < nnz; e += W) f_lu[e] = v.at(c->b_F + 8 * e);
+    for (int k = lane_id(); k < n; k += W) dx_piv[k] = v.at(c->b_x + 8 * k);
 }
 
 }  // namespace
@@ -166,52 +138,38 @@ hipError_t launch_lds_probe(int nr, const CPlan* cp, const DPlan* P, const doubl
     return hipGetLastError();
 }
 
-int pack_max_blocks(int nr, size_t lds) {
-    int nb = 0;
-    hipError_t e = hipErrorInvalidValue;
-    switch (nr) {
-        case 1: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_tran_pack<1>, W * kPackWaves, lds); break;
-        case 2: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_tran_pack<2>, W * kPackWaves, lds); break;
-        case 4: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_tran_pack<4>, W * kPackWaves, lds); break;
-        default: break;
+namespace {
+typedef void (*PackKernel)(const LdsArgs*);
+PackKernel pack_kernel(const PackShape& k) {
+    switch (k.nr) {
+        case 1:
+            if (k.occ == 4) return k.dyn ? k_tran_pack<1, true, 4> : k_tran_pack<1, false, 4>;
+            return k.dyn ? k_tran_pack<1, true, 2> : k_tran_pack<1, false, 2>;
+        case 2:
+            if (k.occ == 4) return k.dyn ? k_tran_pack<2, true, 4> : k_tran_pack<2, false, 4>;
+            return k.dyn ? k_tran_pack<2, true, 2> : k_tran_pack<2, false, 2>;
+        case 4: return k.dyn ? k_tran_pack<4, true, 2> : k_tran_pack<4, false, 2>;
+        default: return nullptr;
     }
-    return e == hipSuccess ? nb : 0;
+}
+}  // namespace
+
+int pack_max_blocks(const PackShape& k, size_t lds) {
+    int nb = 0;
+    const PackKernel f = pack_kernel(k);
+    if (!f || hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, W * k.waves, lds) != hipSuccess) return 0;
+    return nb;
 }
 
-hipError_t launch_tran_pack(int nr, const LdsArgs& a, int nblocks, size_t lds, hipStream_t s) {
-    switch (nr) {
-        case 1: hipLaunchKernelGGL(k_tran_pack<1>, dim3(nblocks), dim3(W * kPackWaves), lds, s, a); break;
-        case 2: hipLaunchKernelGGL(k_tran_pack<2>, dim3(nblocks), dim3(W * kPackWaves), lds, s, a); break;
-        case 4: hipLaunchKernelGGL(k_tran_pack<4>, dim3(nblocks), dim3(W * kPackWaves), lds, s, a); break;
-        default: return hipErrorInvalidValue;
-    }
+hipError_t launch_tran_pack(const PackShape& k, const LdsArgs* d_args, int nblocks, size_t lds, hipStream_t s) {
+    const PackKernel f = pack_kernel(k);
+    if (!f) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(f, dim3(nblocks), dim3(W * k.waves), lds, s, d_args);
     return hipGetLastError();
 }
 
 size_t lds_kernel_bytes(int32_t dbl_max, int32_t words_max) {
     return 8 * (size_t)dbl_max + 2 * (size_t)words_max;
-}
-
-int lds_max_blocks(int nr, size_t lds) {
-    int nb = 0;
-    hipError_t e = hipErrorInvalidValue;
-    switch (nr) {
-        case 1: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_tran_lds<1>, W, lds); break;
-        case 2: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_tran_lds<2>, W, lds); break;
-        case 4: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_tran_lds<4>, W, lds); break;
-        default: break;
-    }
-    return e == hipSuccess ? nb : 0;
-}
-
-hipError_t launch_tran_lds(int nr, const LdsArgs& a, int nblocks, size_t lds, hipStream_t s) {
-    switch (nr) {
-        case 1: hipLaunchKernelGGL(k_tran_lds<1>, dim3(nblocks), dim3(W), lds, s, a); break;
-        case 2: hipLaunchKernelGGL(k_tran_lds<2>, dim3(nblocks), dim3(W), lds, s, a); break;
-        case 4: hipLaunchKernelGGL(k_tran_lds<4>, dim3(nblocks), dim3(W), lds, s, a); break;
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
 }
 
 }  // namespace cedar

@@ -209,7 +209,8 @@ const char* cs_last_error(const cs_ctx* ctx);
 int cs_analyze(const cs_netlist* nl, cs_circuit_info* info, int32_t* lu_rowptr,
                int32_t* lu_col, int32_t* rownat, int32_t* colnat);
 /* The packed batched launch's chunks for counts[c] instances of each of the
- * n_circ circuits (the same packing as cs_batch_create, host only; no
+ * n_circ circuits (the same packing as cs_batch_create uses for a batch of
+ * more than 7 instances per CU, which fills its chunks; host only; no
  * counterpart in the reference, a check of the batching): chunk k's segments
  * (circuit index, instance count) are seg_circ/seg_count[seg_ptr[k] ..
  * seg_ptr[k+1]-1], chunks in packing order (largest circuit first, before
