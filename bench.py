@@ -18,6 +18,7 @@ the CPU oracle (OpenMP across instances) on a bounded sample; both are
 reported as instances/s.  Prints one JSON line.
 """
 import argparse
+import dataclasses
 import json
 import os
 import sys
@@ -238,10 +239,11 @@ def main():
     if not args.no_plain and args.plain_sample > 0:
         # plain per-instance path over the full span, on the first instances
         idx = list(range(args.plain_sample))
+        popts = dataclasses.replace(opts, batch_kernel=L.BATCH_KERNEL_GLOBAL)   # cs_tran's plain path
         t0 = time.perf_counter()
         for i in idx:
             s = systems[inst_sys[i]]
-            sol = s.tran(opts, params[i], u0s[i])
+            sol = s.tran(popts, params[i], u0s[i])
             if sol.retcode != "Success":
                 log(f"plain instance {i} failed: {sol.retcode}")
         dt = time.perf_counter() - t0

@@ -50,6 +50,16 @@ struct Circuit {
     std::string compact_why;
     CPlan hcp{};                // device pointers, host copy
     void* cbuf = nullptr;
+    const CPlan* d_cplan = nullptr;
+    // one instance on the LDS-resident kernel (cs_tran, cs_dcop): a device
+    // buffer and its pinned image, kept and grown from call to call
+    int32_t lds_nr = 0;         // rows per lane, 0: does not fit
+    std::string lds_why;
+    bool lds_dyn = false;
+    size_t lds_bytes = 0;
+    char* sbuf = nullptr;
+    char* h_sbuf = nullptr;
+    size_t sbuf_bytes = 0;
     // large circuits: the supernodal path (big.h) instead of all of the above
     BigCircuit* big = nullptr;
 };
@@ -140,8 +150,29 @@ struct Packer {
     }
 };
 
-// The LDS plan image and its pivot-order side arrays in one allocation (the
-// image first, 16-byte aligned).  A circuit whose indices do not fit 16 bits
+// Rows per lane of the LDS-resident kernels, or why the circuit does not fit.
+void lds_shape(Circuit& C) {
+    C.lds_nr = 0;
+    if (!C.compact_ok) { C.lds_why = C.compact_why; return; }
+    const CPlan& cp = C.hcp;
+    int32_t nr = cp.n <= 64 ? 1 : cp.n <= 128 ? 2 : 4;
+    while (nr < 4 && cp.n_mos > 128 * nr) nr *= 2;
+    if (cp.n > 64 * nr || cp.n_mos > 128 * nr || cp.n_src > 64 * 64) {
+        C.lds_why = "circuit exceeds the LDS-resident kernel's per-lane limits (256 unknowns, 512 devices)";
+        return;
+    }
+    C.lds_bytes = lds_kernel_bytes((cp.dbl + 1) & ~1, cp.words);
+    if (C.lds_bytes > kLdsMaxBytes) {
+        C.lds_why = "circuit needs more LDS than one workgroup may hold";
+        return;
+    }
+    C.lds_nr = nr;
+    C.lds_dyn = false;
+    for (const SrcDesc& d : C.plan.src) C.lds_dyn = C.lds_dyn || d.kind != CS_WAVE_DC;
+}
+
+// The plan header, the LDS plan image and its pivot-order side arrays in one
+// allocation (the image 16-byte aligned).  A circuit whose indices do not fit 16 bits
 // keeps compact_ok = false and runs on the global-plan kernel.
 int upload_compact(cs_ctx* ctx, Circuit& C) {
     std::vector<uint16_t> blob;
@@ -151,12 +182,15 @@ int upload_compact(cs_ctx* ctx, Circuit& C) {
     if (C.cbuf) { (void)hipFree(C.cbuf); C.cbuf = nullptr; }
     C.compact_ok = build_compact(C.plan, blob, cp, lpos, colnat, diffrow, probe, dev, devrow, &why);
     C.compact_why = why;
-    if (!C.compact_ok) return CS_OK;
+    if (!C.compact_ok) {
+        lds_shape(C);
+        return CS_OK;
+    }
     Packer pk;
+    const size_t o_hdr = pk.add(std::vector<CPlan>(1));
     size_t o_blob = pk.add(blob), o_lp = pk.add(lpos), o_cn = pk.add(colnat), o_df = pk.add(diffrow), o_pr = pk.add(probe),
            o_dev = pk.add(dev), o_dr = pk.add(devrow);
     HIPCHK(ctx, hipMalloc(&C.cbuf, pk.bytes.size()));
-    HIPCHK(ctx, hipMemcpy(C.cbuf, pk.bytes.data(), pk.bytes.size(), hipMemcpyHostToDevice));
     char* b = (char*)C.cbuf;
     cp.blob = (const uint16_t*)(b + o_blob);
     cp.lpos = (const int32_t*)(b + o_lp);
@@ -168,6 +202,10 @@ int upload_compact(cs_ctx* ctx, Circuit& C) {
     cp.mos_m = C.hd.mos_m;
     cp.src_m = C.hd.src_m;
     C.hcp = cp;
+    std::memcpy(pk.bytes.data() + o_hdr, &cp, sizeof(CPlan));
+    HIPCHK(ctx, hipMemcpy(C.cbuf, pk.bytes.data(), pk.bytes.size(), hipMemcpyHostToDevice));
+    C.d_cplan = (const CPlan*)(b + o_hdr);
+    lds_shape(C);
     return CS_OK;
 }
 
@@ -455,6 +493,8 @@ int cs_destroy(cs_ctx* ctx) {
             if (c->h_norm) (void)hipHostFree(c->h_norm);
             if (c->h_stage) (void)hipHostFree(c->h_stage);
             if (c->cbuf) (void)hipFree(c->cbuf);
+            if (c->sbuf) (void)hipFree(c->sbuf);
+            if (c->h_sbuf) (void)hipHostFree(c->h_sbuf);
             if (c->big) big_destroy(c->big);
         }
     for (hipStream_t st : ctx->side) (void)hipStreamDestroy(st);
@@ -819,6 +859,9 @@ void cs_tran_opts_default(cs_tran_opts* o) {
     o->reserved = 0;
 }
 
+static int dcop_single(cs_ctx* ctx, Circuit& C, const double* p, const cs_tran_opts* o, double* u_out,
+                       cs_tran_stats* st);
+
 int cs_dcop(cs_ctx* ctx, int32_t cid, const double* p, const cs_tran_opts* o, double* u_out,
             cs_tran_stats* st) {
     Circuit* C = get_circuit(ctx, cid);
@@ -832,6 +875,7 @@ int cs_dcop(cs_ctx* ctx, int32_t cid, const double* p, const cs_tran_opts* o, do
         if (rc) ctx->err = err;
         return rc;
     }
+    if (C->lds_nr) return dcop_single(ctx, *C, p, o, u_out, st);
     if ((rc = ensure_workspace(ctx, *C)) || (rc = ensure_graph(ctx, *C))) return rc;
     const Plan& P = C->plan;
     HIPCHK(ctx, hipMemcpyAsync(C->w.p, p, sizeof(double) * P.lay.n_params, hipMemcpyHostToDevice, ctx->stream));
@@ -1195,40 +1239,165 @@ static int tran_plain(cs_ctx* ctx, int32_t cid, const double* p, const double* u
 }
 
 
-// cs_tran with batch_kernel = CS_BATCH_KERNEL_LDS: the circuit runs as a batch
-// of one in the LDS-resident kernel, its whole transient in one launch instead
-// of a launch and a host round trip per Newton iteration.  The outputs and the
-// return code are those of the plain path (the instance's retcode).
-static int tran_batch_of_one(cs_ctx* ctx, int32_t cid, const double* p, const double* u0,
-                             const cs_tran_opts* o, double* wave, double* u_final, cs_tran_stats* st_out) {
-    Circuit* C = get_circuit(ctx, cid);
-    if (!C) return fail(ctx, CS_E_INVALID, "bad argument");
-    if (C->big)
-        return fail(ctx, CS_E_INVALID,
-                    "the LDS-resident kernel runs level-scheduled circuits, not the supernodal solver");
-    int32_t bid = -1;
-    int rc = cs_batch_create(ctx, 1, &cid, p, u0, o, &bid);
+// ---- one instance on the LDS-resident kernel ------------------------------------------
+// The whole analysis in one launch, where the plain path takes a graph launch
+// and a host round trip per Newton iteration.  The circuit keeps the device
+// buffer and its pinned image: one copy up (arguments, parameters, initial
+// state), the kernel, one copy down (stats, final state, waveform).
+struct SingleRun {
+    LdsArgs* args;          // in the pinned image
+    double *p, *u0;
+    cs_tran_stats* st;      // results, in the pinned image
+    double *u, *wave;
+    char* d_args;
+    size_t up, down0, down; // bytes to copy up; the results' range
+};
+
+static int single_buffers(cs_ctx* ctx, Circuit& C, const cs_tran_opts& o, bool with_u0, int32_t n_out, SingleRun& R) {
+    const Plan& P = C.plan;
+    size_t at = 0;
+    auto take = [&](size_t bytes) { const size_t off = at; at = (at + bytes + 15) & ~size_t(15); return off; };
+    const size_t n_wave = (size_t)n_out * P.probe.size();
+    const size_t o_args = take(sizeof(LdsArgs)), o_z = take(64), o_segs = take(2 * sizeof(int4)),
+                 o_p = take(sizeof(double) * P.lay.n_params), o_u0 = take(sizeof(double) * P.n);
+    R.up = at;
+    const size_t o_st = take(sizeof(cs_tran_stats)), o_u = take(sizeof(double) * P.n), o_w = take(sizeof(double) * n_wave);
+    R.down0 = o_st;
+    R.down = at - o_st;
+    if (at > C.sbuf_bytes) {
+        if (C.sbuf) (void)hipFree(C.sbuf);
+        if (C.h_sbuf) (void)hipHostFree(C.h_sbuf);
+        C.sbuf = C.h_sbuf = nullptr;
+        C.sbuf_bytes = 0;
+        const size_t bytes = at + at / 4;
+        HIPCHK(ctx, hipMalloc((void**)&C.sbuf, bytes));
+        HIPCHK(ctx, hipHostMalloc((void**)&C.h_sbuf, bytes, hipHostMallocDefault));
+        C.sbuf_bytes = bytes;
+    }
+    char *h = C.h_sbuf, *d = C.sbuf;
+    std::memset(h, 0, o_p);
+    // zeros at o_z: offsets, instance and circuit numbers; then the queue, and
+    // the chunk's segment range (0, 1)
+    int32_t* z = (int32_t*)(h + o_z);
+    z[9] = 1;
+    int4* sg = (int4*)(h + o_segs);
+    sg[0] = make_int4(0, 0, 1, C.lds_nr);
+    sg[1] = make_int4(0, C.hcp.words / 4, (C.hcp.dbl + 1) & ~1, 0);
+    R.args = (LdsArgs*)(h + o_args);
+    R.p = (double*)(h + o_p);
+    R.u0 = (double*)(h + o_u0);
+    R.st = (cs_tran_stats*)(h + o_st);
+    R.u = (double*)(h + o_u);
+    R.wave = (double*)(h + o_w);
+    R.d_args = d + o_args;
+    LdsArgs& a = *R.args;
+    a.cplans = C.d_cplan;
+    a.plans = C.d_dplan;
+    a.inst_cid = (const int32_t*)(d + o_z);
+    a.p_off = a.u_off = a.w_off = (const int64_t*)(d + o_z);
+    a.params = (const double*)(d + o_p);
+    a.u0 = with_u0 ? (const double*)(d + o_u0) : nullptr;
+    a.wave = n_wave ? (double*)(d + o_w) : nullptr;
+    a.u_final = (double*)(d + o_u);
+    a.stats = (cs_tran_stats*)(d + o_st);
+    a.order = (const int32_t*)(d + o_z);
+    a.queue = (int32_t*)(d + o_z + 16);
+    a.n_inst = 1;
+    a.o = o;
+    a.o.n_out = n_out;
+    a.segs = (const int4*)(d + o_segs);
+    a.chunk_seg = (const int32_t*)(d + o_z + 32);
+    a.n_chunks = 1;
+    return CS_OK;
+}
+
+static int tran_single(cs_ctx* ctx, Circuit& C, const double* p, const double* u0, const cs_tran_opts* o,
+                       double* wave, double* u_final, cs_tran_stats* st_out) {
+    const Plan& P = C.plan;
+    if (o->init == CS_INIT_UIC && !u0) return fail(ctx, CS_E_INVALID, "UIC initialisation needs u0");
+    if (o->init == CS_INIT_UIC && !P.uic_ok)
+        return fail(ctx, CS_E_INVALID, "UIC: a charge-carrying row could not be kept on its own pivot");
+    if (o->n_out > 0 && !(o->dt_out > 0)) return fail(ctx, CS_E_INVALID, "dt_out must be > 0");
+    (void)hipSetDevice(ctx->device);
+    const int32_t n_out = wave ? std::max(o->n_out, 0) : 0;
+    SingleRun R{};
+    int rc = single_buffers(ctx, C, *o, u0 != nullptr, n_out, R);
     if (rc) return rc;
-    cs_tran_stats st{};
-    double ms = 0.0;
-    rc = cs_batch_run(ctx, bid, &ms);
-    if (rc == CS_OK) rc = cs_batch_results(ctx, bid, wave, u_final, &st);
-    const std::string err = ctx->err;
-    (void)cs_batch_destroy(ctx, bid);
-    ctx->err = err;
-    if (rc) return rc;
-    if (st_out) *st_out = st;
-    rc = st.retcode;
+    std::memcpy(R.p, p, sizeof(double) * P.lay.n_params);
+    if (u0) std::memcpy(R.u0, u0, sizeof(double) * P.n);
+    hipStream_t s = ctx->stream;
+    PackShape k;
+    k.nr = C.lds_nr;
+    k.dyn = C.lds_dyn;
+    HIPCHK(ctx, hipMemcpyAsync(C.sbuf, C.h_sbuf, R.up, hipMemcpyHostToDevice, s));
+    HIPCHK(ctx, launch_tran_pack(k, (const LdsArgs*)R.d_args, 1, C.lds_bytes, s));
+    HIPCHK(ctx, hipMemcpyAsync(C.h_sbuf + R.down0, C.sbuf + R.down0, R.down, hipMemcpyDeviceToHost, s));
+    HIPCHK(ctx, hipStreamSynchronize(s));
+    // the samples up to the time reached; a run that stops early leaves the others
+    int32_t rows = 0;
+    if (R.st->retcode != CS_E_NOCONV)
+        while (rows < n_out && o->t_start + rows * o->dt_out <= R.st->t_end + 1e-9 * o->dt_out) rows++;
+    if (rows) std::memcpy(wave, R.wave, sizeof(double) * (size_t)rows * P.probe.size());
+    if (u_final) std::memcpy(u_final, R.u, sizeof(double) * P.n);
+    R.st->busy_s /= ctx->clock_hz;
+    if (st_out) *st_out = *R.st;
+    rc = R.st->retcode;
     if (rc == CS_E_DTMIN) ctx->err = "transient: step size fell below dt_min";
-    else if (rc == CS_E_NOCONV) ctx->err = "transient: initial point did not converge";
+    else if (rc == CS_E_NOCONV)
+        ctx->err = std::string("transient: initial point did not converge") +
+                   (o->init == CS_INIT_UIC ? "" : dc_pivot_note(P));
     else if (rc == CS_E_MAXSTEPS) ctx->err = "transient: max_steps reached";
+    return rc;
+}
+
+// The DC operating point on the same kernel code (k_lds_dcop).
+static int dcop_single(cs_ctx* ctx, Circuit& C, const double* p, const cs_tran_opts* o, double* u_out,
+                       cs_tran_stats* st) {
+    const Plan& P = C.plan;
+    SingleRun R{};
+    int rc = single_buffers(ctx, C, *o, false, 0, R);
+    if (rc) return rc;
+    std::memcpy(R.p, p, sizeof(double) * P.lay.n_params);
+    hipStream_t s = ctx->stream;
+    HIPCHK(ctx, hipMemcpyAsync(C.sbuf, C.h_sbuf, R.up, hipMemcpyHostToDevice, s));
+    HIPCHK(ctx, launch_lds_dcop(C.lds_nr, C.lds_dyn, (const LdsArgs*)R.d_args, C.lds_bytes, s));
+    HIPCHK(ctx, hipMemcpyAsync(C.h_sbuf + R.down0, C.sbuf + R.down0, R.down, hipMemcpyDeviceToHost, s));
+    HIPCHK(ctx, hipStreamSynchronize(s));
+    std::memcpy(u_out, R.u, sizeof(double) * P.n);
+    rc = R.st->retcode;
+    if (st) {
+        std::memset(st, 0, sizeof(*st));
+        st->newton_iters = R.st->newton_iters;
+        st->retcode = rc;
+        st->t_end = o->t_start;
+    }
+    if (rc == CS_E_NOCONV) ctx->err = "DC operating point analysis failed" + dc_pivot_note(P);
     return rc;
 }
 
 int cs_tran(cs_ctx* ctx, int32_t cid, const double* p, const double* u0, const cs_tran_opts* o,
             double* wave, double* u_final, cs_tran_stats* st_out) {
-    if (o && o->batch_kernel == CS_BATCH_KERNEL_LDS)
-        return tran_batch_of_one(ctx, cid, p, u0, o, wave, u_final, st_out);
+    Circuit* C = get_circuit(ctx, cid);
+    if (o && o->batch_kernel == CS_BATCH_KERNEL_LDS) {
+        if (!C || !p) return fail(ctx, CS_E_INVALID, "bad argument");
+        if (C->big)
+            return fail(ctx, CS_E_INVALID,
+                        "the LDS-resident kernel runs level-scheduled circuits, not the supernodal solver");
+        if (o->jac_reuse)
+            return fail(ctx, CS_E_INVALID, "jac_reuse (modified Newton) runs on cs_tran, not in batches");
+        if (!C->lds_nr) return fail(ctx, CS_E_RANGE, "LDS-resident batch kernel: " + C->lds_why);
+        return tran_single(ctx, *C, p, u0, o, wave, u_final, st_out);
+    }
+    // AUTO takes the LDS-resident kernel where the circuit fits it: the same
+    // rules and step sequence, 5 us per Newton iteration of a small circuit
+    // against 90 (an inverter over 4 ns 165 -> 11.9 ms).  Modified Newton,
+    // Verilog-A devices and larger circuits stay on the plain path, and
+    // CS_BATCH_KERNEL_GLOBAL asks for it.  Without nonlinear devices the
+    // factors modified Newton keeps are those full Newton recomputes, so such
+    // a circuit takes the same kernel and the same bits either way.
+    if (o && C && p && !C->big && C->lds_nr && o->batch_kernel == CS_BATCH_KERNEL_AUTO &&
+        (o->jac_reuse == 0 || (o->jac_reuse == 1 && C->plan.n_mos == 0)))
+        return tran_single(ctx, *C, p, u0, o, wave, u_final, st_out);
     return tran_plain(ctx, cid, p, u0, o, wave, u_final, st_out, nullptr);
 }
 
@@ -1274,12 +1443,6 @@ int cs_tran_sens(cs_ctx* ctx, int32_t cid, const double* p, const double* u0, co
     if (rc == CS_OK) rc = tran_plain(ctx, cid, p, u0, o, wave, u_final, st_out, &R);
     (void)hipFree(R.buf);
     return rc;
-}
-
-static bool has_dynamic_source(const Plan& P) {
-    for (const SrcDesc& d : P.src)
-        if (d.kind != CS_WAVE_DC) return true;
-    return false;
 }
 
 // The arguments every LDS-resident launch of a batch shares.
@@ -1341,7 +1504,7 @@ static int build_lds_classes(cs_ctx* ctx, Batch& B, const std::function<int(void
             dbl_max = std::max(dbl_max, (cp.dbl + 1) & ~1);
             words_max = std::max(words_max, cp.words_adj);
             L.nr = std::max(L.nr, B.c_nr[c]);
-            L.dyn = L.dyn || has_dynamic_source(ctx->circuits[c]->plan);
+            L.dyn = L.dyn || ctx->circuits[c]->lds_dyn;
         }
         std::vector<int32_t> order;
         for (int32_t i = 0; i < B.n_inst; i++)
@@ -1405,7 +1568,7 @@ static int build_pack(cs_ctx* ctx, Batch& B, const std::function<int(void**, siz
         dblb[c] = 8 * (size_t)((cp.dbl + 1) & ~1);
         if (img[c] + dblb[c] > kPackLds) return CS_E_RANGE;
         ks.nr = std::max(ks.nr, c_nr[c]);
-        ks.dyn = ks.dyn || has_dynamic_source(ctx->circuits[c]->plan);
+        ks.dyn = ks.dyn || ctx->circuits[c]->lds_dyn;
     }
     const int64_t n_cu = std::max(ctx->n_cu, 1);
     ks.waves = (int32_t)std::min<int64_t>(kPackWaves, (B.n_inst + n_cu - 1) / n_cu);
@@ -1543,22 +1706,8 @@ int cs_batch_create(cs_ctx* ctx, int32_t n_inst, const int32_t* inst_cid, const 
     bool lds_fits = true;
     for (int32_t c : used) {
         const Circuit& C = *ctx->circuits[c];
-        if (!C.compact_ok) { lds_fits = false; lds_why = C.compact_why; break; }
-        const CPlan& cp = C.hcp;
-        int32_t nr = cp.n <= 64 ? 1 : cp.n <= 128 ? 2 : 4;
-        while (nr < 4 && cp.n_mos > 128 * nr) nr *= 2;
-        if (cp.n > 64 * nr || cp.n_mos > 128 * nr || cp.n_src > 64 * 64) {
-            lds_fits = false;
-            lds_why = "circuit exceeds the LDS-resident kernel's per-lane limits (256 unknowns, 512 devices)";
-            break;
-        }
-        const size_t need = lds_kernel_bytes((cp.dbl + 1) & ~1, cp.words);
-        if (need > kLdsMaxBytes) {
-            lds_fits = false;
-            lds_why = "circuit needs more LDS than one workgroup may hold";
-            break;
-        }
-        c_nr[c] = nr;
+        if (!C.lds_nr) { lds_fits = false; lds_why = C.lds_why; break; }
+        c_nr[c] = C.lds_nr;
     }
     if (want == CS_BATCH_KERNEL_LDS && !lds_fits)
         return fail(ctx, CS_E_RANGE, "LDS-resident batch kernel: " + lds_why);

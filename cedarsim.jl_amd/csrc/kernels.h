@@ -211,6 +211,8 @@ struct PackShape {
 };
 int pack_max_blocks(const PackShape& k, size_t lds);   // resident workgroups per CU
 hipError_t launch_tran_pack(const PackShape& k, const LdsArgs* d_args, int nblocks, size_t lds, hipStream_t s);
+// DC operating point of one circuit (args: its plans, params, u_final, stats, o)
+hipError_t launch_lds_dcop(int nr, bool dyn, const LdsArgs* d_args, size_t lds, hipStream_t s);
 // one recorded Newton iteration of the LDS-resident instance code (pivot order)
 hipError_t launch_lds_probe(int nr, const CPlan* cp, const DPlan* P, const double* p, const double* u_piv,
                             const double* qx_piv, double a0, double t, int mode, double* f_asm,

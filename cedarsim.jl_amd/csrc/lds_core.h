@@ -898,10 +898,11 @@ __device__ __forceinline__ void dc_set_start(Hdr c, const View& v, int j) {
 //   phase -1   pinned (UIC, or after the DC point), at most 50 iterations;
 //   phase 0-9  trajectory j from its own start, at most 200 iterations;
 //   phase 10   the gmin ladder from trajectory 0's start, stage by stage.
-template <int NR, int NM, bool DYN>
+// dc_only ends with the DC point.
+template <int NR, int NM, bool DYN, bool ILP>
 __device__ __forceinline__ bool init_point(Hdr c, const View& v, const DPlan* __restrict__ P, const DevRegs<NM>& dr,
                                            double gmin, bool uic, double (&pinv)[NR], const uint32_t (&flag)[NR],
-                                           double t0, double dc_abstol, long long& nit) {
+                                           double t0, double dc_abstol, long long& nit, bool dc_only = false) {
     const int tid = lane_id();
     double qx0[NR];
 #pragma unroll
@@ -914,9 +915,9 @@ __device__ __forceinline__ bool init_point(Hdr c, const View& v, const DPlan* __
     lds_sync();
     for (;;) {
         const Hot h = load_hot(c);
-        eval_mos<NM, false>(h, v, dr, g);
+        eval_mos<NM, ILP>(h, v, dr, g);
         lds_sync();
-        assemble<NR, false>(h, v, 0.0, qx0);
+        assemble<NR, ILP>(h, v, 0.0, qx0);
         if (pin) apply_pins<NR>(c, v, P, pinv, flag);
         lds_sync();
         const double fn = residual_max<NR>(c, v);
@@ -931,7 +932,7 @@ __device__ __forceinline__ bool init_point(Hdr c, const View& v, const DPlan* __
                     continue;
                 }
             }
-            if (!dc_done) return true;                       // the pinned phase converged
+            if (!dc_done || dc_only) return true;            // the pinned phase converged, or the DC point is all
             // the DC point: pin its charge rows, sources at their t0 values
 #pragma unroll
             for (int r = 0; r < NR; r++) {
@@ -959,7 +960,7 @@ __device__ __forceinline__ bool init_point(Hdr c, const View& v, const DPlan* __
             lds_sync();
             continue;
         }
-        factor_solve<false>(h, v);
+        factor_solve<ILP>(h, v);
 #pragma unroll
         for (int r = 0; r < NR; r++) {
             const int k = tid + W * r;
@@ -1049,7 +1050,7 @@ __device__ __forceinline__ void run_lds(Rec& rec, Hdr c, ConstPtr<LdsArgs> A, co
     lds_sync();
 
     long long steps = 0, rej = 0, nit = 0;
-    int rc = init_point<NR, NM, DYN>(c, v, P, dr, gmin, uic, pinv, flag, A->o.t_start, A->o.dc_abstol, nit)
+    int rc = init_point<NR, NM, DYN, ILP>(c, v, P, dr, gmin, uic, pinv, flag, A->o.t_start, A->o.dc_abstol, nit)
                  ? CS_OK : CS_E_NOCONV;
 
     A = fresh(A);

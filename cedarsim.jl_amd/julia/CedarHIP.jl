@@ -435,7 +435,7 @@ function CedarSim.tran!(circ, tspan, be::HIPBackend; reltol=1e-6, abstol=1e-9, n
     o.dt_out = (tspan[2] - tspan[1]) / (n_out - 1)
     o.init = u0 === nothing ? CS_INIT_DCOP : CS_INIT_UIC
     o.jac_reuse = jac_reuse && kernel == :plain ? 1 : 0   # IDA's Jacobian reuse within a step
-    o.batch_kernel = kernel == :lds ? CS_BATCH_KERNEL_LDS : CS_BATCH_KERNEL_AUTO
+    o.batch_kernel = kernel == :lds ? CS_BATCH_KERNEL_LDS : CS_BATCH_KERNEL_GLOBAL
     wave = zeros(s.n, n_out)                         # column k = sample k
     uf = zeros(s.n)
     st = CsTranStats()

@@ -316,15 +316,18 @@ void cs_tran_opts_default(cs_tran_opts* o);
 /* dc!(circ): Newton on F(0,u,p,0)=0 in DC mode (src/dcop.jl:53-155). */
 int cs_dcop(cs_ctx* ctx, int32_t cid, const double* p, const cs_tran_opts* o,
             double* u_out, cs_tran_stats* st);
-/* tran!(circ, tspan): the plain per-instance GPU path.  The host runs the
- * BDF step control; every Newton iteration is one launch of a captured
- * hipGraph (device eval -> assembly -> LU refactor -> solve -> norm).
+/* tran!(circ, tspan).  By default a circuit that fits runs its whole transient
+ * in one launch of the LDS-resident kernel, as a batch of one; circuits that
+ * do not fit (more than 256 unknowns or 512 devices, Verilog-A devices, 64 KiB
+ * of LDS), supernodal ones, and modified Newton (jac_reuse) on a circuit with
+ * nonlinear devices take the plain path: the host runs the BDF step control
+ * and every Newton iteration is one launch of a captured hipGraph (device
+ * eval -> assembly -> LU refactor -> solve -> norm).  Both follow the same
+ * rules; results agree to rounding.  o->batch_kernel = CS_BATCH_KERNEL_LDS
+ * asks for the first (refused for supernodal circuits, circuits that do not
+ * fit, and jac_reuse), CS_BATCH_KERNEL_GLOBAL for the plain path.
  * wave: n_out x n_probe samples; u_final: n.  u0 may be NULL for INIT_DCOP.
- * With o->batch_kernel = CS_BATCH_KERNEL_LDS the circuit instead runs as a
- * batch of one in the LDS-resident kernel (the whole transient in one
- * launch; same outputs and return code; refused for supernodal circuits,
- * circuits that do not fit, and jac_reuse).  Other batch_kernel values: the
- * plain path. */
+ * cs_dcop takes the same kernel code where the circuit fits. */
 int cs_tran(cs_ctx* ctx, int32_t cid, const double* p, const double* u0,
             const cs_tran_opts* o, double* wave, double* u_final,
             cs_tran_stats* st);

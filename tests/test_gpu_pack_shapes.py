@@ -59,3 +59,58 @@ def test_packed_shapes_match_oracle(engine, kind, count):
         assert r.stats[i].steps == st[q].steps
         assert np.all(np.abs(r.wave[i] - w[q]) <= 1e-6 * np.abs(w[q]) + 1e-9)
         assert np.all(np.abs(r.u_final[i] - uf[q]) <= 1e-6 * np.abs(uf[q]) + 1e-9)
+
+
+@pytest.mark.parametrize("name", ["inverter", "ring5", "ring67", "ring149", "mesh", "butterworth", "vr"])
+def test_cs_tran_and_dcop_take_one_launch(engine, name):
+    """cs_tran by default and cs_dcop on the LDS-resident kernel against the
+    plain path (batch_kernel = CS_BATCH_KERNEL_GLOBAL) and the oracle, with
+    probes, without an output grid, and a second call with other values."""
+    import circuits as K
+    print(f"[gpu] single launch {name}", flush=True)
+    rng = np.random.default_rng(4)
+    u0 = None
+    if name.startswith("ring"):
+        flat, span = ch.lower(ring_oscillator(int(name[4:]))), 4e-12
+        u0 = ring_initial_state(flat, rng)
+    else:
+        flat, span = {"inverter": (ch.lower(inverter()), 0.3e-9), "mesh": (rc_mesh(7, 6, 5, seed=3), 20e-12),
+                      "butterworth": (ch.lower(K.butterworth), 0.5), "vr": (ch.lower(K.vr), 1e-3)}[name]
+    s = engine.load(flat, solver=L.SOLVER_LEVEL)
+    kw = {"init": L.INIT_UIC} if u0 is not None else {}
+    for trial in range(2):
+        p = flat.params()
+        if trial and len(flat.arrays["mos_vth"]):
+            p[flat.layout()["mos_vth"]] += 0.05
+        o = ch.grid_options((0.0, span), n_out=7, **kw)
+        w, uf, st, rc = O.tran(flat, p, u0, o)
+        a = s.tran(o, p, u0)
+        b = s.tran(ch.grid_options((0.0, span), n_out=7, batch_kernel=L.BATCH_KERNEL_GLOBAL, **kw), p, u0)
+        c = s.tran(ch.TranOptions(t_start=0.0, t_stop=span, **kw), p, u0)
+        assert a.retcode == b.retcode == c.retcode == "Success" and rc == 0
+        assert a.stats.steps == b.stats.steps == st.steps and a.stats.newton_iters == b.stats.newton_iters
+        for r in (a, b):
+            assert np.all(np.abs(r.wave - w) <= 1e-6 * np.abs(w) + 1e-9)
+            assert np.all(np.abs(r.u_final - uf) <= 1e-6 * np.abs(uf) + 1e-9)
+        assert np.array_equal(c.u_final, a.u_final) and c.wave.shape[0] == 0
+        if u0 is None:
+            ud, _, rcd = O.dcop(flat, p)
+            dc = s.dcop(p)
+            assert dc.retcode == "Success" and rcd == 0
+            assert np.max(np.abs(dc.u - ud)) <= 1e-9 * max(1.0, np.max(np.abs(ud)))
+    s.set_probes([1, 0])
+    d = s.tran(ch.grid_options((0.0, span), n_out=7, **kw), p, u0)
+    assert np.array_equal(d.wave, a.wave[:, [1, 0]])
+
+
+def test_early_stop_leaves_later_samples(engine):
+    """A run that ends at max_steps fills the samples up to its time only, on both kernels."""
+    print("[gpu] early stop", flush=True)
+    flat = ch.lower(inverter())
+    s = engine.load(flat)
+    for kern in (L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_GLOBAL):
+        r = s.tran(ch.grid_options((0.0, 1e-9), n_out=101, max_steps=150, batch_kernel=kern))
+        assert r.retcode == "MaxIters" and r.stats.steps + r.stats.rejected == 150
+        done = r.t <= r.stats.t_end * (1 + 1e-9)
+        assert done.any() and not done.all()
+        assert np.all(r.wave[done, 0] > 1.0) and np.all(r.wave[~done] == 0.0)
