@@ -130,8 +130,12 @@ void launch_charges(const DPlan* dp, const InstDev& w, const double* v, double* 
 // ---------------------------------------------------------------------------
 namespace {
 
+// No register limit beyond the wavefront's own: held to 128 VGPRs (four
+// wavefronts per SIMD) the compiler spilled 74 of them, among them the ones
+// it keeps spilled scalar registers in, and in a build without Verilog-A
+// models the kernel's answers were wrong (runs ended with DtLessThanMin).
 template <int NR>
-__global__ __launch_bounds__(NT, 4) void k_tran_batch(BatchArgs A) {
+__global__ __launch_bounds__(NT) void k_tran_batch(BatchArgs A) {
     extern __shared__ double lds[];
     __shared__ int s_idx;
     Lds L;
