@@ -23,7 +23,7 @@
 // descriptors, pointers and index pairs took five), the next step's record
 // requested before the current step computes, and few register spills: with
 // the plan header's 44 words in scalar registers the packed kernel spilled
-// 233 scalar and 146 vector registers (now 99 and 7), and reloaded them
+// 233 scalar and 146 vector registers (now 133 and 0), and reloaded them
 // inside the iteration.  Instructions per iteration, averaged over that
 // batch, before and after: vector 1895 -> 995, scalar 1087 -> 470, LDS 359 ->
 // 218.
@@ -100,6 +100,11 @@ __device__ __forceinline__ double step_accept(double s, int k) {
 
 // Value of lane src (uniform) for the whole wavefront.
 __device__ __forceinline__ double bcast(double v, int src) { return readlane_f64(v, src); }
+
+// A value that every lane holds, moved to scalar registers: the step control's
+// numbers live across the Newton iterations, and as vector registers they
+// would be two each in every lane.
+__device__ __forceinline__ double uniform(double v) { return readlane_f64(v, 0); }
 
 // Sum over the wavefront in a fixed order (wave_reduce): every lane ends
 // with the same value, the same on every run.
@@ -329,6 +334,24 @@ __device__ __forceinline__ double sin_degrees(double x) {
     return k & 2 ? -s : s;
 }
 
+// 1/13! .. 1/0! and the two parts of ln 2, in memory as above.
+static __device__ const double kExp[16] = {
+    1.0 / 6227020800.0, 1.0 / 479001600.0, 1.0 / 39916800.0, 1.0 / 3628800.0, 1.0 / 362880.0, 1.0 / 40320.0,
+    1.0 / 5040.0, 1.0 / 720.0, 1.0 / 120.0, 1.0 / 24.0, 1.0 / 6.0, 0.5, 1.0, 1.0,
+    0x1.62e42fefa0000p-1, 0x1.cf79abc9e3b3ap-40};
+
+// e^x: x = k ln 2 + r, the Taylor sum of e^r (next term below 1e-17), scaled.
+__device__ __forceinline__ double exp_taylor(double x) {
+    const double y = x < -1100.0 ? -1100.0 : x > 1100.0 ? 1100.0 : x;
+    const double k = rint(y / kExp[14]);
+    const double r = __builtin_fma(-k, kExp[15], __builtin_fma(-k, kExp[14], y));
+    double s = kExp[0];
+#pragma nounroll
+    for (int j = 1; j < 14; j++) s = __builtin_fma(s, r, kExp[j]);
+    s = ldexp(s, (int)k);
+    return x == x ? s : x;
+}
+
 // source_value of rules.h without calls: every operation inline, so that the
 // transient loop keeps its registers across it.
 __device__ __forceinline__ double source_at(int kind, const double* d, int len, double dc, double t, int mode) {
@@ -347,7 +370,7 @@ __device__ __forceinline__ double source_at(int kind, const double* d, int len, 
     double ang = d[5], amp = d[1];
     if (d[3] < t && t < d[6] / d[2]) {
         ang = 360.0 * d[2] * (t - d[3]) + d[5];
-        if (d[4] != 0.0) amp *= exp(-(t - d[3]) * d[4]);
+        if (d[4] != 0.0) amp *= exp_taylor(-(t - d[3]) * d[4]);
     }
     return d[0] + amp * sin_degrees(ang);
 }
@@ -851,7 +874,7 @@ __device__ __forceinline__ bool newton(Hdr c, const View& v, const DevRegs<NM>& 
                                        long long& nit) {
     const Hot h = load_hot(c);
     const int n = h.n, bx = h.b_x, bu = h.b_u;
-    const double lim = tol * tol * n;   // WRMS <= tol
+    const double lim = uniform(tol * tol * n);   // WRMS <= tol
 #pragma nounroll
     for (int it = 0; it < maxit; it++) {
         eval_mos<NM, ILP>(h, v, dr, gmin);
@@ -1069,8 +1092,8 @@ __device__ __forceinline__ void run_lds(Rec& rec, Hdr c, ConstPtr<LdsArgs> A, co
         int npts = 1;
         // step_defaults of rules.h
         const double span = A->o.t_stop - t_start;
-        double h = A->o.dt_init > 0 ? A->o.dt_init : span * 1e-9;
-        const double dt_min = A->o.dt_min > 0 ? A->o.dt_min : span * 1e-15;
+        double h = uniform(A->o.dt_init > 0 ? A->o.dt_init : span * 1e-9);
+        const double dt_min = uniform(A->o.dt_min > 0 ? A->o.dt_min : span * 1e-15);
         double* const wave = A->wave ? A->wave + A->w_off[inst] : nullptr;
         int kout = 0;
         const int n_probe = P->n_probe;
@@ -1118,7 +1141,7 @@ __device__ __forceinline__ void run_lds(Rec& rec, Hdr c, ConstPtr<LdsArgs> A, co
                         const double b = next_bp(d[0], &v.at(d[1]), d[2], t);
                         if (b < lb) lb = b;
                     }
-                    tb = wave_reduce(lb, OpMin());
+                    tb = uniform(wave_reduce(lb, OpMin()));
                     srcbp = tb < t_stop;
                     if (!srcbp) tb = t_stop;
                 }
@@ -1126,12 +1149,19 @@ __device__ __forceinline__ void run_lds(Rec& rec, Hdr c, ConstPtr<LdsArgs> A, co
             const double dt_max = A->o.dt_max > 0 ? A->o.dt_max : quot(t_stop - t_start, 10.0);
             double hh = h < dt_max ? h : dt_max;
             int hit;
-            const double tn = clip_step(t, hh, tb, hit);
+            const double tn = uniform(clip_step(t, hh, tb, hit));
+            hh = uniform(hh);
             const int k = bdf_order(npts, A->o.max_order);
             double a0, a1, a2, w0, w1, w2;
             step_bdf(k, tn, T0, T1, a0, a1, a2);
+            a0 = uniform(a0);
+            a1 = uniform(a1);
+            a2 = uniform(a2);
             const int np = npts < k + 1 ? npts : k + 1;
             step_pred(np, tn, T0, T1, T2, w0, w1, w2);
+            w0 = uniform(w0);
+            w1 = uniform(w1);
+            w2 = uniform(w2);
             const int lane = fresh_lane(tid);
 #pragma unroll
             for (int r = 0; r < NR; r++) {
@@ -1148,14 +1178,14 @@ __device__ __forceinline__ void run_lds(Rec& rec, Hdr c, ConstPtr<LdsArgs> A, co
             if (!newton<NR, NM, ILP>(c, v, dr, gmin, a0, qx, A->o.newton_maxit, A->o.newton_tol, A->o.reltol,
                                 A->o.abstol, nit)) {
                 rej++;
-                h = 0.25 * hh;
+                h = uniform(0.25 * hh);
                 if (h < dt_min) { rc = CS_E_DTMIN; break; }
                 continue;
             }
             A = fresh(A);
             double fac = 2.0;
             if (npts >= 2) {
-                const double cl = step_lte(k, tn, T0, T1, T2, a0, a1, a2);
+                const double cl = uniform(step_lte(k, tn, T0, T1, T2, a0, a1, a2));
                 double ss = 0.0;
                 const int lane = fresh_lane(tid);
 #pragma unroll
@@ -1169,11 +1199,11 @@ __device__ __forceinline__ void run_lds(Rec& rec, Hdr c, ConstPtr<LdsArgs> A, co
                 const double err2 = quot(wave_sum(ss), (double)n);
                 if (!(err2 <= 1.0)) {
                     rej++;
-                    h = hh * step_reject(err2, k);
+                    h = uniform(hh * step_reject(err2, k));
                     if (h < dt_min) { rc = CS_E_DTMIN; break; }
                     continue;
                 }
-                fac = step_accept(err2, k);
+                fac = uniform(step_accept(err2, k));
             }
             // accept
 #pragma unroll
@@ -1209,6 +1239,7 @@ __device__ __forceinline__ void run_lds(Rec& rec, Hdr c, ConstPtr<LdsArgs> A, co
                 h = 0.1 * h;
                 if (h < dt_min) h = dt_min;
             }
+            h = uniform(h);
         }
     }
     A = fresh(A);
