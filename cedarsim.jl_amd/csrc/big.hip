@@ -589,7 +589,8 @@ __global__ __launch_bounds__(kBT) void k_mf_trsm(const BigDev* P, double* pool, 
 
 // F[i0:i0+64, j0:j0+64] -= L U for the L panel rows A[c][i] (transposed) and
 // the U panel columns Bt[c][j] staged in LDS, on the vector ALUs
-__device__ __forceinline__ void tile_update_valu(const double (*A)[kTile + 1], const double (*Bt)[kTile + 1],
+template <int LD>
+__device__ __forceinline__ void tile_update_valu(const double (*A)[LD], const double (*Bt)[LD],
                                                  double* G, int m, int i0, int j0, int nb) {
     const int ti = (threadIdx.x % 16) * 4, tj = (threadIdx.x / 16) * 4;
     double acc[4][4] = {};
@@ -632,21 +633,6 @@ __device__ __forceinline__ void load_panel_tiles(double (*A)[kTile + 1], double 
         A[q / kTile][q % kTile] = va[r];
         Bt[q % kNb][q / kNb] = vb[r];
     }
-}
-
-// The nb x nb diagonal block at (p0, p0) of G (leading dimension m) into D
-// (leading dimension kNb), all loads before the first store
-__device__ __forceinline__ void load_diag_block(double* D, const double* G, int m, int p0, int nb) {
-    constexpr int R = kNb * kNb / kBT;
-    static_assert(R * kBT == kNb * kNb, "diagonal block splits evenly over the threads");
-    double v[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int q = (int)threadIdx.x + r * kBT, j = q / kNb, i = q % kNb;
-        v[r] = (i < nb && j < nb) ? G[(int64_t)(p0 + j) * m + p0 + i] : 0.0;
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++) D[(int)threadIdx.x + r * kBT] = v[r];
 }
 
 // tile = (front, p0, i0, j0): F[i0:i0+64, j0:j0+64] -= L[.., p0:p0+nb] U[p0:p0+nb, ..]
@@ -713,7 +699,8 @@ __device__ __forceinline__ void tile_load_mfma(const double* G, int m, int i0, i
 }
 
 // tile_update_mfma with the tile's entries already in cv
-__device__ __forceinline__ void tile_update_mfma_c(const double (*A)[kTile + 1], const double (*Bt)[kTile + 1],
+template <int LD>
+__device__ __forceinline__ void tile_update_mfma_c(const double (*A)[LD], const double (*Bt)[LD],
                                                    double* G, int m, int i0, int j0, int nb, const double (&cv)[16]) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wi = (wave & 1) * 32, wj = (wave >> 1) * 32;
@@ -753,13 +740,73 @@ __global__ __launch_bounds__(kBT) void k_mf_gemm_mfma(const BigDev* P, double* p
     tile_update_mfma(A, Bt, G, m, i0, j0, nb);
 }
 
+// Lane src's value (src uniform) for the whole wavefront, by readlane.
+__device__ __forceinline__ double wave_bcast(double v, int src) {
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(b & 0xffffffffll), src);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), src);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Pivots [p, min(p + kStage, nb)) of a panel step, one panel row (Col:
+// column) per lane in registers; lanes 0..31 carry the diagonal block's, the
+// pivot's own lane p supplies the step's other operand by readlane.  The
+// registers rotate by one per pivot, so a[0] is always the entry of the
+// pivot's column (Col: row) and every register index is fixed:
+//   row i:     l = a[0] * (1 / u(p,p)) is L(i,p);    a[j] = a[j+1] - l u(p,j)
+//   column j:  a[0] is U(p,j);  a[i] = a[i+1] - l(i,p) a[0], the same l
+// Each finished entry goes to out (one entry of the panel per pivot, kPanLd
+// apart).  Lanes at or before the pivot go on computing; nothing reads what
+// they hold.  W registers are still needed when the stage begins.
+constexpr int kStage = 8;
+constexpr int kPanLd = kNb + kTile + 1;
+template <bool Col, int W>
+__device__ __forceinline__ void panel_stage(double (&a)[kNb], int& p, int nb, double& ip, double* out) {
+#pragma unroll 1
+    for (int q = 0; q < kStage && p < nb; q++, p++) {
+        const double l = Col ? a[0] : a[0] * ip;
+        out[p * kPanLd] = l;
+        // the next pivot first: its reciprocal runs beside the other updates
+        const double ipc = ip;
+        {
+            const double o = wave_bcast(a[1], p);
+            a[0] = Col ? a[1] - (o * ipc) * l : a[1] - l * o;
+        }
+        ip = 1.0 / wave_bcast(a[0], p + 1);
+#pragma unroll
+        for (int i = 1; i < W - 1; i++) {
+            const double o = wave_bcast(a[i + 1], p);
+            a[i] = Col ? a[i + 1] - (o * ipc) * l : a[i + 1] - l * o;
+        }
+    }
+}
+template <bool Col>
+__device__ __forceinline__ void panel_lu(double (&a)[kNb], int nb, double* out) {
+    int p = 0;
+    double ip = 1.0 / wave_bcast(a[0], 0);
+    panel_stage<Col, 32>(a, p, nb, ip, out);
+    panel_stage<Col, 24>(a, p, nb, ip, out);
+    panel_stage<Col, 16>(a, p, nb, ip, out);
+    panel_stage<Col, 8>(a, p, nb, ip, out);
+}
+static_assert(kNb == 4 * kStage && kTile == 64 && kBT == 256, "panel_lu's stages and wavefronts");
+
 // One step of the blocked front LU in one launch.  item = (front, p0, i0,
-// j0): every workgroup factors the diagonal block [p0, p1) itself, solves
-// the L rows [i0, i0+64) and the U columns [j0, j0+64) it needs, and
-// updates the trailing tile F[i0:, j0:]; (front, p0, -1, -1) is a step with
-// no trailing matrix (p1 = m).  The operations and their order are those of
-// k_mf_diag, k_mf_trsm and the trailing update, so the factors are the same
-// bits.  Workgroups of the step read the unfactored panel from the front,
+// j0): every workgroup factors the diagonal block [p0, p1), solves the L
+// rows [i0, i0+64) and the U columns [j0, j0+64) it needs, and updates the
+// trailing tile F[i0:, j0:]; (front, p0, -1, -1) is a step with no trailing
+// matrix (p1 = m).  The operations and their order are those of k_mf_diag,
+// k_mf_trsm and the trailing update, so the factors are the same bits.
+//
+// The step is one serial chain over its pivots.  The factorization of the
+// diagonal block, then staged coefficients, then the triangular solves were
+// three such phases, with an LDS round trip and a barrier per pivot in the
+// first.  Now four wavefronts each carry the diagonal block's 32 rows (or
+// columns) beside 32 rows of L (columns of U) and go through the pivots
+// once, in registers, with no barrier and no LDS read: a step
+// of a 450 x 450 grid's factorization took 36 us, now 25.
+//
+// Workgroups of the step read the unfactored panel from the front,
 // so the factored panel goes to the workspace W instead (the same layout,
 // at woff[front]): the diagonal block from the tile (p1, p1) or the item
 // without trailing matrix, L rows from the tiles with j0 = p1, U columns
@@ -768,69 +815,86 @@ __global__ __launch_bounds__(kBT) void k_mf_gemm_mfma(const BigDev* P, double* p
 template <bool Mfma>
 __global__ __launch_bounds__(kBT) void k_mf_panel(const BigDev* P, double* pool, double* dinv, double* W,
                                                   const int64_t* woff, const int4* items) {
-    __shared__ double D[kNb * kNb];
-    __shared__ double cb[2][kNb], rb[2][kNb];
-    __shared__ double ipv[kNb];
-    __shared__ double EU[kCoef], EL[kCoef];
-    __shared__ double A[kNb][kTile + 1];
-    __shared__ double Bt[kNb][kTile + 1];
+    // A[c][i]: rows of the panel's column c, the diagonal block's 32 first,
+    // then the L rows; Bt[c][j]: columns of its row c, likewise
+    __shared__ double A[kNb][kPanLd];
+    __shared__ double Bt[kNb][kPanLd];
     const int4 it = items[blockIdx.x];
     const int s = it.x, p0 = it.y, i0 = it.z, j0 = it.w;
     const int m = P->sn_m[s], k = sn_k(P, s), f0 = P->sn_first[s];
     const int nb = (k - p0) < kNb ? (k - p0) : kNb, p1 = p0 + nb;
     double* G = pool + P->sn_off[s];
     double* Wf = W + woff[s];
-    load_diag_block(D, G, m, p0, nb);
-    double cv[16];   // the trailing tile, read ahead of the LU (MFMA form)
-    if (i0 >= 0) {
-        load_panel_tiles(A, Bt, G, m, p0, i0, j0, nb);
-        if (Mfma) tile_load_mfma(G, m, i0, j0, cv);
+    const bool tile = i0 >= 0;
+    {
+        // all loads before the first LDS store, addresses running down the
+        // front's columns; zero past the block, the panel and the front
+        constexpr int RD = kNb * kNb / kBT, RT = kNb * kTile / kBT;
+        double vd[RD], va[RT], vb[RT];
+#pragma unroll
+        for (int r = 0; r < RD; r++) {
+            const int q = (int)threadIdx.x + r * kBT, j = q / kNb, i = q % kNb;
+            vd[r] = (i < nb && j < nb) ? G[(int64_t)(p0 + j) * m + p0 + i] : 0.0;
+        }
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            const int q = (int)threadIdx.x + r * kBT;
+            const int c = q / kTile, i = q % kTile;       // A: column c, row i
+            const int cu = q % kNb, ju = q / kNb;         // Bt: row cu, column ju
+            va[r] = (tile && c < nb && i0 + i < m) ? G[(int64_t)(p0 + c) * m + i0 + i] : 0.0;
+            vb[r] = (tile && cu < nb && j0 + ju < m) ? G[(int64_t)(j0 + ju) * m + p0 + cu] : 0.0;
+        }
+#pragma unroll
+        for (int r = 0; r < RD; r++) {
+            const int q = (int)threadIdx.x + r * kBT, j = q / kNb, i = q % kNb;
+            A[j][i] = vd[r];
+            Bt[i][j] = vd[r];
+        }
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            const int q = (int)threadIdx.x + r * kBT;
+            A[q / kTile][kNb + q % kTile] = va[r];
+            Bt[q % kNb][kNb + q / kNb] = vb[r];
+        }
     }
+    double cv[16];   // the trailing tile, read ahead of the LU (MFMA form)
+    if (Mfma && tile) tile_load_mfma(G, m, i0, j0, cv);
     __syncthreads();
-    diag_lu_block<kBT>(D, ipv, nb, cb, rb);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // wavefronts 0 and 1: rows, 2 and 3: columns
+    double* mine = &(wave < 2 ? A : Bt)[0][lane < kNb ? lane : lane + (wave & 1) * kNb];
+    double a[kNb];
+#pragma unroll
+    for (int c = 0; c < kNb; c++) a[c] = mine[c * kPanLd];
+    __syncthreads();   // the diagonal block is read by two wavefronts, then overwritten (same values) by both
+    const int nbu = __builtin_amdgcn_readfirstlane(nb);
+    if (wave < 2) panel_lu<false>(a, nbu, mine);
+    else panel_lu<true>(a, nbu, mine);
     __syncthreads();
-    const bool diag_owner = i0 < 0 || (i0 == p1 && j0 == p1);
+    // the diagonal block: L below the diagonal in A, U in Bt
+    const bool diag_owner = !tile || (i0 == p1 && j0 == p1);
     if (diag_owner) {
         for (int q = threadIdx.x; q < nb * nb; q += kBT) {
             const int j = q / nb, i = q % nb;
-            Wf[(int64_t)(p0 + j) * m + p0 + i] = D[j * kNb + i];
+            Wf[(int64_t)(p0 + j) * m + p0 + i] = i > j ? A[j][i] : Bt[i][j];
         }
-        if ((int)threadIdx.x < nb) dinv[f0 + p0 + threadIdx.x] = ipv[threadIdx.x];
+        if ((int)threadIdx.x < nb) dinv[f0 + p0 + threadIdx.x] = 1.0 / Bt[threadIdx.x][threadIdx.x];
     }
-    if (i0 < 0) return;
-    load_coef<true>(EU, D, kNb, nb);
-    load_coef<false>(EL, D, kNb, nb);
-    __syncthreads();
-    const int t = threadIdx.x;
-    if (t < kTile) {
-        if (i0 + t < m) {
-            double a[kNb];
-#pragma unroll
-            for (int c = 0; c < kNb; c++) a[c] = c < nb ? A[c][t] : 0.0;
-            rot_solve<true>(a, EU, ipv, nb, [&](int c, double x) { A[c][t] = x; });
-        }
-    } else if (t < 2 * kTile) {
-        const int jj = t - kTile;
-        if (j0 + jj < m) {
-            double a[kNb];
-#pragma unroll
-            for (int c = 0; c < kNb; c++) a[c] = c < nb ? Bt[c][jj] : 0.0;
-            rot_solve<false>(a, EL, nullptr, nb, [&](int c, double x) { Bt[c][jj] = x; });
-        }
-    }
-    __syncthreads();
+    if (!tile) return;
     if (j0 == p1)
         for (int q = threadIdx.x; q < nb * kTile; q += kBT) {
             const int c = q / kTile, i = q % kTile;
-            if (i0 + i < m) Wf[(int64_t)(p0 + c) * m + i0 + i] = A[c][i];
+            if (i0 + i < m) Wf[(int64_t)(p0 + c) * m + i0 + i] = A[c][kNb + i];
         }
     if (i0 == p1)
         for (int q = threadIdx.x; q < nb * kTile; q += kBT) {
             const int jj = q / nb, c = q % nb;
-            if (j0 + jj < m) Wf[(int64_t)(j0 + jj) * m + p0 + c] = Bt[c][jj];
+            if (j0 + jj < m) Wf[(int64_t)(j0 + jj) * m + p0 + c] = Bt[c][kNb + jj];
         }
-    if (Mfma) tile_update_mfma_c(A, Bt, G, m, i0, j0, nb, cv);
-    else tile_update_valu(A, Bt, G, m, i0, j0, nb);
+    const double (*At)[kPanLd] = (const double (*)[kPanLd])&A[0][kNb];
+    const double (*Ut)[kPanLd] = (const double (*)[kPanLd])&Bt[0][kNb];
+    if (Mfma) tile_update_mfma_c(At, Ut, G, m, i0, j0, nb, cv);
+    else tile_update_valu(At, Ut, G, m, i0, j0, nb);
 }
 
 // item = (front, j0): copies the factored panels of columns [j0, j0+4) back
@@ -1052,14 +1116,6 @@ __global__ __launch_bounds__(kBT) void k_mf_lvl_big(const BigDev* P, double* poo
 }
 
 // ---- multifrontal solves ----------------------------------------------------------------
-// Lane src's value (src uniform) for the whole wavefront, by readlane.
-__device__ __forceinline__ double wave_bcast(double v, int src) {
-    const long long b = __double_as_longlong(v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(b & 0xffffffffll), src);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), src);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
 // forward: y = L^-1 b by levels; update vectors of the fronts in uvec
 // The solves' diagonal block: S[pp * 65 + ii] = G[(b0 + pp) m + b0 + ii]
 // for pp < nbk (zero for ii >= nbk); a thread's loads of each group of up to
