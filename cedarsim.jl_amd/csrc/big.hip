@@ -43,7 +43,10 @@ constexpr int kBT = 256;      // threads of the device-wide kernels
 constexpr int kSmallM = 96;   // fronts up to this size factor in LDS
 constexpr int kNb = 32;       // panel width of the blocked front LU
 constexpr int kTile = 64;     // trailing-update tile
-constexpr int kGatherChunk = 8192;
+constexpr int kGatherChunk = 8192;   // entries a gather tile can hold in LDS
+// entries a gather tile should have: a tile is a chain of dependent loads
+// per child and per 4 entries of a thread, so smaller tiles end earlier
+constexpr int kGatherTile = 2048;
 constexpr int kRowBlocks = 1024;
 
 struct BigDev {
@@ -338,6 +341,20 @@ __device__ __forceinline__ void gsync() {
     __syncthreads();
 }
 
+// Barrier of the NT threads that work on one front in LDS: the workgroup,
+// or a wavefront of a workgroup whose wavefronts work on fronts of their own
+// (a wavefront's LDS operations complete in order: only the compiler must
+// keep them so).
+template <int NT>
+__device__ __forceinline__ void front_sync() {
+    if (NT > 64) {
+        __syncthreads();
+        return;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Columns [j0, j1) of front s = the sum of its children's contribution
 // blocks, children in order, into F (column j0 at F[0], leading dimension
 // m): the columns are zeroed, then each child's block is added (one
@@ -346,13 +363,14 @@ __device__ __forceinline__ void gsync() {
 // when given, holds per child the range of its block columns that land in
 // [j0, j1) (rel is ascending); without it every column does.  Every entry
 // sees its children's values in the same order as a sum over the children.
-// NT threads; Global: F in global memory (fenced barriers), else in LDS.
+// NT threads, this one number tid; Global: F in global memory (fenced
+// barriers), else in LDS.
 template <int NT, bool Global>
 __device__ __forceinline__ void scatter_cb(const BigDev* P, const double* pool, double* F, int m, int s, int j0,
-                                           int j1, const int2* br) {
-    for (int q = threadIdx.x; q < (j1 - j0) * m; q += NT) F[q] = 0.0;
+                                           int j1, const int2* br, int tid) {
+    for (int q = tid; q < (j1 - j0) * m; q += NT) F[q] = 0.0;
     if (Global) gsync();
-    else __syncthreads();
+    else front_sync<NT>();
     const int c0 = P->ch_ptr[s], c1 = P->ch_ptr[s + 1];
     for (int cq = c0; cq < c1; cq++) {
         const int c = P->ch_sn[cq];
@@ -370,7 +388,7 @@ __device__ __forceinline__ void scatter_cb(const BigDev* P, const double* pool, 
         // distinct entries of F, so the order within a child is free.
         constexpr int U = 4;
         const int tot = (b1 - b0) * rc;
-        for (int q0 = threadIdx.x; q0 < tot; q0 += NT * U) {
+        for (int q0 = tid; q0 < tot; q0 += NT * U) {
             int dst[U];
             double sv[U];
 #pragma unroll
@@ -387,25 +405,36 @@ __device__ __forceinline__ void scatter_cb(const BigDev* P, const double* pool, 
                 if (q0 + u * NT < tot) F[dst[u]] += sv[u];
         }
         if (Global) gsync();
-        else __syncthreads();
+        else front_sync<NT>();
     }
 }
 
 // tile = (front, first column, end column, offset of its per-child column
 // ranges in cbr): the tile (at most kGatherChunk entries) is summed in LDS
-// and written once
+// and written once.  With op, the Jacobian entries of the tile's columns
+// (positions op[0, n_op)) are added before that; they land on distinct
+// entries, so their order is free.
+__device__ __forceinline__ void gather_tile(const BigDev* P, double* pool, const int4 t, const int2* cbr, double* Ft,
+                                            const double* Aval, const int32_t* op, int n_op) {
+    const int s = t.x, m = P->sn_m[s];
+    const int64_t off = P->sn_off[s] + (int64_t)t.y * m;
+    double* G = pool + off;
+    const bool fits = (t.z - t.y) * m <= kGatherChunk;
+    if (fits) {
+        scatter_cb<kBT, false>(P, pool, Ft, m, s, t.y, t.z, cbr + t.w, threadIdx.x);
+        for (int q = threadIdx.x; q < n_op; q += kBT) Ft[P->nat_dest[op[q]] - off] += Aval[op[q]];
+        if (n_op) __syncthreads();
+        for (int q = threadIdx.x; q < (t.z - t.y) * m; q += kBT) G[q] = Ft[q];
+    } else {   // a single column longer than the LDS tile
+        scatter_cb<kBT, true>(P, pool, G, m, s, t.y, t.z, cbr + t.w, threadIdx.x);
+        for (int q = threadIdx.x; q < n_op; q += kBT) G[P->nat_dest[op[q]] - off] += Aval[op[q]];
+    }
+}
+
 __global__ __launch_bounds__(kBT) void k_mf_gather(const BigDev* P, double* pool, const int4* tiles,
                                                    const int2* cbr) {
-    __shared__ double Ft[kGatherChunk];
-    const int4 t = tiles[blockIdx.x];
-    const int s = t.x, m = P->sn_m[s];
-    double* G = pool + P->sn_off[s] + (int64_t)t.y * m;
-    if ((t.z - t.y) * m > kGatherChunk) {   // a single column longer than the LDS tile
-        scatter_cb<kBT, true>(P, pool, G, m, s, t.y, t.z, cbr + t.w);
-        return;
-    }
-    scatter_cb<kBT, false>(P, pool, Ft, m, s, t.y, t.z, cbr + t.w);
-    for (int q = threadIdx.x; q < (t.z - t.y) * m; q += kBT) G[q] = Ft[q];
+    extern __shared__ double lds_f[];
+    gather_tile(P, pool, tiles[blockIdx.x], cbr, lds_f, nullptr, nullptr, 0);
 }
 
 __global__ __launch_bounds__(kBT) void k_mf_orig(const BigDev* P, const double* Aval, double* pool,
@@ -901,9 +930,8 @@ __global__ __launch_bounds__(kBT) void k_mf_panel(const BigDev* P, double* pool,
 // from the workspace, i.e. the entries (i, j) with min(i, j) < k: the whole
 // column for j < k, its rows [0, k) for j >= k
 constexpr int kFlushCols = 4;
-__global__ __launch_bounds__(kBT) void k_mf_flush(const BigDev* P, double* pool, const double* W,
-                                                  const int64_t* woff, const int2* items) {
-    const int2 it = items[blockIdx.x];
+__device__ __forceinline__ void flush_cols(const BigDev* P, double* pool, const double* W, const int64_t* woff,
+                                           const int2 it) {
     const int s = it.x, m = P->sn_m[s], k = sn_k(P, s);
     double* G = pool + P->sn_off[s];
     const double* Wf = W + woff[s];
@@ -913,6 +941,11 @@ __global__ __launch_bounds__(kBT) void k_mf_flush(const BigDev* P, double* pool,
         const int64_t o = (int64_t)j * m;
         for (int i = threadIdx.x; i < rows; i += kBT) G[o + i] = Wf[o + i];
     }
+}
+__global__ __launch_bounds__(kBT) void k_mf_flush(const BigDev* P, double* pool, const double* W,
+                                                  const int64_t* woff, const int2* items) {
+    const int2 it = items[blockIdx.x];
+    flush_cols(P, pool, W, woff, it);
 }
 
 // ---- fused per-level front kernels (one workgroup per front) ------------------------------
@@ -926,22 +959,23 @@ __global__ __launch_bounds__(kBT) void k_mf_flush(const BigDev* P, double* pool,
 // pivots ascending).  Fronts are bucketed by size so that the small ones
 // run as single wavefronts with few registers.
 template <int TL, int R>
-__global__ __launch_bounds__(TL * TL) void k_mf_lvl_small(const BigDev* P, double* pool, double* dinv,
-                                                          const double* Aval, const int32_t* fronts) {
+constexpr int small_doubles(int m_max) { return m_max * m_max + 4 * TL * R; }
+template <int TL, int R>
+__device__ __forceinline__ void small_front(const BigDev* P, double* pool, double* dinv, const double* Aval,
+                                            int s, double* lds, int tid) {
     constexpr int NT = TL * TL, MX = TL * R;
-    extern __shared__ double lds_f[];
-    __shared__ double cb[2][MX], rb[2][MX];
-    double* F = lds_f;
-    const int s = fronts[blockIdx.x];
+    double (*cb)[MX] = (double (*)[MX])lds;
+    double (*rb)[MX] = cb + 2;
+    double* F = lds + 4 * MX;
     const int m = P->sn_m[s], k = sn_k(P, s), f0 = P->sn_first[s];
     const int64_t off = P->sn_off[s];
-    scatter_cb<NT, false>(P, pool, F, m, s, 0, m, nullptr);
+    scatter_cb<NT, false>(P, pool, F, m, s, 0, m, nullptr, tid);
     // the front's Jacobian entries (distinct positions: order free), four
     // per thread with their loads ahead of the adds
     {
         constexpr int U = 4;
         const int q1 = P->osn_ptr[s + 1];
-        for (int q0 = P->osn_ptr[s] + threadIdx.x; q0 < q1; q0 += NT * U) {
+        for (int q0 = P->osn_ptr[s] + tid; q0 < q1; q0 += NT * U) {
             int e[U];
 #pragma unroll
             for (int u = 0; u < U; u++) e[u] = q0 + u * NT < q1 ? P->osn_pos[q0 + u * NT] : 0;
@@ -958,8 +992,8 @@ __global__ __launch_bounds__(TL * TL) void k_mf_lvl_small(const BigDev* P, doubl
                 if (q0 + u * NT < q1) F[d[u]] += v[u];
         }
     }
-    __syncthreads();
-    const int ti = threadIdx.x % TL, tj = threadIdx.x / TL;
+    front_sync<NT>();
+    const int ti = tid % TL, tj = tid / TL;
     double a[R][R];
 #pragma unroll
     for (int y = 0; y < R; y++)
@@ -970,11 +1004,11 @@ __global__ __launch_bounds__(TL * TL) void k_mf_lvl_small(const BigDev* P, doubl
             if (j == 0) cb[0][i] = a[y][x];
             if (i == 0) rb[0][j] = a[y][x];
         }
-    __syncthreads();
+    front_sync<NT>();
     for (int p = 0; p < k; p++) {
         const int b = p & 1;
         const double ip = 1.0 / rb[b][p];
-        if (threadIdx.x == 0) dinv[f0 + p] = ip;
+        if (tid == 0) dinv[f0 + p] = ip;
         double l[R], u[R];
         // the pivot row and column are read unconditionally (in bounds: the
         // buffers hold MX entries) and the update is selected, not branched
@@ -1004,7 +1038,7 @@ __global__ __launch_bounds__(TL * TL) void k_mf_lvl_small(const BigDev* P, doubl
                 if (i == p + 1) rb[b ^ 1][j] = a[y][x];
             }
         }
-        __syncthreads();
+        front_sync<NT>();
     }
     double* G = pool + off;
 #pragma unroll
@@ -1015,10 +1049,50 @@ __global__ __launch_bounds__(TL * TL) void k_mf_lvl_small(const BigDev* P, doubl
             if (i < m && j < m) G[(int64_t)j * m + i] = a[y][x];
         }
 }
+template <int TL, int R>
+__global__ __launch_bounds__(TL * TL) void k_mf_lvl_small(const BigDev* P, double* pool, double* dinv,
+                                                          const double* Aval, const int32_t* fronts) {
+    extern __shared__ double lds_f[];
+    small_front<TL, R>(P, pool, dinv, Aval, fronts[blockIdx.x], lds_f, threadIdx.x);
+}
 // size buckets: (threads per side, entries per side per thread)
 constexpr int kSmallBuckets = 3;
 constexpr int kBucketMax[kSmallBuckets] = {32, 64, kSmallM};
 static_assert(8 * 4 >= 32 && 16 * 4 >= 64 && 16 * 6 >= kSmallM, "small-front buckets exceed their kernels");
+
+// The independent work at the head of a level in one launch: its small
+// fronts of every bucket, the gather tiles of its large ones (with their
+// Jacobian entries), and the copies of the previous level's factored panels
+// from the workspace (this level reads only that level's contribution
+// blocks).  As launches of their own these ran one after the other, each
+// with too few workgroups to fill the chip: a 150 x 150 grid's factorization
+// went from 1.34 to 1.00 ms (98 launches to 56).
+// item = (kind, a, b, c):
+//   kHeadSmall32: fronts[a, a + b), one wavefront each, b <= 4
+//   kHeadSmall64 / kHeadSmall96: front fronts[a]
+//   kHeadGather: tile a, Jacobian positions borig[b, c)
+//   kHeadFlush: flush item a
+enum { kHeadSmall32, kHeadSmall64, kHeadSmall96, kHeadGather, kHeadFlush };
+__global__ __launch_bounds__(kBT) void k_mf_head(const BigDev* P, double* pool, double* dinv, const double* Aval,
+                                                 const int4* items, const int32_t* fronts, const int4* tiles,
+                                                 const int2* cbr, const int32_t* borig, const double* W,
+                                                 const int64_t* woff, const int2* flush, int lds32) {
+    extern __shared__ double lds_f[];
+    const int4 it = items[blockIdx.x];
+    if (it.x == kHeadSmall32) {
+        const int wave = threadIdx.x >> 6;
+        if (wave < it.z)
+            small_front<8, 4>(P, pool, dinv, Aval, fronts[it.y + wave], lds_f + wave * lds32, threadIdx.x & 63);
+    } else if (it.x == kHeadSmall64) {
+        small_front<16, 4>(P, pool, dinv, Aval, fronts[it.y], lds_f, threadIdx.x);
+    } else if (it.x == kHeadSmall96) {
+        small_front<16, 6>(P, pool, dinv, Aval, fronts[it.y], lds_f, threadIdx.x);
+    } else if (it.x == kHeadGather) {
+        gather_tile(P, pool, tiles[it.y], cbr, lds_f, Aval, borig + it.z, it.w - it.z);
+    } else {
+        flush_cols(P, pool, W, woff, flush[it.y]);
+    }
+}
 
 // Large fronts, one workgroup each: gather, then blocked right-looking
 // partial LU in global memory (L2-resident): diagonal block in LDS, row and
@@ -1036,7 +1110,7 @@ __global__ __launch_bounds__(kBT) void k_mf_lvl_big(const BigDev* P, double* poo
     const int m = P->sn_m[s], k = sn_k(P, s), f0 = P->sn_first[s];
     const int64_t off = P->sn_off[s];
     double* G = pool + off;
-    scatter_cb<kBT, true>(P, pool, G, m, s, 0, m, nullptr);
+    scatter_cb<kBT, true>(P, pool, G, m, s, 0, m, nullptr, threadIdx.x);
     for (int q = P->osn_ptr[s] + threadIdx.x; q < P->osn_ptr[s + 1]; q += kBT) {
         const int e = P->osn_pos[q];
         G[P->nat_dest[e] - off] += Aval[e];
@@ -1426,6 +1500,10 @@ struct BigCircuit {
         int ld_off;   // offset of the solves' diagonal block in their LDS
         int solve_bt;   // the solves' workgroup size (64, 256 or 512)
         int flush_b, flush_n;
+        int tile_lds;                 // bytes of the largest gather tile in LDS
+        int head_b, head_n, head_nf, head_lds;   // one-launch head (k_mf_head) without and with the
+                                                 // previous level's flush; head_n 0: separate launches
+        int head_lds32;               // its LDS per small32 front, in doubles
         std::vector<Panel> panels;
     };
     std::vector<Level> levels;
@@ -1437,6 +1515,7 @@ struct BigCircuit {
     int4* d_gemm = nullptr;
     int4* d_pan = nullptr;
     int2* d_flush = nullptr;
+    int4* d_head = nullptr;
     int64_t* d_woff = nullptr;   // per front: offset of its factored panels in wpan
     double* wpan = nullptr;
     int32_t* d_borig = nullptr;   // Jacobian positions of the large fronts, by level
@@ -1485,6 +1564,13 @@ void prof_mark(BigCircuit& C, hipStream_t s, int kind, int level) {
     } while (0)
 
 namespace {
+
+// Levels of up to this many head items go as one launch.  k_mf_head holds the
+// registers and LDS of its largest kind for every item, so where the small
+// fronts alone fill the chip many times over the separate kernels are faster:
+// the leaf levels of a 450 x 450 grid took 79 + 23, 50 + 41 and 34 + 38 us
+// apart and 157, 91 and 64 us as one; of a 150 x 150 grid 34 + 13 and 36 us.
+constexpr int kHeadItems = 4096;
 
 template <class T>
 size_t pack_add(std::vector<char>& bytes, const std::vector<T>& v) {
@@ -1574,7 +1660,7 @@ int upload(BigCircuit& C, std::string& err) {
     BCHK(hipMemcpy(C.d_dev, &C.hd, sizeof(BigDev), hipMemcpyHostToDevice));
 
     // launch tables
-    std::vector<int4> tiles, trsm, gemm, pan;
+    std::vector<int4> tiles, trsm, gemm, pan, head;
     std::vector<int32_t> fronts, borig;
     std::vector<int2> diag, cbr, flush;
     std::vector<int64_t> woff(std::max(B.ns, 1), 0);
@@ -1594,6 +1680,8 @@ int upload(BigCircuit& C, std::string& err) {
         Lv.tile_b = (int)tiles.size();
         int small_max[kSmallBuckets] = {}, m_max = 0;
         std::vector<int32_t> small[kSmallBuckets], large;
+        std::vector<int4> h_gather;
+        Lv.tile_lds = 0;
         Lv.orig_b = (int)borig.size();
         for (int q = B.lev_ptr[l]; q < B.lev_ptr[l + 1]; q++) {
             const int s = B.lev_sn[q], m = B.sn_m[s];
@@ -1604,9 +1692,21 @@ int upload(BigCircuit& C, std::string& err) {
                 small_max[bk] = std::max(small_max[bk], m);
             } else {
                 large.push_back(s);
-                const int step = std::max(1, kGatherChunk / std::max(m, 1));
+                // the front's Jacobian positions by column, so that those of a
+                // tile are one range
+                const size_t ob = borig.size();
+                borig.insert(borig.end(), B.osn_pos.begin() + B.osn_ptr[s], B.osn_pos.begin() + B.osn_ptr[s + 1]);
+                auto col_of = [&](int32_t pos) { return (int)((B.nat_dest[pos] - B.sn_off[s]) / m); };
+                std::stable_sort(borig.begin() + ob, borig.end(),
+                                 [&](int32_t a, int32_t b) { return col_of(a) < col_of(b); });
+                size_t op = ob;
+                const int step = std::max(1, kGatherTile / std::max(m, 1));
                 for (int j = 0; j < m; j += step) {
                     const int j1 = std::min(m, j + step);
+                    const size_t o0 = op;
+                    while (op < borig.size() && col_of(borig[op]) < j1) op++;
+                    h_gather.push_back(make_int4(kHeadGather, (int)tiles.size(), (int)o0, (int)op));
+                    Lv.tile_lds = std::max<int>(Lv.tile_lds, sizeof(double) * std::min((j1 - j) * m, kGatherChunk));
                     tiles.push_back(make_int4(s, j, j1, (int)cbr.size()));
                     for (int cq = B.ch_ptr[s]; cq < B.ch_ptr[s + 1]; cq++) {
                         const int c = B.ch_sn[cq];
@@ -1616,7 +1716,6 @@ int upload(BigCircuit& C, std::string& err) {
                                                 (int)(std::lower_bound(rl, rl + rc, j1) - rl)));
                     }
                 }
-                borig.insert(borig.end(), B.osn_pos.begin() + B.osn_ptr[s], B.osn_pos.begin() + B.osn_ptr[s + 1]);
             }
             m_max = std::max(m_max, m);
         }
@@ -1626,8 +1725,33 @@ int upload(BigCircuit& C, std::string& err) {
             Lv.small_b[bk] = (int)fronts.size();
             fronts.insert(fronts.end(), small[bk].begin(), small[bk].end());
             Lv.small_n[bk] = (int)small[bk].size();
-            Lv.small_lds[bk] = sizeof(double) * (size_t)small_max[bk] * small_max[bk];
+            const int sm = small_max[bk];
+            Lv.small_lds[bk] = sizeof(double) * (bk == 0   ? small_doubles<8, 4>(sm)
+                                                 : bk == 1 ? small_doubles<16, 4>(sm)
+                                                           : small_doubles<16, 6>(sm));
         }
+        // the head's items: what takes longest first, the previous level's
+        // panel copies last (left out when that level wrote no workspace)
+        Lv.head_b = (int)head.size();
+        Lv.head_lds32 = (int)(Lv.small_lds[0] / sizeof(double));
+        Lv.head_lds = 0;
+        for (int bk = 2; bk >= 1; bk--) {
+            for (int q = 0; q < Lv.small_n[bk]; q++)
+                head.push_back(make_int4(bk == 2 ? kHeadSmall96 : kHeadSmall64, Lv.small_b[bk] + q, 0, 0));
+            if (Lv.small_n[bk]) Lv.head_lds = std::max(Lv.head_lds, (int)Lv.small_lds[bk]);
+        }
+        head.insert(head.end(), h_gather.begin(), h_gather.end());
+        Lv.head_lds = std::max(Lv.head_lds, Lv.tile_lds);
+        for (int q = 0; q < Lv.small_n[0]; q += 4)
+            head.push_back(make_int4(kHeadSmall32, Lv.small_b[0] + q, std::min(4, Lv.small_n[0] - q), 0));
+        if (Lv.small_n[0])
+            Lv.head_lds = std::max(Lv.head_lds, std::min(4, Lv.small_n[0]) * (int)Lv.small_lds[0]);
+        Lv.head_n = (int)head.size() - Lv.head_b;
+        if (l > 0)
+            for (int q = 0; q < C.levels[l - 1].flush_n; q++)
+                head.push_back(make_int4(kHeadFlush, C.levels[l - 1].flush_b + q, 0, 0));
+        Lv.head_nf = (int)head.size() - Lv.head_b;
+        if (Lv.head_n > kHeadItems) Lv.head_n = 0;
         Lv.fr_b = (int)fronts.size();
         for (int q = B.lev_ptr[l]; q < B.lev_ptr[l + 1]; q++) fronts.push_back(B.lev_sn[q]);
         Lv.fr_n = (int)fronts.size() - Lv.fr_b;
@@ -1689,7 +1813,7 @@ int upload(BigCircuit& C, std::string& err) {
     std::vector<char> tb;
     size_t o_t = pack_add(tb, tiles), o_f = pack_add(tb, fronts), o_d = pack_add(tb, diag),
            o_tr = pack_add(tb, trsm), o_g = pack_add(tb, gemm), o_bo = pack_add(tb, borig), o_cb = pack_add(tb, cbr),
-           o_pa = pack_add(tb, pan), o_fl = pack_add(tb, flush), o_wo = pack_add(tb, woff);
+           o_pa = pack_add(tb, pan), o_fl = pack_add(tb, flush), o_he = pack_add(tb, head), o_wo = pack_add(tb, woff);
     BCHK(hipMalloc(&C.tbuf, tb.size()));
     BCHK(hipMemcpy(C.tbuf, tb.data(), tb.size(), hipMemcpyHostToDevice));
     char* t = (char*)C.tbuf;
@@ -1702,6 +1826,7 @@ int upload(BigCircuit& C, std::string& err) {
     C.d_cbr = (int2*)(t + o_cb);
     C.d_pan = (int4*)(t + o_pa);
     C.d_flush = (int2*)(t + o_fl);
+    C.d_head = (int4*)(t + o_he);
     C.d_woff = (int64_t*)(t + o_wo);
 
     // workspace
@@ -1748,30 +1873,51 @@ int upload(BigCircuit& C, std::string& err) {
 //          large fronts: diagonal block, triangular solves, trailing update
 //          spread over many workgroups.
 // Both compute the same values in the same order (bit-identical fronts).
-void launch_level(BigCircuit& C, hipStream_t s, int l, bool fused) {
+// pend: the level whose factored panels still wait in the workspace, or -1;
+// with pend null the level's own are copied back at once.
+void launch_flush(BigCircuit& C, hipStream_t s, int l) {
+    auto& Lv = C.levels[l];
+    MF_LAUNCH(CS_MFK_FLUSH, l, k_mf_flush, dim3(Lv.flush_n), dim3(kBT), 0, s, C.d_dev, C.pool, C.wpan, C.d_woff,
+              C.d_flush + Lv.flush_b);
+}
+void launch_level(BigCircuit& C, hipStream_t s, int l, bool fused, int* pend = nullptr) {
     const BigDev* P = C.d_dev;
     auto& Lv = C.levels[l];
-    if (Lv.small_n[0])
-        MF_LAUNCH(CS_MFK_SMALL32, l, (k_mf_lvl_small<8, 4>), dim3(Lv.small_n[0]), dim3(64), Lv.small_lds[0], s, P,
-                  C.pool, C.dinv, C.Aval, C.d_fronts + Lv.small_b[0]);
-    if (Lv.small_n[1])
-        MF_LAUNCH(CS_MFK_SMALL64, l, (k_mf_lvl_small<16, 4>), dim3(Lv.small_n[1]), dim3(256), Lv.small_lds[1], s, P,
-                  C.pool, C.dinv, C.Aval, C.d_fronts + Lv.small_b[1]);
-    if (Lv.small_n[2])
-        MF_LAUNCH(CS_MFK_SMALL96, l, (k_mf_lvl_small<16, 6>), dim3(Lv.small_n[2]), dim3(256), Lv.small_lds[2], s, P,
-                  C.pool, C.dinv, C.Aval, C.d_fronts + Lv.small_b[2]);
-    if (!Lv.big_n) return;
-    if (fused) {
-        MF_LAUNCH(CS_MFK_FRONT, l, k_mf_lvl_big, dim3(Lv.big_n), dim3(kBT), 0, s, P, C.pool, C.dinv, C.Aval,
-                  C.d_fronts + Lv.big_b);
-        return;
+    const bool head = Lv.head_n > 0 && !fused;
+    if (pend && *pend >= 0 && !(head && *pend == l - 1)) {
+        launch_flush(C, s, *pend);
+        *pend = -1;
     }
-    if (Lv.tile_n)
-        MF_LAUNCH(CS_MFK_GATHER, l, k_mf_gather, dim3(Lv.tile_n), dim3(kBT), 0, s, P, C.pool, C.d_tiles + Lv.tile_b,
-                  C.d_cbr);
-    if (Lv.orig_e > Lv.orig_b)
-        MF_LAUNCH(CS_MFK_ORIG, l, k_mf_orig, dim3(grid_for(Lv.orig_e - Lv.orig_b)), dim3(kBT), 0, s, P, C.Aval,
-                  C.pool, C.d_borig, Lv.orig_b, Lv.orig_e);
+    if (head) {
+        const int n_head = pend && *pend >= 0 ? Lv.head_nf : Lv.head_n;
+        MF_LAUNCH(CS_MFK_HEAD, l, k_mf_head, dim3(n_head), dim3(kBT), Lv.head_lds, s, P, C.pool, C.dinv, C.Aval,
+                  C.d_head + Lv.head_b, C.d_fronts, C.d_tiles, C.d_cbr, C.d_borig, C.wpan, C.d_woff, C.d_flush,
+                  Lv.head_lds32);
+        if (pend) *pend = -1;
+        if (!Lv.big_n) return;
+    } else {
+        if (Lv.small_n[0])
+            MF_LAUNCH(CS_MFK_SMALL32, l, (k_mf_lvl_small<8, 4>), dim3(Lv.small_n[0]), dim3(64), Lv.small_lds[0], s,
+                      P, C.pool, C.dinv, C.Aval, C.d_fronts + Lv.small_b[0]);
+        if (Lv.small_n[1])
+            MF_LAUNCH(CS_MFK_SMALL64, l, (k_mf_lvl_small<16, 4>), dim3(Lv.small_n[1]), dim3(256), Lv.small_lds[1],
+                      s, P, C.pool, C.dinv, C.Aval, C.d_fronts + Lv.small_b[1]);
+        if (Lv.small_n[2])
+            MF_LAUNCH(CS_MFK_SMALL96, l, (k_mf_lvl_small<16, 6>), dim3(Lv.small_n[2]), dim3(256), Lv.small_lds[2],
+                      s, P, C.pool, C.dinv, C.Aval, C.d_fronts + Lv.small_b[2]);
+        if (!Lv.big_n) return;
+        if (fused) {
+            MF_LAUNCH(CS_MFK_FRONT, l, k_mf_lvl_big, dim3(Lv.big_n), dim3(kBT), 0, s, P, C.pool, C.dinv, C.Aval,
+                      C.d_fronts + Lv.big_b);
+            return;
+        }
+        if (Lv.tile_n)
+            MF_LAUNCH(CS_MFK_GATHER, l, k_mf_gather, dim3(Lv.tile_n), dim3(kBT), Lv.tile_lds, s, P, C.pool,
+                      C.d_tiles + Lv.tile_b, C.d_cbr);
+        if (Lv.orig_e > Lv.orig_b)
+            MF_LAUNCH(CS_MFK_ORIG, l, k_mf_orig, dim3(grid_for(Lv.orig_e - Lv.orig_b)), dim3(kBT), 0, s, P, C.Aval,
+                      C.pool, C.d_borig, Lv.orig_b, Lv.orig_e);
+    }
     if (!C.split_panels) {
         for (auto& pn : Lv.panels) {
             if (C.mfma)
@@ -1781,8 +1927,8 @@ void launch_level(BigCircuit& C, hipStream_t s, int l, bool fused) {
                 MF_LAUNCH(CS_MFK_PANEL, l, k_mf_panel<false>, dim3(pn.pan_n), dim3(kBT), 0, s, P, C.pool, C.dinv,
                           C.wpan, C.d_woff, C.d_pan + pn.pan_b);
         }
-        MF_LAUNCH(CS_MFK_FLUSH, l, k_mf_flush, dim3(Lv.flush_n), dim3(kBT), 0, s, P, C.pool, C.wpan, C.d_woff,
-                  C.d_flush + Lv.flush_b);
+        if (pend) *pend = l;
+        else launch_flush(C, s, l);
         return;
     }
     for (auto& pn : Lv.panels) {
@@ -1803,7 +1949,9 @@ void launch_level(BigCircuit& C, hipStream_t s, int l, bool fused) {
 }
 
 void launch_factor(BigCircuit& C, hipStream_t s) {
-    for (int l = 0; l < (int)C.levels.size(); l++) launch_level(C, s, l, C.lvl_fused[l] != 0);
+    int pend = -1;
+    for (int l = 0; l < (int)C.levels.size(); l++) launch_level(C, s, l, C.lvl_fused[l] != 0, &pend);
+    if (pend >= 0) launch_flush(C, s, pend);
 }
 
 // The autotuner: for every level of this pattern, time both forms (the

@@ -280,6 +280,7 @@ int cs_big_times(cs_ctx* ctx, int32_t cid, double* factor_ms, double* solve_ms);
 #define CS_MFK_BWD     10  /* backward substitution of one level                       */
 #define CS_MFK_PANEL   11  /* one panel step in one launch (diagonal block, solves, update) */
 #define CS_MFK_FLUSH   12  /* factored panels of a level back from the workspace          */
+#define CS_MFK_HEAD    13  /* a level's small fronts, gather tiles and the last level's flush */
 int cs_big_profile(cs_ctx* ctx, int32_t cid, int32_t* kinds, int32_t* levels, float* ms, int32_t cap,
                    int32_t* count);
 
