@@ -59,6 +59,10 @@ struct BigDev {
     const double *mos_m, *src_m;           // m-factors, null when every m is 1
     const int32_t *sn_first, *sn_m, *sn_rptr, *sn_rows, *ch_ptr, *ch_sn, *rel_ptr, *rel, *inv, *olev_pos;
     const int32_t *osn_ptr, *osn_pos;
+    // per entry of ch_sn: (rows of the child's contribution block, its leading
+    // dimension, its rel_ptr, unused), and the block's offset in the pool
+    const int4* ch_rec;
+    const int64_t* ch_blk;
     const int32_t *row_long, *long_rows;   // rows too long for one lane (supply node, ...)
     const int32_t* long_cptr;              // [n_long+1] chunk range of each long row
     const int4* long_chunks;               // (row, kind, begin, end)
@@ -357,7 +361,7 @@ __device__ __forceinline__ void front_sync() {
 
 // Columns [j0, j1) of front s = the sum of its children's contribution
 // blocks, children in order, into F (column j0 at F[0], leading dimension
-// m): the columns are zeroed, then each child's block is added (one
+// ld): the columns are zeroed, then each child's block is added (one
 // wavefront per block column, lanes down the rows), with a barrier between
 // children.  Update row a of child c sits at row rel[a] of the parent.  br,
 // when given, holds per child the range of its block columns that land in
@@ -366,17 +370,23 @@ __device__ __forceinline__ void front_sync() {
 // NT threads, this one number tid; Global: F in global memory (fenced
 // barriers), else in LDS.
 template <int NT, bool Global>
-__device__ __forceinline__ void scatter_cb(const BigDev* P, const double* pool, double* F, int m, int s, int j0,
+__device__ __forceinline__ void scatter_cb(const BigDev* P, const double* pool, double* F, int ld, int s, int j0,
                                            int j1, const int2* br, int tid) {
-    for (int q = tid; q < (j1 - j0) * m; q += NT) F[q] = 0.0;
+    for (int q = tid; q < (j1 - j0) * ld; q += NT) F[q] = 0.0;
     if (Global) gsync();
     else front_sync<NT>();
     const int c0 = P->ch_ptr[s], c1 = P->ch_ptr[s + 1];
+    // the next child's record is read while this one is added
+    int4 next = c0 < c1 ? P->ch_rec[c0] : make_int4(0, 0, 0, 0);
+    int64_t next_blk = c0 < c1 ? P->ch_blk[c0] : 0;
     for (int cq = c0; cq < c1; cq++) {
-        const int c = P->ch_sn[cq];
-        const int mc = P->sn_m[c], kc = sn_k(P, c), rc = mc - kc;
-        const int* rl = P->rel + P->rel_ptr[c];
-        const double* blk = pool + P->sn_off[c] + (int64_t)kc * mc + kc;
+        const int rc = next.x, mc = next.y;
+        const int* rl = P->rel + next.z;
+        const double* blk = pool + next_blk;
+        if (cq + 1 < c1) {
+            next = P->ch_rec[cq + 1];
+            next_blk = P->ch_blk[cq + 1];
+        }
         int b0 = 0, b1 = rc;
         if (br) {
             const int2 r = br[cq - c0];
@@ -396,7 +406,7 @@ __device__ __forceinline__ void scatter_cb(const BigDev* P, const double* pool, 
                 const int q = q0 + u * NT;
                 if (q < tot) {
                     const int b = b0 + q / rc, a = q % rc;
-                    dst[u] = (rl[b] - j0) * m + rl[a];
+                    dst[u] = (rl[b] - j0) * ld + rl[a];
                     sv[u] = blk[(int64_t)b * mc + a];
                 }
             }
@@ -784,39 +794,65 @@ __device__ __forceinline__ double wave_bcast(double v, int src) {
 // pivot's column (Col: row) and every register index is fixed:
 //   row i:     l = a[0] * (1 / u(p,p)) is L(i,p);    a[j] = a[j+1] - l u(p,j)
 //   column j:  a[0] is U(p,j);  a[i] = a[i+1] - l(i,p) a[0], the same l
-// Each finished entry goes to out (one entry of the panel per pivot, kPanLd
-// apart).  Lanes at or before the pivot go on computing; nothing reads what
-// they hold.  W registers are still needed when the stage begins.
+// Lanes at or before the pivot go on computing; nothing reads what
+// holds.  W registers are still needed when the stage begins.  put(p, x, ip)
+// takes each finished entry x (row: L(i,p); column: U(p,j)) and 1 / u(p,p).
 constexpr int kStage = 8;
 constexpr int kPanLd = kNb + kTile + 1;
-template <bool Col, int W>
-__device__ __forceinline__ void panel_stage(double (&a)[kNb], int& p, int nb, double& ip, double* out) {
+template <bool Col, int W, class Put>
+__device__ __forceinline__ void panel_stage(double (&a)[kNb], int& p, int nb, double& ip, Put put) {
 #pragma unroll 1
     for (int q = 0; q < kStage && p < nb; q++, p++) {
         const double l = Col ? a[0] : a[0] * ip;
-        out[p * kPanLd] = l;
-        // the next pivot first: its reciprocal runs beside the other updates
+        put(p, l, ip);
         const double ipc = ip;
-        {
-            const double o = wave_bcast(a[1], p);
-            a[0] = Col ? a[1] - (o * ipc) * l : a[1] - l * o;
-        }
-        ip = 1.0 / wave_bcast(a[0], p + 1);
-#pragma unroll
-        for (int i = 1; i < W - 1; i++) {
+        auto update = [&](int i) {
             const double o = wave_bcast(a[i + 1], p);
             a[i] = Col ? a[i + 1] - (o * ipc) * l : a[i + 1] - l * o;
-        }
+        };
+        // the next pivot first; the dependent operations of its reciprocal
+        // (1.0 / x, step by step) then alternate with the other updates
+        update(0);
+        const double x = wave_bcast(a[0], p + 1);
+        constexpr int G = (W - 2 + 8) / 9;
+        int i = 1;
+        auto group = [&] {
+#pragma unroll
+            for (int g = 0; g < G; g++)
+                if (i < W - 1) update(i++);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        bool fd, fn;
+        const double d = __builtin_amdgcn_div_scale(1.0, x, false, &fd);
+        double r = __builtin_amdgcn_rcp(d);
+        group();
+        double e = __builtin_fma(-d, r, 1.0);
+        group();
+        r = __builtin_fma(r, e, r);
+        group();
+        e = __builtin_fma(-d, r, 1.0);
+        group();
+        r = __builtin_fma(r, e, r);
+        group();
+        const double n = __builtin_amdgcn_div_scale(1.0, x, true, &fn);
+        const double t = n * r;
+        group();
+        e = __builtin_fma(-d, t, n);
+        group();
+        e = __builtin_amdgcn_div_fmas(e, r, t, fn);
+        group();
+        ip = __builtin_amdgcn_div_fixup(e, x, 1.0);
+        group();
     }
 }
-template <bool Col>
-__device__ __forceinline__ void panel_lu(double (&a)[kNb], int nb, double* out) {
+template <bool Col, class Put>
+__device__ __forceinline__ void panel_lu(double (&a)[kNb], int nb, Put put) {
     int p = 0;
     double ip = 1.0 / wave_bcast(a[0], 0);
-    panel_stage<Col, 32>(a, p, nb, ip, out);
-    panel_stage<Col, 24>(a, p, nb, ip, out);
-    panel_stage<Col, 16>(a, p, nb, ip, out);
-    panel_stage<Col, 8>(a, p, nb, ip, out);
+    if (nb > 24) panel_stage<Col, 32>(a, p, nb, ip, put);
+    if (nb > 16) panel_stage<Col, 24>(a, p, nb, ip, put);
+    if (nb > 8) panel_stage<Col, 16>(a, p, nb, ip, put);
+    panel_stage<Col, 8>(a, p, nb, ip, put);
 }
 static_assert(kNb == 4 * kStage && kTile == 64 && kBT == 256, "panel_lu's stages and wavefronts");
 
@@ -833,7 +869,7 @@ static_assert(kNb == 4 * kStage && kTile == 64 && kBT == 256, "panel_lu's stages
 // first.  Now four wavefronts each carry the diagonal block's 32 rows (or
 // columns) beside 32 rows of L (columns of U) and go through the pivots
 // once, in registers, with no barrier and no LDS read: a step
-// of a 450 x 450 grid's factorization took 36 us, now 25.
+// of a 450 x 450 grid's factorization took 36 us, now 24.
 //
 // Workgroups of the step read the unfactored panel from the front,
 // so the factored panel goes to the workspace W instead (the same layout,
@@ -897,8 +933,9 @@ __global__ __launch_bounds__(kBT) void k_mf_panel(const BigDev* P, double* pool,
     for (int c = 0; c < kNb; c++) a[c] = mine[c * kPanLd];
     __syncthreads();   // the diagonal block is read by two wavefronts, then overwritten (same values) by both
     const int nbu = __builtin_amdgcn_readfirstlane(nb);
-    if (wave < 2) panel_lu<false>(a, nbu, mine);
-    else panel_lu<true>(a, nbu, mine);
+    auto put = [&](int p, double x, double) { mine[p * kPanLd] = x; };
+    if (wave < 2) panel_lu<false>(a, nbu, put);
+    else panel_lu<true>(a, nbu, put);
     __syncthreads();
     // the diagonal block: L below the diagonal in A, U in Bt
     const bool diag_owner = !tile || (i0 == p1 && j0 == p1);
@@ -1049,16 +1086,96 @@ __device__ __forceinline__ void small_front(const BigDev* P, double* pool, doubl
             if (i < m && j < m) G[(int64_t)j * m + i] = a[y][x];
         }
 }
+// Fronts of 33 to kSmallM rows, one workgroup each, in LDS (odd leading
+// dimension: a wavefront reads its columns without bank conflicts): blocks
+// of up to 32 pivots go as in k_mf_panel (wavefronts 0 and 1 rows, 2 and 3
+// columns, the block's own in lanes [0, nb) of each; 2 (64 - nb) lanes are
+// left for at most kSmallM - nb further ones), then the trailing block on
+// the FP64 matrix cores, the front's own value as the first addend, so an
+// entry is summed as the column sweep sums it.  Before, every pivot published
+// its row and column in LDS behind a barrier, with 16 or 36 entries a thread:
+// the fronts of 33 to 96 rows of a 450 x 450 grid took 0.73 ms per
+// factorization, now 0.45; a 150 x 150 grid's level heads 0.57 ms, now 0.37.
+static_assert(2 * (64 - kNb) >= kSmallM - kNb, "a panel's rows fit two wavefronts");
+__device__ __forceinline__ void mid_front(const BigDev* P, double* pool, double* dinv, const double* Aval, int s,
+                                          double* F) {
+    const int m = __builtin_amdgcn_readfirstlane(P->sn_m[s]), k = __builtin_amdgcn_readfirstlane(sn_k(P, s));
+    const int f0 = P->sn_first[s], ld = m | 1;
+    const int64_t off = P->sn_off[s];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    scatter_cb<kBT, false>(P, pool, F, ld, s, 0, m, nullptr, threadIdx.x);
+    for (int q = P->osn_ptr[s] + threadIdx.x; q < P->osn_ptr[s + 1]; q += kBT) {
+        const int e = P->osn_pos[q], d = (int)(P->nat_dest[e] - off), j = d / m;
+        F[j * ld + d - j * m] += Aval[e];
+    }
+    __syncthreads();
+    const int r16 = lane & 15, q4 = lane >> 4;
+    for (int p0 = 0; p0 < k; p0 += kNb) {
+        const int nb = (k - p0) < kNb ? (k - p0) : kNb, p1 = p0 + nb, rows = m - p1;
+        const bool col = wave >= 2, work = !(wave & 1) || rows > 64 - nb;
+        const int idx = lane < nb ? p0 + lane : p1 + (wave & 1) * (64 - nb) + lane - nb;
+        double* mine = F + (col ? idx * ld + p0 : p0 * ld + idx);
+        const int st = col ? 1 : ld;
+        double a[kNb];
+        if (work) {
+#pragma unroll
+            for (int c = 0; c < kNb; c++) a[c] = (c < nb && idx < m) ? mine[c * st] : 0.0;
+        }
+        __syncthreads();   // before a block row or column is overwritten
+        if (work) {
+            // of the diagonal block the rows keep what is below the diagonal,
+            // the columns the rest; both wavefronts of a kind store the same
+            const int lc = idx < m ? lane + (col ? 1 : 0) : -1;
+            auto put = [&](int p, double x, double ip) {
+                if (lc > p) mine[p * st] = x;
+                if (threadIdx.x == 0) dinv[f0 + p0 + p] = ip;
+            };
+            if (col) panel_lu<true>(a, nb, put);
+            else panel_lu<false>(a, nb, put);
+        }
+        __syncthreads();
+        const int nt = (rows + 15) >> 4;
+        for (int t = wave; t < nt * nt; t += kBT / 64) {
+            const int i0 = p1 + (t % nt) * 16, j0 = p1 + (t / nt) * 16;
+            dbl4 acc;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int i = i0 + q4 + 4 * v, j = j0 + r16;
+                acc[v] = (i < m && j < m) ? F[j * ld + i] : 0.0;
+            }
+            for (int kk = 0; kk < nb; kk += 4) {
+                const int c = kk + q4, i = i0 + r16, j = j0 + r16;
+                const double av = (c < nb && i < m) ? F[(p0 + c) * ld + i] : 0.0;
+                const double bv = (c < nb && j < m) ? F[j * ld + p0 + c] : 0.0;
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-av, bv, acc, 0, 0, 0);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int i = i0 + q4 + 4 * v, j = j0 + r16;
+                if (i < m && j < m) F[j * ld + i] = acc[v];
+            }
+        }
+        __syncthreads();
+    }
+    double* G = pool + off;
+    for (int j = wave; j < m; j += kBT / 64)
+        for (int i = lane; i < m; i += 64) G[j * m + i] = F[j * ld + i];
+}
+__global__ __launch_bounds__(kBT) void k_mf_lvl_mid(const BigDev* P, double* pool, double* dinv, const double* Aval,
+                                                    const int32_t* fronts) {
+    extern __shared__ double lds_f[];
+    mid_front(P, pool, dinv, Aval, fronts[blockIdx.x], lds_f);
+}
 template <int TL, int R>
 __global__ __launch_bounds__(TL * TL) void k_mf_lvl_small(const BigDev* P, double* pool, double* dinv,
                                                           const double* Aval, const int32_t* fronts) {
     extern __shared__ double lds_f[];
     small_front<TL, R>(P, pool, dinv, Aval, fronts[blockIdx.x], lds_f, threadIdx.x);
 }
-// size buckets: (threads per side, entries per side per thread)
+// size buckets: one wavefront per front, then one workgroup (by LDS size)
 constexpr int kSmallBuckets = 3;
 constexpr int kBucketMax[kSmallBuckets] = {32, 64, kSmallM};
-static_assert(8 * 4 >= 32 && 16 * 4 >= 64 && 16 * 6 >= kSmallM, "small-front buckets exceed their kernels");
+static_assert(8 * 4 >= kBucketMax[0], "small fronts exceed their kernel");
 
 // The independent work at the head of a level in one launch: its small
 // fronts of every bucket, the gather tiles of its large ones (with their
@@ -1069,10 +1186,10 @@ static_assert(8 * 4 >= 32 && 16 * 4 >= 64 && 16 * 6 >= kSmallM, "small-front buc
 // went from 1.34 to 1.00 ms (98 launches to 56).
 // item = (kind, a, b, c):
 //   kHeadSmall32: fronts[a, a + b), one wavefront each, b <= 4
-//   kHeadSmall64 / kHeadSmall96: front fronts[a]
+//   kHeadMid: front fronts[a]
 //   kHeadGather: tile a, Jacobian positions borig[b, c)
 //   kHeadFlush: flush item a
-enum { kHeadSmall32, kHeadSmall64, kHeadSmall96, kHeadGather, kHeadFlush };
+enum { kHeadSmall32, kHeadMid, kHeadGather, kHeadFlush };
 __global__ __launch_bounds__(kBT) void k_mf_head(const BigDev* P, double* pool, double* dinv, const double* Aval,
                                                  const int4* items, const int32_t* fronts, const int4* tiles,
                                                  const int2* cbr, const int32_t* borig, const double* W,
@@ -1083,10 +1200,8 @@ __global__ __launch_bounds__(kBT) void k_mf_head(const BigDev* P, double* pool, 
         const int wave = threadIdx.x >> 6;
         if (wave < it.z)
             small_front<8, 4>(P, pool, dinv, Aval, fronts[it.y + wave], lds_f + wave * lds32, threadIdx.x & 63);
-    } else if (it.x == kHeadSmall64) {
-        small_front<16, 4>(P, pool, dinv, Aval, fronts[it.y], lds_f, threadIdx.x);
-    } else if (it.x == kHeadSmall96) {
-        small_front<16, 6>(P, pool, dinv, Aval, fronts[it.y], lds_f, threadIdx.x);
+    } else if (it.x == kHeadMid) {
+        mid_front(P, pool, dinv, Aval, fronts[it.y], lds_f);
     } else if (it.x == kHeadGather) {
         gather_tile(P, pool, tiles[it.y], cbr, lds_f, Aval, borig + it.z, it.w - it.z);
     } else {
@@ -1266,10 +1381,12 @@ __global__ __launch_bounds__(BT) void k_mf_fwd(const BigDev* P, const double* po
     const double* G = pool + P->sn_off[s];
     for (int a = threadIdx.x; a < m; a += BT) v[a] = a < k ? x[f0 + a] : 0.0;
     __syncthreads();
-    for (int cq = P->ch_ptr[s]; cq < P->ch_ptr[s + 1]; cq++) {
-        const int c = P->ch_sn[cq];
-        const int rc = P->sn_rptr[c + 1] - P->sn_rptr[c];
-        for (int a = threadIdx.x; a < rc; a += BT) v[P->rel[P->rel_ptr[c] + a]] += uvec[P->rel_ptr[c] + a];
+    const int c0 = P->ch_ptr[s], c1 = P->ch_ptr[s + 1];
+    int4 next = c0 < c1 ? P->ch_rec[c0] : make_int4(0, 0, 0, 0);
+    for (int cq = c0; cq < c1; cq++) {
+        const int rc = next.x, rp = next.z;
+        if (cq + 1 < c1) next = P->ch_rec[cq + 1];
+        for (int a = threadIdx.x; a < rc; a += BT) v[P->rel[rp + a]] += uvec[rp + a];
         __syncthreads();
     }
     // blocks of 64 pivots: the diagonal block (staged in LDS) by the first
@@ -1617,6 +1734,13 @@ int upload(BigCircuit& C, std::string& err) {
     for (int32_t q = 0; q < P.n_mos; q++)
         mos4.push_back(make_int4(P.mos[4 * q], P.mos[4 * q + 1], P.mos[4 * q + 2], P.mos[4 * q + 3]));
     for (auto& s : P.src) src4.push_back(make_int4(s.kind, s.off, s.len, s.dc));
+    std::vector<int4> ch_rec;
+    std::vector<int64_t> ch_blk;
+    for (int32_t c : B.ch_sn) {
+        const int kc = B.sn_first[c + 1] - B.sn_first[c], mc = B.sn_m[c];
+        ch_rec.push_back(make_int4(mc - kc, mc, B.rel_ptr[c], 0));
+        ch_blk.push_back(B.sn_off[c] + (int64_t)kc * mc + kc);
+    }
     size_t o_rp = pack_add(by, P.nat_rowptr), o_col = pack_add(by, P.nat_col), o_lk = pack_add(by, P.lin_kind),
            o_li = pack_add(by, P.lin_idx), o_gp = pack_add(by, P.g_ptr), o_gr = pack_add(by, P.g_ref),
            o_cp = pack_add(by, P.c_ptr), o_cr = pack_add(by, P.c_ref), o_jp = pack_add(by, P.jnl_ptr),
@@ -1630,7 +1754,7 @@ int upload(BigCircuit& C, std::string& err) {
            o_probe = pack_add(by, P.probe), o_osp = pack_add(by, B.osn_ptr), o_osq = pack_add(by, B.osn_pos),
            o_rl = pack_add(by, row_long), o_lr = pack_add(by, long_rows), o_lcp = pack_add(by, long_cptr),
            o_lch = pack_add(by, long_chunks), o_ls = pack_add(by, P.lin_scale), o_mm = pack_add(by, P.mos_m),
-           o_smm = pack_add(by, P.src_m);
+           o_smm = pack_add(by, P.src_m), o_crec = pack_add(by, ch_rec), o_cblk = pack_add(by, ch_blk);
     BCHK(hipMalloc(&C.dbuf, by.size()));
     BCHK(hipMemcpy(C.dbuf, by.data(), by.size(), hipMemcpyHostToDevice));
     char* b = (char*)C.dbuf;
@@ -1652,6 +1776,7 @@ int upload(BigCircuit& C, std::string& err) {
     d.sn_first = I(o_sf); d.sn_m = I(o_sm); d.sn_rptr = I(o_srp); d.sn_rows = I(o_srow);
     d.ch_ptr = I(o_chp); d.ch_sn = I(o_chs); d.rel_ptr = I(o_relp); d.rel = I(o_rel); d.inv = I(o_inv);
     d.olev_pos = I(o_olp); d.sn_off = L(o_soff); d.inv_ptr = L(o_invp); d.nat_dest = L(o_nd);
+    d.ch_rec = (const int4*)(b + o_crec); d.ch_blk = L(o_cblk);
     d.osn_ptr = I(o_osp); d.osn_pos = I(o_osq);
     d.row_long = I(o_rl); d.long_rows = I(o_lr); d.n_long = (int32_t)long_rows.size();
     d.long_cptr = I(o_lcp); d.long_chunks = (const int4*)(b + o_lch); d.n_chunks = (int32_t)long_chunks.size();
@@ -1726,9 +1851,7 @@ int upload(BigCircuit& C, std::string& err) {
             fronts.insert(fronts.end(), small[bk].begin(), small[bk].end());
             Lv.small_n[bk] = (int)small[bk].size();
             const int sm = small_max[bk];
-            Lv.small_lds[bk] = sizeof(double) * (bk == 0   ? small_doubles<8, 4>(sm)
-                                                 : bk == 1 ? small_doubles<16, 4>(sm)
-                                                           : small_doubles<16, 6>(sm));
+            Lv.small_lds[bk] = sizeof(double) * (bk == 0 ? small_doubles<8, 4>(sm) : sm * (sm | 1));
         }
         // the head's items: what takes longest first, the previous level's
         // panel copies last (left out when that level wrote no workspace)
@@ -1737,7 +1860,7 @@ int upload(BigCircuit& C, std::string& err) {
         Lv.head_lds = 0;
         for (int bk = 2; bk >= 1; bk--) {
             for (int q = 0; q < Lv.small_n[bk]; q++)
-                head.push_back(make_int4(bk == 2 ? kHeadSmall96 : kHeadSmall64, Lv.small_b[bk] + q, 0, 0));
+                head.push_back(make_int4(kHeadMid, Lv.small_b[bk] + q, 0, 0));
             if (Lv.small_n[bk]) Lv.head_lds = std::max(Lv.head_lds, (int)Lv.small_lds[bk]);
         }
         head.insert(head.end(), h_gather.begin(), h_gather.end());
@@ -1900,10 +2023,10 @@ void launch_level(BigCircuit& C, hipStream_t s, int l, bool fused, int* pend = n
             MF_LAUNCH(CS_MFK_SMALL32, l, (k_mf_lvl_small<8, 4>), dim3(Lv.small_n[0]), dim3(64), Lv.small_lds[0], s,
                       P, C.pool, C.dinv, C.Aval, C.d_fronts + Lv.small_b[0]);
         if (Lv.small_n[1])
-            MF_LAUNCH(CS_MFK_SMALL64, l, (k_mf_lvl_small<16, 4>), dim3(Lv.small_n[1]), dim3(256), Lv.small_lds[1],
+            MF_LAUNCH(CS_MFK_SMALL64, l, k_mf_lvl_mid, dim3(Lv.small_n[1]), dim3(256), Lv.small_lds[1],
                       s, P, C.pool, C.dinv, C.Aval, C.d_fronts + Lv.small_b[1]);
         if (Lv.small_n[2])
-            MF_LAUNCH(CS_MFK_SMALL96, l, (k_mf_lvl_small<16, 6>), dim3(Lv.small_n[2]), dim3(256), Lv.small_lds[2],
+            MF_LAUNCH(CS_MFK_SMALL96, l, k_mf_lvl_mid, dim3(Lv.small_n[2]), dim3(256), Lv.small_lds[2],
                       s, P, C.pool, C.dinv, C.Aval, C.d_fronts + Lv.small_b[2]);
         if (!Lv.big_n) return;
         if (fused) {

@@ -15,6 +15,7 @@ import scipy.sparse.linalg as spl
 
 import cedarhip as ch
 from cedarhip import lib as L
+from cedarhip.netlist import Gnd, Named, R, lower, net
 from cedarhip.workloads import rc_mesh
 from oracle import oracle as O
 
@@ -173,3 +174,45 @@ def test_full_span_matches_oracle(engine):
     wb = np.asarray(sol.wave)
     wr = np.asarray(w).reshape(wb.shape)
     assert np.all(np.abs(wb - wr) <= 1e-6 * np.abs(wr) + 1e-9)
+
+
+# (k, r): a clique of k nodes eliminated against a clique of r further ones,
+# so the assembly tree holds fronts of about k + r rows with k pivots and of
+# r: the edges of the one-wavefront kernel (32 rows), of a block of pivots
+# (32), of the wavefronts that carry a block's rows (64), of the fronts kept
+# whole in LDS (96) and of the panel steps above
+@pytest.mark.parametrize("k,r", [(1, 31), (1, 32), (8, 57), (8, 88), (31, 33), (32, 32), (33, 30), (32, 64),
+                                 (33, 63), (64, 32), (95, 1), (33, 64), (65, 40), (3, 130)])
+def test_front_sizes_match_sparse_lu(engine, k, r):
+    """Factor and solve at the edges of the front kernels.  The conductance
+    matrix is diagonally dominant, so elimination without pivoting grows no
+    entry beyond twice the largest, and the normwise backward error of LU and
+    its two solves stays within 3 m (rows of a front) units of rounding of
+    the growth: 6 m eps."""
+    rng = np.random.default_rng(1000 * k + r)
+    n = 3 * k + r
+    cliques = [np.r_[c * k:(c + 1) * k, 3 * k:n] for c in range(3)]   # three children, one shared separator
+    pairs = np.unique(np.vstack([np.stack([c[i], c[j]], 1) for c in cliques
+                                 for i, j in [np.triu_indices(len(c), 1)]]), axis=0)
+
+    def circuit():
+        gnd = Named(net, "gnd")()
+        v = [Named(net, f"v{i}")() for i in range(n)]
+        for q, (i, j) in enumerate(pairs):
+            Named(R(rng.uniform(0.5, 2.0)), f"R{q}")(v[i], v[j])
+        for i in range(n):
+            Named(R(rng.uniform(0.5, 2.0)), f"G{i}")(v[i], gnd)
+        Gnd()(gnd)
+
+    f = lower(circuit)
+    s = engine.load(f, solver=L.SOLVER_SUPERNODAL)
+    A = s.jac_matrix(None, np.zeros(s.n), f.params(), 0.0, 0.0)
+    b = rng.standard_normal(s.n)
+    s.lu_refactor(A.data)
+    x = s.lu_solve(b)
+    berr = np.max(np.abs(A @ x - b)) / (abs(A).sum(axis=1).max() * np.max(np.abs(x)) + np.max(np.abs(b)))
+    _say(f"k {k} r {r}: max front {s.big_info.max_front}, max pivots {s.big_info.max_pivots}, "
+         f"backward error {berr:.2e}")
+    assert berr < 6 * (k + r) * 2.0**-53
+    s.lu_refactor(A.data)
+    assert np.array_equal(x, s.lu_solve(b))
