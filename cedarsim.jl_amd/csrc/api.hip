@@ -1401,6 +1401,94 @@ int cs_tran(cs_ctx* ctx, int32_t cid, const double* p, const double* u0, const c
     return tran_plain(ctx, cid, p, u0, o, wave, u_final, st_out, nullptr);
 }
 
+// A sensitivity run goes in one launch (k_tran_sens) where a wavefront holds
+// one unknown per lane, the factors fit the default LDS, and every
+// parameter's wavefront is resident at once (four per CU).  Modified Newton,
+// Verilog-A devices and larger circuits keep the host's step control, and
+// CS_BATCH_KERNEL_GLOBAL asks for it.
+static bool sens_fits(const cs_ctx* ctx, const Circuit& C, const cs_tran_opts& o, int32_t n_sp) {
+    const Plan& P = C.plan;
+    return o.batch_kernel == CS_BATCH_KERNEL_AUTO && o.jac_reuse == 0 && P.n_va == 0 && P.n <= kSensMaxN &&
+           tran_sens_lds(P.n, P.nnz, P.n_stamp) <= 40 * 1024 && n_sp <= 4 * std::max(ctx->n_cu, 1);
+}
+
+static int sens_single(cs_ctx* ctx, Circuit& C, const double* p, const double* u0, const cs_tran_opts* o,
+                       const std::vector<SensParam>& sp, double* wave, double* sens, double* u_final,
+                       cs_tran_stats* st_out) {
+    const Plan& P = C.plan;
+    int rc = check_params(ctx, P, p);
+    if (rc) return rc;
+    const bool uic = o->init == CS_INIT_UIC;
+    if (uic && !u0) return fail(ctx, CS_E_INVALID, "UIC initialisation needs u0");
+    if (uic && !P.uic_ok)
+        return fail(ctx, CS_E_INVALID, "UIC: a charge-carrying row could not be kept on its own pivot");
+    if (o->n_out > 0 && !(o->dt_out > 0)) return fail(ctx, CS_E_INVALID, "dt_out must be > 0");
+    (void)hipSetDevice(ctx->device);
+    const int32_t n = P.n, n_sp = (int32_t)sp.size(), np = (int32_t)P.probe.size(), n_out = std::max(o->n_out, 0);
+    size_t at = 0;
+    auto take = [&](size_t bytes) { const size_t off = at; at = (at + bytes + 255) & ~size_t(255); return off; };
+    const size_t blk = (size_t)n_sp * np;
+    SensRunArgs a{};
+    a.ws_stride = (size_t)P.n_lin + 2 * (size_t)P.nnz;
+    const size_t o_sp = take(sizeof(SensParam) * n_sp), o_prow = take(sizeof(int32_t) * n),
+                 o_p = take(sizeof(double) * P.lay.n_params), o_u0 = take(sizeof(double) * n),
+                 o_ws = take(sizeof(double) * a.ws_stride * n_sp), o_st = take(sizeof(cs_tran_stats)),
+                 o_u = take(sizeof(double) * n), o_w = take(sizeof(double) * (size_t)n_out * np),
+                 o_s = take(sizeof(double) * (size_t)n_out * blk);
+    char* d = nullptr;
+    HIPCHK(ctx, hipMalloc((void**)&d, at));
+    a.P = C.d_dplan;
+    a.p = (const double*)(d + o_p);
+    a.u0 = uic ? (const double*)(d + o_u0) : nullptr;
+    a.prow = (const int32_t*)(d + o_prow);
+    a.sp = (const SensParam*)(d + o_sp);
+    a.ws = (double*)(d + o_ws);
+    a.wave = n_out && np ? (double*)(d + o_w) : nullptr;
+    a.sens = (double*)(d + o_s);
+    a.u_final = (double*)(d + o_u);
+    a.stats = (cs_tran_stats*)(d + o_st);
+    a.n_sp = n_sp; a.n = n; a.nnz = P.nnz; a.n_lin = P.n_lin; a.n_stamp = P.n_stamp; a.n_probe = np;
+    a.o = *o;
+    hipStream_t s = ctx->stream;
+    cs_tran_stats st{};
+    std::vector<double> u(n), hw((size_t)n_out * np), hs((size_t)n_out * blk);
+    auto run = [&]() -> int {
+        HIPCHK(ctx, hipMemcpyAsync(d + o_sp, sp.data(), sizeof(SensParam) * n_sp, hipMemcpyHostToDevice, s));
+        HIPCHK(ctx, hipMemcpyAsync(d + o_prow, P.prow.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, s));
+        HIPCHK(ctx, hipMemcpyAsync(d + o_p, p, sizeof(double) * P.lay.n_params, hipMemcpyHostToDevice, s));
+        if (uic) HIPCHK(ctx, hipMemcpyAsync(d + o_u0, u0, sizeof(double) * n, hipMemcpyHostToDevice, s));
+        HIPCHK(ctx, launch_tran_sens(a, s));
+        HIPCHK(ctx, hipMemcpyAsync(&st, d + o_st, sizeof(st), hipMemcpyDeviceToHost, s));
+        HIPCHK(ctx, hipMemcpyAsync(u.data(), d + o_u, sizeof(double) * n, hipMemcpyDeviceToHost, s));
+        if (a.wave) {
+            HIPCHK(ctx, hipMemcpyAsync(hw.data(), a.wave, sizeof(double) * hw.size(), hipMemcpyDeviceToHost, s));
+            HIPCHK(ctx, hipMemcpyAsync(hs.data(), a.sens, sizeof(double) * hs.size(), hipMemcpyDeviceToHost, s));
+        }
+        HIPCHK(ctx, hipStreamSynchronize(s));
+        return CS_OK;
+    };
+    rc = run();
+    (void)hipFree(d);
+    if (rc) return rc;
+    // the samples up to the time reached; a run that stops early leaves the others
+    int32_t rows = 0;
+    if (a.wave && st.retcode != CS_E_NOCONV)
+        while (rows < n_out && o->t_start + rows * o->dt_out <= st.t_end + 1e-9 * o->dt_out) rows++;
+    if (rows) {
+        std::memcpy(wave, hw.data(), sizeof(double) * (size_t)rows * np);
+        std::memcpy(sens, hs.data(), sizeof(double) * (size_t)rows * blk);
+    }
+    if (u_final) std::memcpy(u_final, u.data(), sizeof(double) * n);
+    st.busy_s = 0.0;
+    if (st_out) *st_out = st;
+    rc = st.retcode;
+    if (rc == CS_E_DTMIN) ctx->err = "transient: step size fell below dt_min";
+    else if (rc == CS_E_NOCONV)
+        ctx->err = std::string("transient: initial point did not converge") + (uic ? "" : dc_pivot_note(P));
+    else if (rc == CS_E_MAXSTEPS) ctx->err = "transient: max_steps reached";
+    return rc;
+}
+
 int cs_tran_sens(cs_ctx* ctx, int32_t cid, const double* p, const double* u0, const cs_tran_opts* o,
                  int32_t n_sp, const int32_t* sp_idx, double* wave, double* sens, double* u_final,
                  cs_tran_stats* st_out) {
@@ -1420,6 +1508,7 @@ int cs_tran_sens(cs_ctx* ctx, int32_t cid, const double* p, const double* u0, co
         R.sp[j].val = p ? p[sp_idx[j]] : 0.0;
     }
     if (!p) return fail(ctx, CS_E_INVALID, "bad argument");
+    if (sens_fits(ctx, *C, *o, n_sp)) return sens_single(ctx, *C, p, u0, o, R.sp, wave, sens, u_final, st_out);
     const int n = P.n, np = (int)P.probe.size();
     R.S.assign(3 * (size_t)n_sp * np, 0.0);
     R.s_nat.assign((size_t)n_sp * n, 0.0);

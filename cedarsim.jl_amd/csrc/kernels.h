@@ -110,6 +110,27 @@ struct SensArgs {
 };
 hipError_t launch_sens(const SensArgs& a, hipStream_t s);
 
+// A whole sensitivity run in one launch (k_tran_sens): one wavefront per
+// parameter.
+struct SensRunArgs {
+    const DPlan* P;
+    const double* p;
+    const double* u0;         // may be null (DC-op init)
+    const int32_t* prow;      // natural row -> pivot row
+    const SensParam* sp;
+    double* ws;               // per parameter: ws_stride doubles (linear slots, G, C)
+    size_t ws_stride;
+    double* wave;             // [n_out][n_probe], or null: no output samples
+    double* sens;             // [n_out][n_sp][n_probe]
+    double* u_final;
+    cs_tran_stats* stats;
+    int32_t n_sp, n, nnz, n_lin, n_stamp, n_probe;
+    cs_tran_opts o;
+};
+constexpr int kSensMaxN = 64;   // one unknown per lane
+size_t tran_sens_lds(int32_t n, int32_t nnz, int32_t n_stamp);
+hipError_t launch_tran_sens(const SensRunArgs& a, hipStream_t s);
+
 struct CPlan;
 
 // LDS-resident batched transient (tran_lds.hip): one launch per size class.

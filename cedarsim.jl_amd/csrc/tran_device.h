@@ -4,8 +4,9 @@
 // wavefront) owns one circuit instance; lane l owns unknowns l, l+64, ...
 // (NR of them) and keeps their history in registers.
 //
-// Rec is a recording policy called on every accepted point (including the
-// initial one, as step 0); the batch passes NoRec.
+// Rec is called at the points a forward sensitivity run needs (sens.hip): the
+// DC point and the initial point, each with its Jacobian just assembled in
+// L.F, every accepted step, and every output sample; the batch passes NoRec.
 #pragma once
 #include "dcop_rules.h"
 #include "device.h"
@@ -15,19 +16,16 @@ namespace cedar {
 
 constexpr int NT = kBatchThreads;
 
-struct NoRec {
-    template <int NR>
-    __device__ __forceinline__ bool on_accept(const DPlan*, const double*, double, double, int,
-                                              long long, const double*, const double*,
-                                              const double*) {
-        return true;
-    }
-    __device__ __forceinline__ void on_finish(int, long long) {}
-};
-
-
 struct Lds {
     double *F, *inv, *u, *x, *qx, *st;
+};
+
+struct NoRec {
+    __device__ __forceinline__ void on_dc(const DPlan*, const double*, const Lds&, const double*) {}
+    __device__ __forceinline__ void on_initial(const DPlan*, const double*, const Lds&, const double*, bool) {}
+    __device__ __forceinline__ void on_step(const DPlan*, const double*, const Lds&, const double*, const double*,
+                                            double, int, double, double, double) {}
+    __device__ __forceinline__ void on_output(const DPlan*, int, double, double, double) {}
 };
 
 template <int NR, class Rec>
@@ -88,6 +86,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
                     }
                 }
                 if (!dc_done) { ok = true; break; }
+                rec.on_dc(P, p, L, Clin);
                 for (int i = tid; i < n; i += NT) L.qx[i] = L.u[i];
                 dev_sources<NT>(P, p, o.t_start, CS_MODE_TRAN, L.st);
                 pin = L.qx;
@@ -129,6 +128,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
     double t = o.t_start;
     if (rc == CS_OK) {
         __syncthreads();
+        rec.on_initial(P, p, L, Clin, uic);
         dev_charges<NT>(P, Clin, L.u, L.qx);
         __syncthreads();
 #pragma unroll
@@ -136,7 +136,6 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
             const int i = tid + NT * r;
             if (i < n) { Uh0[r] = L.u[i]; Qh0[r] = L.qx[i]; }
         }
-        rec.template on_accept<NR>(P, L.u, o.t_start, o.t_start, 0, 0, Uh0, Uh1, Uh2);
         double T0 = o.t_start, T1 = 0.0, T2 = 0.0;
         int npts = 1;
         double h = sd.dt_init;
@@ -152,6 +151,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
                         if (sl >= 0) wave[(size_t)kout * n_probe + sl] = Uh0[r];
                     }
                 }
+                rec.on_output(P, kout, 1.0, 0.0, 0.0);
                 kout++;
             }
         }
@@ -248,6 +248,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
                 fac = accept_factor(err, k);
             }
             // accept
+            rec.on_step(P, p, L, Glin, Clin, gmin, k, a0, a1, a2);
             dev_charges<NT>(P, Clin, L.u, L.qx);
             __syncthreads();
 #pragma unroll
@@ -257,10 +258,6 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
                     Uh2[r] = Uh1[r]; Uh1[r] = Uh0[r]; Uh0[r] = L.u[i];
                     Qh1[r] = Qh0[r]; Qh0[r] = L.qx[i];
                 }
-            }
-            if (!rec.template on_accept<NR>(P, L.u, tn, T0, npts, steps + 1, Uh0, Uh1, Uh2)) {
-                rc = CS_E_RANGE;
-                break;
             }
             T2 = T1; T1 = T0; T0 = tn;
             if (npts < 3) npts++;
@@ -289,6 +286,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
                                     l0 * Uh0[r] + l1 * Uh1[r] + l2 * Uh2[r];
                         }
                     }
+                    rec.on_output(P, kout, l0, l1, l2);
                     kout++;
                 }
             }
@@ -306,7 +304,6 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
         const int i = tid + NT * r;
         if (i < n) ufin[i] = (rc == CS_OK || steps > 0) ? Uh0[r] : L.u[i];
     }
-    rec.on_finish(rc, steps);
     if (tid == 0) {
         stp->steps = steps;
         stp->rejected = rej;

@@ -20,7 +20,7 @@ import pytest
 import cedarhip as ch
 from cedarhip import lib as L
 from cedarhip.netlist import WAVE_DC
-from cedarhip.workloads import inverter
+from cedarhip.workloads import VDD, inverter, ring_oscillator
 from oracle import oracle as O
 
 import circuits as K
@@ -120,3 +120,47 @@ def test_refuses_unsupported_parameters(engine):
     lay = flat.layout()
     with pytest.raises(ch.CedarHIPError):
         sys_.tran_sens(ch.grid_options((0.0, 1e-10), n_out=3), [lay["gmin"]])
+
+
+@pytest.mark.parametrize("case", ["inverter", "butterworth_uic", "controlled", "ring61_uic", "ring63_uic"])
+def test_one_launch_matches_host_step_control(engine, case):
+    """A sensitivity run of up to 64 unknowns goes in one launch; with
+    BATCH_KERNEL_GLOBAL the host controls its steps.  The same rules on the
+    same plan, with sums reduced over 64 lanes instead of 256: the same
+    steps, and values equal up to rounding carried through the steps, held to
+    the bar of the waveform parity tests (1e-6 relative) and 1e-9 of the
+    parameter's largest sensitivity.  63 and 65 unknowns are the sizes beside the limit; the
+    last takes the host's path either way."""
+    u0, kw = None, {}
+    if case == "inverter":
+        flat, span = ch.lower(inverter()), (0.0, 1e-9)
+        names = ["MN.vth", "MN.kp", "MP.w", "MP.l", "CL", "VDD.dc"]
+    elif case == "butterworth_uic":
+        flat, span = ch.lower(K.butterworth), (0.0, 4.0)
+        names, u0 = ["L1", "C2", "L3", "R4"], np.zeros(flat.n)
+    elif case == "controlled":
+        flat, span = ch.lower(K.spice_controlled), (0.0, 1e-6)
+        names = [nm for nm, (kind, k) in flat.device_names.items() if kind in ("vccs", "vcvs", "res")]
+    else:
+        ns = 61 if case == "ring61_uic" else 63
+        flat, span = ch.lower(ring_oscillator(ns)), (0.0, 2e-11)
+        names = ["MN0.vth", f"MP{ns - 1}.w", "VDD.dc"]
+        u0 = np.zeros(flat.n)
+        u0[flat.names["vdd"]] = VDD
+        for k in range(ns):
+            u0[flat.names[f"s{k}"]] = VDD * (k % 2)
+    if u0 is not None:
+        kw["init"] = L.INIT_UIC
+    sys_ = engine.load(flat, solver=L.SOLVER_LEVEL)
+    run = {}
+    for kern in (L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_GLOBAL):
+        o = ch.grid_options(span, n_out=21, batch_kernel=kern, **kw)
+        run[kern] = sys_.tran_sens(o, names, flat.params(), u0=u0)
+    (ra, ga), (rg, gg) = run[L.BATCH_KERNEL_AUTO], run[L.BATCH_KERNEL_GLOBAL]
+    assert ra.retcode == rg.retcode == "Success"
+    assert ra.stats.steps == rg.stats.steps and ra.stats.rejected == rg.stats.rejected
+    assert np.all(np.abs(ra.wave - rg.wave) <= 1e-6 * np.abs(rg.wave) + 1e-9)
+    for j in range(len(names)):
+        a, b = ga[:, j], gg[:, j]
+        _say(f"{case} {names[j]}: max |s| {np.max(np.abs(b)):.3e}, difference {np.max(np.abs(a - b)):.2e}")
+        assert np.all(np.abs(a - b) <= 1e-6 * np.abs(b) + 1e-9 * np.max(np.abs(b)) + 1e-300), names[j]
