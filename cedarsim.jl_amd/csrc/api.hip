@@ -2040,10 +2040,15 @@ int ac_sweep(cs_ctx* ctx, Circuit& C, AcArgs a, const double* omega, const std::
              const std::vector<int32_t>& obs_piv, const std::vector<int32_t>& nz_rows,
              const std::vector<double>& nz_pwr, const std::vector<double>& nz_exp, double* out, double* psd) {
     const Plan& P = C.plan;
-    const size_t stride = 2 * (size_t)P.nnz + 4 * (size_t)P.n + 2;
+    // a frequency in LDS where at least two fit a CU, else in the workspace.
+    // Those circuits have few hundred unknowns at most: one wavefront (four
+    // measured the same on a 12 x 11 mesh)
+    const size_t fit = ac_lds(P.n, P.nnz);
+    const size_t lds = P.n <= 512 && fit <= 76 * 1024 ? fit : 0;
+    const size_t stride = lds ? 0 : 2 * (size_t)P.nnz + 4 * (size_t)P.n + 2;
     const size_t budget = (size_t)1 << 28;   // doubles of workspace: 2 GiB
     int64_t nblocks = std::min<int64_t>(a.n_freq, std::max<int64_t>(4 * std::max(ctx->n_cu, 1), 1));
-    nblocks = std::max<int64_t>(1, std::min<int64_t>(nblocks, (int64_t)(budget / stride)));
+    nblocks = std::max<int64_t>(1, std::min<int64_t>(nblocks, (int64_t)(budget / std::max<size_t>(stride, 1))));
     Packer pk;
     std::vector<double> om(omega, omega + a.n_freq);
     const size_t o_om = pk.add(om), o_rhs = pk.add(rhs), o_obs = pk.add(obs_piv), o_nr = pk.add(nz_rows),
@@ -2072,7 +2077,7 @@ int ac_sweep(cs_ctx* ctx, Circuit& C, AcArgs a, const double* omega, const std::
         a.psd = d_out;
         a.ws = d_out + n_out_al;
         a.ws_stride = stride;
-        HIPCHK(ctx, launch_ac(a, (int)nblocks, P.n <= 512 ? 64 : 256, s));
+        HIPCHK(ctx, launch_ac(a, (int)nblocks, P.n <= 512 ? 64 : 256, lds, s));
         HIPCHK(ctx, hipMemcpyAsync(a.transposed ? psd : out, d_out, sizeof(double) * n_out, hipMemcpyDeviceToHost, s));
         HIPCHK(ctx, hipStreamSynchronize(s));
         return CS_OK;

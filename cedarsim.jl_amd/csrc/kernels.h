@@ -69,7 +69,10 @@ struct AcArgs {
     const double* nz_exp;
     double* psd;              // [n_freq]
 };
-hipError_t launch_ac(const AcArgs& a, int nblocks, int nt, hipStream_t s);
+// LDS for one frequency's factors, reciprocals, solution and substitution
+// schedules; lds = 0 keeps the first three in the workspace
+size_t ac_lds(int32_t n, int32_t nnz);
+hipError_t launch_ac(const AcArgs& a, int nblocks, int nt, size_t lds, hipStream_t s);
 
 // Forward parameter sensitivities of the plain-path transient (sens.hip):
 // one parameter's stamps.  Indices are natural (-1: ground).

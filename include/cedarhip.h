@@ -424,7 +424,7 @@ int cs_bsimcmg_eval_noalloc(cs_ctx* ctx, int64_t n, const double* L, const doubl
                             const double* v, double temp_c, double* out, int32_t* iters);
 
 /* ODEForwardSensitivityProblem + extract_local_sensitivities
- * (test/sensitivity.jl:13-66): cs_tran (plain path) together with the
+ * (test/sensitivity.jl:13-66): cs_tran together with the
  * forward sensitivities d(probed unknown)/d p of n_sp parameters, sp_idx[j]
  * an index into the parameter vector: res_r, cap_c, ind_l, vccs_gain,
  * vcvs_gain, mos_vth/kp/w/l, and wave_dc of a source (its DC value, which
@@ -436,6 +436,8 @@ int cs_bsimcmg_eval_noalloc(cs_ctx* ctx, int64_t n, const double* L, const doubl
  * follow its construction (charge rows fixed at u0 under UIC; with the DC
  * operating point, the DC point's sensitivity pins them).  wave as cs_tran
  * (required); sens: n_out x n_sp x n_probe, interpolated like wave.
+ * Circuits of up to 64 unknowns run in one launch; larger ones, jac_reuse,
+ * Verilog-A devices and CS_BATCH_KERNEL_GLOBAL take the plain path.
  * Circuits on the supernodal solver are refused. */
 int cs_tran_sens(cs_ctx* ctx, int32_t cid, const double* p, const double* u0, const cs_tran_opts* o,
                  int32_t n_sp, const int32_t* sp_idx, double* wave, double* sens, double* u_final,

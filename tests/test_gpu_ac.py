@@ -140,3 +140,36 @@ def test_rc_mesh_ac_and_noise(engine, nx, ny):
             yb = np.where(nb >= 0, y[np.maximum(nb, 0)], 0)
             ref[f] = np.sum(pwr * np.abs(ya - yb) ** 2)
     np.testing.assert_allclose(psd, ref, rtol=1e-10)
+
+
+@pytest.mark.parametrize("nx,ny,nf", [(1, 1, 3), (8, 8, 7), (13, 5, 1100), (12, 12, 9), (16, 15, 9), (20, 19, 9)])
+def test_ac_kernel_forms(engine, nx, ny, nf):
+    """Sizes around the kernel's choices: one unknown, 64 and 65 (a level fills
+    the wavefront or not), meshes that keep a frequency in LDS and that do
+    not, and more frequencies than workgroups.  A dense complex solve of the
+    same G + jwC bounds the difference by the condition of a passive mesh
+    (below 1e2 at these values) times 6 n units of rounding: 1e-12 with room."""
+    flat = ch.lower(_mesh(nx, ny, nx * 100 + ny))
+    sys_ = engine.load(flat, solver=L.SOLVER_LEVEL)
+    dc = sys_.dcop()
+    ws = np.logspace(7, 12, nf)
+    obs = ["n0_0", f"n{nx - 1}_{ny - 1}"]
+    X = sys_.ac(dc.u, ws, obs)
+    o = flat.index(obs[-1])
+    psd = sys_.noise(dc.u, ws, o)
+    G = O.jacobian(flat, flat.params(), dc.u, 0.0, 0.0, L.MODE_DCOP)
+    Cm = O.cmatrix(flat, flat.params(), dc.u)
+    rows = flat.arrays["res_nodes"].reshape(-1, 2)
+    r = flat.params()[flat.layout()["res_r"]:][:len(rows)]
+    b = np.zeros(flat.n)
+    b[flat.index("n0_0")] = 1.0
+    e = np.zeros(flat.n)
+    e[o] = 1.0
+    for k in range(0, nf, max(1, nf // 11)):
+        J = G + 1j * ws[k] * Cm
+        x = np.linalg.solve(J, b)
+        got, ref = X[k], x[[flat.index(q) for q in obs]]
+        assert np.max(np.abs(got - ref)) <= 1e-12 * np.max(np.abs(x)), (k, got, ref)
+        y = np.append(np.linalg.solve(J.T, e), 0.0)   # -1: ground
+        ref = np.sum(4 * 1.380649e-23 * 300.15 / r * np.abs(y[rows[:, 0]] - y[rows[:, 1]]) ** 2)
+        assert abs(psd[k] - ref) <= 1e-10 * ref
