@@ -1253,6 +1253,19 @@ struct SingleRun {
     size_t up, down0, down; // bytes to copy up; the results' range
 };
 
+// The device buffer and its pinned image outlive the call up to kSingleKeep
+// bytes; a run whose samples need more than kSingleMax stays on the plain
+// path, which writes them straight to the caller's array.
+constexpr size_t kSingleKeep = (size_t)64 << 20, kSingleMax = (size_t)1 << 30;
+
+static void single_trim(Circuit& C) {
+    if (C.sbuf_bytes <= kSingleKeep) return;
+    (void)hipFree(C.sbuf);
+    (void)hipHostFree(C.h_sbuf);
+    C.sbuf = C.h_sbuf = nullptr;
+    C.sbuf_bytes = 0;
+}
+
 static int single_buffers(cs_ctx* ctx, Circuit& C, const cs_tran_opts& o, bool with_u0, int32_t n_out, SingleRun& R) {
     const Plan& P = C.plan;
     size_t at = 0;
@@ -1342,6 +1355,7 @@ static int tran_single(cs_ctx* ctx, Circuit& C, const double* p, const double* u
     R.st->busy_s /= ctx->clock_hz;
     if (st_out) *st_out = *R.st;
     rc = R.st->retcode;
+    single_trim(C);   // R's pointers end here
     if (rc == CS_E_DTMIN) ctx->err = "transient: step size fell below dt_min";
     else if (rc == CS_E_NOCONV)
         ctx->err = std::string("transient: initial point did not converge") +
@@ -1396,6 +1410,7 @@ int cs_tran(cs_ctx* ctx, int32_t cid, const double* p, const double* u0, const c
     // factors modified Newton keeps are those full Newton recomputes, so such
     // a circuit takes the same kernel and the same bits either way.
     if (o && C && p && !C->big && C->lds_nr && o->batch_kernel == CS_BATCH_KERNEL_AUTO &&
+        (!wave || sizeof(double) * std::max(o->n_out, 0) * C->plan.probe.size() <= kSingleMax) &&
         (o->jac_reuse == 0 || (o->jac_reuse == 1 && C->plan.n_mos == 0)))
         return tran_single(ctx, *C, p, u0, o, wave, u_final, st_out);
     return tran_plain(ctx, cid, p, u0, o, wave, u_final, st_out, nullptr);
@@ -1403,13 +1418,15 @@ int cs_tran(cs_ctx* ctx, int32_t cid, const double* p, const double* u0, const c
 
 // A sensitivity run goes in one launch (k_tran_sens) where a wavefront holds
 // one unknown per lane, the factors fit the default LDS, and every
-// parameter's wavefront is resident at once (four per CU).  Modified Newton,
+// parameter's wavefront is resident at once (four per CU); its samples are
+// held on the device up to kSingleMax bytes.  Modified Newton,
 // Verilog-A devices and larger circuits keep the host's step control, and
 // CS_BATCH_KERNEL_GLOBAL asks for it.
 static bool sens_fits(const cs_ctx* ctx, const Circuit& C, const cs_tran_opts& o, int32_t n_sp) {
     const Plan& P = C.plan;
     return o.batch_kernel == CS_BATCH_KERNEL_AUTO && o.jac_reuse == 0 && P.n_va == 0 && P.n <= kSensMaxN &&
-           tran_sens_lds(P.n, P.nnz, P.n_stamp) <= 40 * 1024 && n_sp <= 4 * std::max(ctx->n_cu, 1);
+           tran_sens_lds(P.n, P.nnz, P.n_stamp) <= 40 * 1024 && n_sp <= 4 * std::max(ctx->n_cu, 1) &&
+           sizeof(double) * std::max(o.n_out, 0) * P.probe.size() * (n_sp + 1) <= kSingleMax;
 }
 
 static int sens_single(cs_ctx* ctx, Circuit& C, const double* p, const double* u0, const cs_tran_opts* o,

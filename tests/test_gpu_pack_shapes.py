@@ -114,3 +114,19 @@ def test_early_stop_leaves_later_samples(engine):
         done = r.t <= r.stats.t_end * (1 + 1e-9)
         assert done.any() and not done.all()
         assert np.all(r.wave[done, 0] > 1.0) and np.all(r.wave[~done] == 0.0)
+
+
+def test_large_sample_buffer_is_given_back(engine):
+    """More than 64 MiB of samples: the buffer kept per circuit is freed after
+    the call, and the next calls, large and small, give the same samples
+    (every 100,000th sample of the large run is one of the small run's)."""
+    print("[gpu] large sample buffer", flush=True)
+    flat = ch.lower(inverter())
+    s = engine.load(flat)
+    m = 100_000
+    n_out = 20 * m + 1
+    assert n_out * len(s.probes) * 8 > 64 << 20
+    runs = [s.tran(ch.grid_options((0.0, 1e-9), n_out=k)) for k in (21, n_out, 21, n_out)]
+    assert all(r.retcode == "Success" for r in runs)
+    assert np.array_equal(runs[0].wave, runs[2].wave) and np.array_equal(runs[1].wave, runs[3].wave)
+    assert np.all(np.abs(runs[1].wave[::m] - runs[0].wave) <= 1e-9 * np.abs(runs[0].wave) + 1e-9)
