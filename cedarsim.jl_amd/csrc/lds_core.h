@@ -51,7 +51,8 @@ constexpr int W = 64;
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & (W - 1)); }
 
 // 1/a: the hardware estimate and two Newton corrections (error below one
-// ulp); an infinite estimate (a = 0 or subnormal) stands as it is.
+// ulp); where they are not defined (a infinite, 0 or subnormal with an infinite
+// estimate) the estimate stands: 0 or an infinity, as a division gives.
 __device__ __forceinline__ double recip(double a) {
     const double r0 = __builtin_amdgcn_rcp(a);
     double r = r0;
@@ -59,14 +60,15 @@ __device__ __forceinline__ double recip(double a) {
     r = __builtin_fma(r, e, r);
     e = __builtin_fma(-a, r, 1.0);
     r = __builtin_fma(r, e, r);
-    return __builtin_isinf(r0) ? r0 : r;
+    return r == r ? r : r0;
 }
 
 // a / b for step control: the quotient by recip, corrected once by its
-// residual.
+// residual (which is not defined for an infinite a or quotient).
 __device__ __forceinline__ double quot(double a, double b) {
     const double r = recip(b), q = a * r;
-    return __builtin_fma(__builtin_fma(-q, b, a), r, q);
+    const double e = __builtin_fma(-q, b, a);
+    return e == e ? __builtin_fma(e, r, q) : q;
 }
 
 // s^(-1/(2(k+1))), k = 1 or 2, for s within [1e-6, 1e8]: the step factor's

@@ -130,3 +130,30 @@ def test_large_sample_buffer_is_given_back(engine):
     assert all(r.retcode == "Success" for r in runs)
     assert np.array_equal(runs[0].wave, runs[2].wave) and np.array_equal(runs[1].wave, runs[3].wave)
     assert np.all(np.abs(runs[1].wave[::m] - runs[0].wave) <= 1e-9 * np.abs(runs[0].wave) + 1e-9)
+
+
+def test_infinite_tolerance_and_span(engine):
+    """abstol = inf weighs every error with 0: each step converges in one
+    iteration and is accepted.  An infinite t_stop has no default for dt_max,
+    and the run ends at max_steps.  The LDS-resident kernels divide by a
+    reciprocal of their own, so 1/inf and inf/x are theirs to get right: the
+    one launch and a batch take the plain path's and the oracle's steps."""
+    print("[gpu] infinite abstol, infinite t_stop", flush=True)
+    flat = ch.lower(inverter())
+    s = engine.load(flat)
+    p = flat.params()
+    for kw, n_out, want in (({"abstol": np.inf, "t_stop": 1e-9, "dt_out": 2.5e-10}, 5, "Success"),
+                            ({"t_stop": np.inf, "dt_init": 1e-13, "dt_min": 1e-20, "max_steps": 60}, 0, "MaxIters")):
+        runs = []
+        for kern in (L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_GLOBAL):
+            r = s.tran(ch.TranOptions(n_out=n_out, batch_kernel=kern, **kw), p)
+            runs.append((r.retcode, r.stats, r.wave, r.u_final))
+        o = ch.TranOptions(n_out=n_out, batch_kernel=L.BATCH_KERNEL_LDS, **kw)
+        b = ch.tran_batch([flat, flat], [p, p], o, engine=engine)
+        runs += [(b.retcodes[i], b.stats[i], b.wave[i], b.u_final[i]) for i in range(2)]
+        w, uf, st, rc = O.tran(flat, p, None, o)
+        for code, stats, wave, u in runs:
+            assert code == want
+            assert (stats.steps, stats.rejected, stats.newton_iters) == (st.steps, st.rejected, st.newton_iters)
+            assert np.all(np.abs(wave - w[:n_out]) <= 1e-6 * np.abs(w[:n_out]) + 1e-9)
+            assert np.all(np.abs(u - uf) <= 1e-6 * np.abs(uf) + 1e-9)
