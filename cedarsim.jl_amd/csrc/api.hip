@@ -875,7 +875,7 @@ int cs_dcop(cs_ctx* ctx, int32_t cid, const double* p, const cs_tran_opts* o, do
         if (rc) ctx->err = err;
         return rc;
     }
-    if (C->lds_nr) return dcop_single(ctx, *C, p, o, u_out, st);
+    if (C->lds_nr && o->batch_kernel != CS_BATCH_KERNEL_GLOBAL) return dcop_single(ctx, *C, p, o, u_out, st);
     if ((rc = ensure_workspace(ctx, *C)) || (rc = ensure_graph(ctx, *C))) return rc;
     const Plan& P = C->plan;
     HIPCHK(ctx, hipMemcpyAsync(C->w.p, p, sizeof(double) * P.lay.n_params, hipMemcpyHostToDevice, ctx->stream));

@@ -328,7 +328,8 @@ int cs_dcop(cs_ctx* ctx, int32_t cid, const double* p, const cs_tran_opts* o,
  * asks for the first (refused for supernodal circuits, circuits that do not
  * fit, and jac_reuse), CS_BATCH_KERNEL_GLOBAL for the plain path.
  * wave: n_out x n_probe samples; u_final: n.  u0 may be NULL for INIT_DCOP.
- * cs_dcop takes the same kernel code where the circuit fits. */
+ * cs_dcop takes the same kernel code where the circuit fits, and the plain
+ * path with CS_BATCH_KERNEL_GLOBAL. */
 int cs_tran(cs_ctx* ctx, int32_t cid, const double* p, const double* u0,
             const cs_tran_opts* o, double* wave, double* u_final,
             cs_tran_stats* st);

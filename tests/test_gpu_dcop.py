@@ -1,6 +1,7 @@
 """GPU DC operating point: CedarDCOp's trajectories (src/dcop.jl:53-94) and
-the gmin ladder on every path - plain (cs_dcop, cs_tran), supernodal, and
-both batched kernels (INIT_DCOP) - against the oracle and the closed form."""
+the gmin ladder on every path - the one launch and the plain path (cs_dcop,
+cs_tran), supernodal, and both batched kernels (INIT_DCOP) - against the
+oracle and the closed form."""
 import numpy as np
 import pytest
 
@@ -15,12 +16,16 @@ pytestmark = pytest.mark.gpu
 CASES = [("restart_vth0", 0.0), ("gmin_ladder_vth04", 0.4)]
 
 
+KERNELS = [L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_GLOBAL]   # the one launch (where a circuit fits), the plain path
+
+
 @pytest.mark.parametrize("name,vth", CASES)
 @pytest.mark.parametrize("solver", [L.SOLVER_LEVEL, L.SOLVER_SUPERNODAL])
-def test_dcop_restarts_plain(engine, name, vth, solver):
-    print(f"[gpu] dcop {name} solver {solver}", flush=True)
+@pytest.mark.parametrize("kernel", KERNELS)
+def test_dcop_restarts_plain(engine, name, vth, solver, kernel):
+    print(f"[gpu] dcop {name} solver {solver} kernel {kernel}", flush=True)
     flat = ch.lower(K.diode_nmos(vth), gmin=0.0)
-    sol = engine.load(flat, solver=solver).dcop()
+    sol = engine.load(flat, solver=solver).dcop(opts=ch.TranOptions(batch_kernel=kernel))
     u_ref, _, rc = O.dcop(flat, flat.params())
     assert rc == 0 and sol.retcode == "Success"
     assert sol["a"] == pytest.approx(K.diode_nmos_exact(vth), abs=1e-6)
@@ -45,10 +50,11 @@ def test_dcop_restarts_batched(engine, kernel):
     assert r.retcodes[2] == "InitialFailure"
 
 
-def test_dcop_failure_plain(engine):
-    print("[gpu] dcop failure plain", flush=True)
+@pytest.mark.parametrize("kernel", KERNELS)
+def test_dcop_failure_plain(engine, kernel):
+    print(f"[gpu] dcop failure plain, kernel {kernel}", flush=True)
     flat = ch.lower(K.floating_cap)
     sys = engine.load(flat)
-    assert sys.dcop().retcode == "InitialFailure"
-    sol = sys.tran(ch.grid_options((0.0, 1e-9), n_out=11))
+    assert sys.dcop(opts=ch.TranOptions(batch_kernel=kernel)).retcode == "InitialFailure"
+    sol = sys.tran(ch.grid_options((0.0, 1e-9), n_out=11, batch_kernel=kernel))
     assert sol.retcode == "InitialFailure"

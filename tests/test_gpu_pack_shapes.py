@@ -10,7 +10,7 @@ import pytest
 
 import cedarhip as ch
 from cedarhip import lib as L
-from cedarhip.workloads import inverter, rc_mesh, ring_initial_state, ring_oscillator
+from cedarhip.workloads import NMOS, PMOS, VDD, inverter, rc_mesh, ring_initial_state, ring_oscillator
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -63,7 +63,7 @@ def test_packed_shapes_match_oracle(engine, kind, count):
 
 @pytest.mark.parametrize("name", ["inverter", "ring5", "ring67", "ring149", "mesh", "butterworth", "vr"])
 def test_cs_tran_and_dcop_take_one_launch(engine, name):
-    """cs_tran by default and cs_dcop on the LDS-resident kernel against the
+    """cs_tran and cs_dcop by default, on the LDS-resident kernel, against the
     plain path (batch_kernel = CS_BATCH_KERNEL_GLOBAL) and the oracle, with
     probes, without an output grid, and a second call with other values."""
     import circuits as K
@@ -95,9 +95,9 @@ def test_cs_tran_and_dcop_take_one_launch(engine, name):
         assert np.array_equal(c.u_final, a.u_final) and c.wave.shape[0] == 0
         if u0 is None:
             ud, _, rcd = O.dcop(flat, p)
-            dc = s.dcop(p)
-            assert dc.retcode == "Success" and rcd == 0
-            assert np.max(np.abs(dc.u - ud)) <= 1e-9 * max(1.0, np.max(np.abs(ud)))
+            for dc in (s.dcop(p), s.dcop(p, ch.TranOptions(batch_kernel=L.BATCH_KERNEL_GLOBAL))):
+                assert dc.retcode == "Success" and rcd == 0
+                assert np.max(np.abs(dc.u - ud)) <= 1e-9 * max(1.0, np.max(np.abs(ud)))
     s.set_probes([1, 0])
     d = s.tran(ch.grid_options((0.0, span), n_out=7, **kw), p, u0)
     assert np.array_equal(d.wave, a.wave[:, [1, 0]])
@@ -157,3 +157,43 @@ def test_infinite_tolerance_and_span(engine):
             assert (stats.steps, stats.rejected, stats.newton_iters) == (st.steps, st.rejected, st.newton_iters)
             assert np.all(np.abs(wave - w[:n_out]) <= 1e-6 * np.abs(w[:n_out]) + 1e-9)
             assert np.all(np.abs(u - uf) <= 1e-6 * np.abs(uf) + 1e-9)
+
+
+def test_dcop_kernel_choice(engine):
+    """cs_dcop runs on the kernel that batch_kernel names.  Without charges the
+    initial point of a transient is the DC point itself, so a run of no steps
+    returns each kernel's own point, to the bit; the two kernels sum in
+    another order, and over a few parameter sets their points differ."""
+    print("[gpu] dcop kernel choice", flush=True)
+
+    def circuit():
+        vdd, vin, gnd = (ch.Named(ch.net, k)() for k in ("vdd", "in", "gnd"))
+        ch.Named(ch.V(VDD), "VDD")(vdd, gnd)
+        ch.Named(ch.V(0.85), "VIN")(vin, gnd)
+        a = vin
+        for k in range(8):
+            y = ch.Named(ch.net, f"s{k}")()
+            ch.Named(ch.SquareLawMOSFET(**NMOS), f"MN{k}")(y, a, gnd, gnd)
+            ch.Named(ch.SquareLawMOSFET(**PMOS), f"MP{k}")(y, a, vdd, vdd)
+            a = y
+        ch.Gnd()(gnd)
+
+    flat = ch.lower(circuit)
+    s = engine.load(flat)
+    lay = flat.layout()
+    rng = np.random.default_rng(11)
+    differ = 0
+    for _ in range(8):
+        p = flat.params()
+        p[lay["mos_vth"]:lay["mos_vth"] + 16] += 0.02 * rng.standard_normal(16)
+        ud, _, rcd = O.dcop(flat, p)
+        u = {}
+        for kern in (L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_GLOBAL):
+            o = ch.TranOptions(t_stop=1e-9, max_steps=0, batch_kernel=kern)
+            dc = s.dcop(p, o)
+            assert dc.retcode == "Success" and rcd == 0
+            assert np.max(np.abs(dc.u - ud)) <= 1e-9 * np.max(np.abs(ud))
+            assert np.array_equal(dc.u, s.tran(o, p).u_final)
+            u[kern] = dc.u
+        differ += not np.array_equal(u[L.BATCH_KERNEL_AUTO], u[L.BATCH_KERNEL_GLOBAL])
+    assert differ > 0
