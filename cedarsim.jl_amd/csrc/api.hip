@@ -1654,7 +1654,9 @@ static int build_lds_classes(cs_ctx* ctx, Batch& B, const std::function<int(void
 // Monte Carlo be resident at once.  A batch that does not fill the device is
 // spread over its CUs instead: a chunk takes no more instances than there
 // would be per CU, since wavefronts on one CU share its LDS and issue ports
-// (60 rings over 500 ps: 8 CUs at 8 wavefronts each before).  Returns
+// (60 rings over 500 ps: 8 CUs at 8 wavefronts each before).  A workgroup has
+// the wavefronts of the fullest chunk, no more: where LDS holds only a few
+// instances, idle ones would keep a second workgroup off the CU.  Returns
 // CS_E_RANGE when a circuit does not fit even one wavefront beside its image.
 static int build_pack(cs_ctx* ctx, Batch& B, const std::function<int(void**, size_t)>& dalloc) {
     const std::vector<int32_t>&used = B.used, &c_nr = B.c_nr;
@@ -1677,16 +1679,33 @@ static int build_pack(cs_ctx* ctx, Batch& B, const std::function<int(void**, siz
         ks.dyn = ks.dyn || ctx->circuits[c]->lds_dyn;
     }
     const int64_t n_cu = std::max(ctx->n_cu, 1);
-    ks.waves = (int32_t)std::min<int64_t>(kPackWaves, (B.n_inst + n_cu - 1) / n_cu);
-    // four wavefronts per SIMD only where the batch has more than two
-    ks.occ = ks.nr <= 2 && B.n_inst > kPackWaves * n_cu ? 4 : 2;
+    const int32_t spread = (int32_t)std::min<int64_t>(kPackWaves, (B.n_inst + n_cu - 1) / n_cu);
     std::vector<std::vector<int32_t>> per(nc);
     for (int32_t i = 0; i < B.n_inst; i++) per[B.cid[i]].push_back(i);
     std::vector<size_t> rem(nc, 0), next(nc, 0);
     for (int32_t c : cs) rem[c] = per[c].size();
     size_t need = 0;
-    const std::vector<std::vector<PackSeg>> chunks = pack_chunks(cs, img, dblb, rem, ks.waves, kPackSegs, kPackLds, &need);
+    const std::vector<std::vector<PackSeg>> chunks = pack_chunks(cs, img, dblb, rem, spread, kPackSegs, kPackLds, &need);
     if (chunks.empty() && B.n_inst > 0) return CS_E_RANGE;
+    const size_t C = chunks.size();
+    for (const auto& ch : chunks) {
+        int32_t cnt = 0;
+        for (const PackSeg& g : ch) cnt += g.cnt;
+        ks.waves = std::max(ks.waves, cnt);
+    }
+    int per_cu = pack_max_blocks(ks, need);
+    // the registers for four wavefronts per SIMD where the batch has more than
+    // two, or where only they hold every chunk at once
+    if (ks.nr <= 2) {
+        PackShape k4 = ks;
+        k4.occ = 4;
+        const int per_cu4 = pack_max_blocks(k4, need);
+        if (B.n_inst > kPackWaves * n_cu || ((int64_t)C > per_cu * n_cu && per_cu4 > per_cu)) {
+            ks = k4;
+            per_cu = per_cu4;
+        }
+    }
+    if (per_cu <= 0) return fail(ctx, CS_E_RANGE, "packed LDS kernel does not fit on a CU");
     // When the chunks outnumber the resident workgroups by E, the E extra
     // chunks start when the first workgroups finish.  The chunks come largest
     // circuit first, and a larger circuit takes longer; so the queue puts the
@@ -1694,9 +1713,6 @@ static int build_pack(cs_ctx* ctx, Batch& B, const std::function<int(void**, siz
     // E smallest (descending): the workgroups that finish first take a second
     // small chunk, the largest of those first, instead of a large chunk being
     // followed by a small one.
-    const int per_cu = pack_max_blocks(ks, need);
-    if (per_cu <= 0) return fail(ctx, CS_E_RANGE, "packed LDS kernel does not fit on a CU");
-    const size_t C = chunks.size();
     B.pack_blocks = (int32_t)std::min<int64_t>((int64_t)C, per_cu * n_cu);
     std::vector<size_t> qorder(C);
     for (size_t i = 0; i < C; i++) qorder[i] = i;

@@ -23,10 +23,14 @@ using namespace lds;
 // 101 ms; 1001 inverters over 2 ns from their DC points 16.5 -> 11.0 ms.
 //
 // OCC wavefronts per SIMD.  OCC = 4 (128 VGPRs): two workgroups of eight per
-// CU, so that every instance of a 4096-instance batch is resident at once.
-// OCC = 2 (256 VGPRs) for batches that fill no more, and for circuits of
-// more than 128 rows (NR = 4), which are LDS-bound below that.  DYN: some
-// circuit has a source that is not DC.
+// CU, so that every instance of a 4096-instance batch is resident at once; also
+// where LDS holds few instances beside an image and only so many registers
+// let a second workgroup in (2048 101-stage rings over 20 ps, five to a
+// workgroup: 12.3 ms in two rounds, 7.9 in one).  OCC = 2 (256 VGPRs) for
+// batches that fill no more, and for circuits of more than 128 rows (NR = 4,
+// 196 VGPRs, of which LDS holds at most three beside an image: two workgroups
+// of their own size fit; 1536 149-stage rings 15.0 ms when workgroups had eight
+// wavefronts, 8.5 now).  DYN: some circuit has a source that is not DC.
 template <int NR, bool DYN, int OCC>
 __global__ __launch_bounds__(W* kPackWaves) __attribute__((amdgpu_waves_per_eu(OCC)))
 void k_tran_pack(const LdsArgs* args) {
@@ -191,11 +195,19 @@ PackKernel pack_kernel(const PackShape& k) {
 }
 }  // namespace
 
+// A CU deals a workgroup's wavefronts to its four SIMDs from the first one on,
+// so a workgroup of five takes two places on that one: of three per SIMD they
+// leave no room for a second workgroup, which the occupancy query (twelve
+// places, ten taken) admits.  2048 101-stage rings, five to a workgroup,
+// went in two rounds that way.
 int pack_max_blocks(const PackShape& k, size_t lds) {
-    int nb = 0;
+    int nb = 0, per_simd = 0;
     const PackKernel f = pack_kernel(k);
-    if (!f || hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, W * k.waves, lds) != hipSuccess) return 0;
-    return nb;
+    if (!f || hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, W * k.waves, lds) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_simd, f, W * 4, 0) != hipSuccess)
+        return 0;
+    const int by_simd = per_simd / ((k.waves + 3) / 4);
+    return nb < by_simd ? nb : by_simd;
 }
 
 hipError_t launch_tran_pack(const PackShape& k, const LdsArgs* d_args, int nblocks, size_t lds, hipStream_t s) {

@@ -10,6 +10,7 @@ import pytest
 
 import cedarhip as ch
 from cedarhip import lib as L
+from cedarhip.engine import pack_plan
 from cedarhip.workloads import NMOS, PMOS, VDD, inverter, rc_mesh, ring_initial_state, ring_oscillator
 from oracle import oracle as O
 
@@ -197,3 +198,27 @@ def test_dcop_kernel_choice(engine):
             u[kern] = dc.u
         differ += not np.array_equal(u[L.BATCH_KERNEL_AUTO], u[L.BATCH_KERNEL_GLOBAL])
     assert differ > 0
+
+
+@pytest.mark.parametrize("n,count", [(101, 1300), (101, 2048), (149, 1536), (175, 1024)])
+def test_lds_bound_batch_is_resident_at_once(engine, n, count):
+    """Batches whose chunks hold five, three or two instances for LDS: two
+    workgroups share a CU, so the launch lasts as long as its longest
+    instance.  In two rounds it takes twice that."""
+    print(f"[gpu] resident batch {n} {count}", flush=True)
+    rng = np.random.default_rng(n)
+    flat = ch.lower(ring_oscillator(n))
+    u0 = ring_initial_state(flat, rng)
+    chunks, _ = pack_plan([flat], [count])
+    assert 256 < len(chunks) <= 512   # more than the CUs, no more than two each
+    o = ch.TranOptions(t_stop=5e-12, init=L.INIT_UIC, batch_kernel=L.BATCH_KERNEL_LDS)
+    s = engine.load(flat)
+    b = ch.Batch(engine, [s], [0] * count, [flat.params()] * count, o, [u0] * count)
+    try:
+        b.run()
+        ms = b.run()
+        r = b.results(ms)
+    finally:
+        b.close()
+    assert set(r.retcodes) == {"Success"}
+    assert ms <= 1.4e3 * max(st.busy_s for st in r.stats)
