@@ -363,13 +363,11 @@ AdjKernel adj_kernel(int nr, bool dyn, bool reverse) {
 }
 }  // namespace
 
-int adj_lds_max_blocks(int nr, bool dyn, size_t lds) {
-    int nb[2] = {0, 0};
-    for (int r = 0; r < 2; r++) {
-        const AdjKernel f = adj_kernel(nr, dyn, r != 0);
-        if (!f || hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb[r], f, W, lds) != hipSuccess) return 0;
-    }
-    return nb[0] < nb[1] ? nb[0] : nb[1];
+int adj_lds_max_blocks(int nr, bool dyn, bool reverse, size_t lds) {
+    int nb = 0;
+    const AdjKernel f = adj_kernel(nr, dyn, reverse);
+    if (!f || hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, W, lds) != hipSuccess) return 0;
+    return nb;
 }
 
 hipError_t launch_adj_lds(int nr, bool dyn, bool reverse, const AdjLdsArgs* a, int nblocks, size_t lds, hipStream_t s) {

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <functional>
 #include <cstdio>
@@ -68,12 +69,13 @@ constexpr size_t kLdsMaxBytes = 64 * 1024;   // dynamic LDS of one workgroup
 constexpr size_t kPackLds = 80 * 1024 - 256; // packed launch: two workgroups per CU
 constexpr size_t kSideStreams = 4;           // hardware queues of one process
 
-// One launch of the LDS-resident kernel: the instances of circuits whose
-// LDS footprints are within a factor of each other.
+// One launch of the adjoint's forward kernel and one of its reverse kernel:
+// the instances of circuits whose LDS footprints are within a factor of each
+// other.
 struct LdsClass {
     int32_t nr = 1, n_inst = 0;
     bool dyn = false;                          // some source is not DC
-    size_t lds = 0;
+    size_t lds[2] = {0, 0};                    // forward (the image without the adjoint's part), reverse
     LdsArgs args{};
 };
 
@@ -1604,11 +1606,12 @@ static int build_lds_classes(cs_ctx* ctx, Batch& B, const std::function<int(void
     B.d_queues = (int32_t*)d_q;
     for (size_t k = 0; k < members.size(); k++) {
         LdsClass L;
-        int32_t dbl_max = 2, words_max = 8;
+        int32_t dbl_max = 2, words_max[2] = {8, 8};
         for (int32_t c : members[k]) {
             const CPlan& cp = ctx->circuits[c]->hcp;
             dbl_max = std::max(dbl_max, (cp.dbl + 1) & ~1);
-            words_max = std::max(words_max, cp.words_adj);
+            words_max[0] = std::max(words_max[0], cp.words);
+            words_max[1] = std::max(words_max[1], cp.words_adj);
             L.nr = std::max(L.nr, B.c_nr[c]);
             L.dyn = L.dyn || ctx->circuits[c]->lds_dyn;
         }
@@ -1620,7 +1623,7 @@ static int build_lds_classes(cs_ctx* ctx, Batch& B, const std::function<int(void
         if ((rc = dalloc(&d_order, sizeof(int32_t) * order.size()))) return rc;
         HIPCHK(ctx, hipMemcpy(d_order, order.data(), sizeof(int32_t) * order.size(), hipMemcpyHostToDevice));
         L.n_inst = (int32_t)order.size();
-        L.lds = lds_kernel_bytes(dbl_max, words_max);
+        for (int r = 0; r < 2; r++) L.lds[r] = lds_kernel_bytes(dbl_max, words_max[r]);
         L.args = base;
         L.args.order = (const int32_t*)d_order;
         L.args.queue = B.d_queues + k;
@@ -2460,14 +2463,19 @@ int cs_adjoint_batch(cs_ctx* ctx, int32_t n_inst, const int32_t* inst_cid, const
     HIPCHK(ctx, hipMemcpy(d_goff, g_off.data(), sizeof(int64_t) * n_inst, hipMemcpyHostToDevice));
     HIPCHK(ctx, hipMemcpy(d_obj, obj.data(), sizeof(int32_t) * obj.size(), hipMemcpyHostToDevice));
     std::vector<AdjLdsArgs> args(ncls);
-    std::vector<int> nblk(ncls);
+    // resident workgroups of each kernel by its own LDS: the forward kernel's
+    // image is a quarter smaller (768 185-stage rings over 3 ps: 14.4 ms with
+    // both at the reverse's, 11.9 now)
+    std::vector<std::array<int, 2>> nblk(ncls);
     for (size_t k = 0; k < ncls; k++) {
         const LdsClass& L = B->classes[k];
-        const int per_cu = adj_lds_max_blocks(L.nr, L.dyn, L.lds);
-        if (per_cu <= 0) return fail(ctx, CS_E_RANGE, "adjoint kernels do not fit on a CU");
-        nblk[k] = (int)std::min<int64_t>(L.n_inst, (int64_t)per_cu * std::max(ctx->n_cu, 1));
+        for (int r = 0; r < 2; r++) {
+            const int per_cu = adj_lds_max_blocks(L.nr, L.dyn, r == 1, L.lds[r]);
+            if (per_cu <= 0) return fail(ctx, CS_E_RANGE, "adjoint kernels do not fit on a CU");
+            nblk[k][r] = (int)std::min<int64_t>(L.n_inst, (int64_t)per_cu * std::max(ctx->n_cu, 1));
+        }
         void* d_seg;
-        if ((rc = dalloc(&d_seg, sizeof(double) * (size_t)nblk[k] * K * ck_n))) return rc;
+        if ((rc = dalloc(&d_seg, sizeof(double) * (size_t)nblk[k][1] * K * ck_n))) return rc;
         AdjLdsArgs& a = args[k];
         a.f = L.args;
         a.t_log = (double*)d_tl;
@@ -2497,8 +2505,8 @@ int cs_adjoint_batch(cs_ctx* ctx, int32_t n_inst, const int32_t* inst_cid, const
     for (size_t k = 0; k < ns; k++) HIPCHK(ctx, hipStreamWaitEvent(ctx->side[k], B->ev0, 0));
     for (size_t k = 0; k < ncls; k++) {
         const LdsClass& L = B->classes[k];
-        HIPCHK(ctx, launch_adj_lds(L.nr, L.dyn, false, da + k, nblk[k], L.lds, ctx->side[k % ns]));
-        HIPCHK(ctx, launch_adj_lds(L.nr, L.dyn, true, da + k, nblk[k], L.lds, ctx->side[k % ns]));
+        for (int r = 0; r < 2; r++)
+            HIPCHK(ctx, launch_adj_lds(L.nr, L.dyn, r == 1, da + k, nblk[k][r], L.lds[r], ctx->side[k % ns]));
     }
     for (size_t k = 0; k < ns; k++) {
         HIPCHK(ctx, hipEventRecord(B->class_ev[k], ctx->side[k]));

@@ -242,9 +242,9 @@ hipError_t launch_lds_probe(int nr, const CPlan* cp, const DPlan* P, const doubl
                             const double* qx_piv, double a0, double t, int mode, double* f_asm,
                             double* res_piv, double* f_lu, double* dx_piv, size_t lds, hipStream_t s);
 
-// LDS-resident adjoint: resident workgroups per CU (min over both kernels),
-// launch of the recording forward or the reverse kernel
-int adj_lds_max_blocks(int nr, bool dyn, size_t lds);
+// LDS-resident adjoint: the recording forward or the reverse kernel's resident
+// workgroups per CU, and its launch
+int adj_lds_max_blocks(int nr, bool dyn, bool reverse, size_t lds);
 hipError_t launch_adj_lds(int nr, bool dyn, bool reverse, const AdjLdsArgs* d_args, int nblocks, size_t lds,
                           hipStream_t s);
 

@@ -146,3 +146,40 @@ def test_adjoint_config_51_stage_full_span(engine):
             np.testing.assert_allclose(res.grads[i], g_or, rtol=1e-6, atol=1e-6 * np.max(np.abs(g_or)))
         else:
             assert res.grads[i][k] == pytest.approx(r, rel=1e-5), (i, k)
+
+
+@pytest.mark.parametrize("n", [201, 215, 217, 225, 251])
+def test_adjoint_around_64k_of_lds(engine, n):
+    """Rings whose reverse kernel needs 61 to 76 KB of LDS, on both sides of
+    64 KiB (between 215 and 217 stages), two of them beside a small one:
+    energy and gradients against the oracle's adjoint on the GPU's steps."""
+    _say(f"adjoint {n}-stage ring, 2 ps")
+    flats, params, u0s = _batch([n, 5, n], seed=n)
+    kw = dict(t_start=0.0, t_stop=2e-12, reltol=1e-6, abstol=1e-9, newton_tol=NTOL, newton_maxit=30, init=1)
+    res = ch.adjoint_batch(flats, params, u0s, ch.TranOptions(max_steps=2000, **kw), vsrc=0, ckpt_every=16,
+                           keep_logs=True, max_steps=1000, engine=engine)
+    assert all(r == "Success" for r in res.retcodes), res.retcodes
+    for i, f in enumerate(flats):
+        E_or, g_or, rc = O.adjoint_replay(f, params[i], u0s[i], res.t_logs[i], res.npts_logs[i], 0, **kw)
+        assert rc == 0
+        assert res.energy[i] == pytest.approx(E_or, rel=1e-9)
+        np.testing.assert_allclose(res.grads[i], g_or, rtol=1e-6, atol=1e-6 * np.max(np.abs(g_or)))
+
+
+def test_adjoint_forward_residency(engine):
+    """185-stage rings: three instances of the forward kernel fit a CU's LDS and
+    two of the reverse kernel, so 768 of them take one round forward and two
+    back; with both kernels at the reverse's size they took twice the time of
+    512 (one round each way)."""
+    _say("adjoint residency, 185-stage rings")
+    flat = ch.lower(ring_oscillator(185))
+    p, u0 = flat.params(), ring_initial_state(flat, np.random.default_rng(2))
+    o = ch.TranOptions(t_stop=2e-12, init=1)
+    ms = {}
+    for count in (512, 768):
+        for _ in range(2):
+            r = ch.adjoint_batch([flat] * count, [p] * count, [u0] * count, o, max_steps=1000, engine=engine)
+        assert set(r.retcodes) == {"Success"}
+        ms[count] = r.kernel_ms
+    _say(f"kernel ms {ms}")
+    assert ms[768] <= 1.75 * ms[512]
