@@ -51,16 +51,17 @@ constexpr int W = 64;
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & (W - 1)); }
 
 // 1/a: the hardware estimate and two Newton corrections (error below one
-// ulp); where they are not defined (a infinite, 0 or subnormal with an infinite
-// estimate) the estimate stands: 0 or an infinity, as a division gives.
+// ulp), which an infinite or zero a turns into NaN; the fix-up instruction of
+// the division gives 0 or an infinity there.  It lies on the chain of every
+// pivot, so it is one instruction: a select on the result or on the first
+// residual cost a 33-stage ring's transient 1.4 and 1.9 %, this 0.4.
 __device__ __forceinline__ double recip(double a) {
-    const double r0 = __builtin_amdgcn_rcp(a);
-    double r = r0;
+    double r = __builtin_amdgcn_rcp(a);
     double e = __builtin_fma(-a, r, 1.0);
     r = __builtin_fma(r, e, r);
     e = __builtin_fma(-a, r, 1.0);
     r = __builtin_fma(r, e, r);
-    return r == r ? r : r0;
+    return __builtin_amdgcn_div_fixup(r, a, 1.0);
 }
 
 // a / b for step control: the quotient by recip, corrected once by its
