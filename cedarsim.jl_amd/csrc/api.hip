@@ -1096,7 +1096,7 @@ static int tran_plain(cs_ctx* ctx, int32_t cid, const double* p, const double* u
         double h = sd.dt_init;
         int kout = 0;
         if (wave)
-            while (kout < o->n_out && o->t_start + kout * o->dt_out <= o->t_start + 1e-9 * o->dt_out) {
+            while (kout < o->n_out && out_due(out_time(o->t_start, kout, o->dt_out), o->t_start, o->dt_out)) {
                 for (int s2 = 0; s2 < n_probe; s2++) wave[(size_t)kout * n_probe + s2] = U[P.probe[s2]];
                 if (sr)
                     std::copy(sr->S.begin(), sr->S.begin() + (size_t)sr->n_sp * n_probe,
@@ -1192,8 +1192,8 @@ static int tran_plain(cs_ctx* ctx, int32_t cid, const double* p, const double* u
             st.steps++;
             if (wave) {
                 while (kout < o->n_out) {
-                    const double tq = o->t_start + kout * o->dt_out;
-                    if (tq > tn + 1e-9 * o->dt_out) break;
+                    const double tq = out_time(o->t_start, kout, o->dt_out);
+                    if (!out_due(tq, tn, o->dt_out)) break;
                     double l0, l1, l2 = 0.0;
                     if (npts >= 3) {
                         l0 = (tq - T1) * (tq - T2) / ((T0 - T1) * (T0 - T2));
@@ -1266,6 +1266,16 @@ static void single_trim(Circuit& C) {
     (void)hipHostFree(C.h_sbuf);
     C.sbuf = C.h_sbuf = nullptr;
     C.sbuf_bytes = 0;
+}
+
+// The samples a run on one launch has written: those up to the time it
+// reached; one that stops early leaves the others.
+static int32_t samples_written(const cs_tran_opts& o, int32_t n_out, const cs_tran_stats& st) {
+    if (n_out <= 0 || st.retcode == CS_E_NOCONV) return 0;
+    const double est = (st.t_end - o.t_start) / o.dt_out;   // off by less than one
+    int32_t rows = est > 2.0 ? (int32_t)std::min(est - 2.0, (double)n_out) : 0;
+    while (rows < n_out && out_due(out_time(o.t_start, rows, o.dt_out), st.t_end, o.dt_out)) rows++;
+    return rows;
 }
 
 static int single_buffers(cs_ctx* ctx, Circuit& C, const cs_tran_opts& o, bool with_u0, int32_t n_out, SingleRun& R) {
@@ -1348,10 +1358,7 @@ static int tran_single(cs_ctx* ctx, Circuit& C, const double* p, const double* u
     HIPCHK(ctx, launch_tran_pack(k, (const LdsArgs*)R.d_args, 1, C.lds_bytes, s));
     HIPCHK(ctx, hipMemcpyAsync(C.h_sbuf + R.down0, C.sbuf + R.down0, R.down, hipMemcpyDeviceToHost, s));
     HIPCHK(ctx, hipStreamSynchronize(s));
-    // the samples up to the time reached; a run that stops early leaves the others
-    int32_t rows = 0;
-    if (R.st->retcode != CS_E_NOCONV)
-        while (rows < n_out && o->t_start + rows * o->dt_out <= R.st->t_end + 1e-9 * o->dt_out) rows++;
+    const int32_t rows = samples_written(*o, n_out, *R.st);
     if (rows) std::memcpy(wave, R.wave, sizeof(double) * (size_t)rows * P.probe.size());
     if (u_final) std::memcpy(u_final, R.u, sizeof(double) * P.n);
     R.st->busy_s /= ctx->clock_hz;
@@ -1489,10 +1496,7 @@ static int sens_single(cs_ctx* ctx, Circuit& C, const double* p, const double* u
     rc = run();
     (void)hipFree(d);
     if (rc) return rc;
-    // the samples up to the time reached; a run that stops early leaves the others
-    int32_t rows = 0;
-    if (a.wave && st.retcode != CS_E_NOCONV)
-        while (rows < n_out && o->t_start + rows * o->dt_out <= st.t_end + 1e-9 * o->dt_out) rows++;
+    const int32_t rows = a.wave ? samples_written(*o, n_out, st) : 0;
     if (rows) {
         std::memcpy(wave, hw.data(), sizeof(double) * (size_t)rows * np);
         std::memcpy(sens, hs.data(), sizeof(double) * (size_t)rows * blk);

@@ -87,6 +87,65 @@ __device__ __forceinline__ double block_reduce(double v, double* red, Op op) {
     }
 }
 
+// The output samples due at an accepted point tn, by one wavefront: up to 64
+// of them at a time, their interpolation weights one sample per lane, then
+// put(kout, m, l0, l1, l2) for samples kout .. kout + m - 1.
+template <class Weights, class Put>
+__device__ __forceinline__ void put_samples(int& kout, double t_start, double dt_out, int n_out, double tn,
+                                            Weights weights, Put put) {
+    while (kout < n_out && out_due(out_time(t_start, kout, dt_out), tn, dt_out)) {
+        const int lane = (int)(threadIdx.x & 63);
+        const double tq = out_time(t_start, kout + (lane < n_out - kout ? lane : 0), dt_out);
+        const int m = __popcll(__ballot(lane < n_out - kout && out_due(tq, tn, dt_out)));
+        double l0, l1, l2;
+        weights(tq, l0, l1, l2);
+        put(kout, m, l0, l1, l2);
+        kout += m;
+    }
+}
+
+// The put of rows held by the lanes: row r of a lane has the values U0, U1, U2
+// at the last three points and goes to place ps[r] of a sample (-1: none).
+// Few samples: one after the other, lanes over the rows.  More samples than
+// rows (a fine grid): the rows one after the other, lanes over the samples.
+// Written one by one a sample cost a whole pass of the wavefront, 225 ns:
+// cs_tran of an inverter (five rows, 1 ns, 786,000 samples) took 169 ms, of
+// which the run itself is 5; now 18.5, and six sensitivities of it at
+// 1,000,001 samples 557 ms, now 124.
+template <int NR>
+__device__ __forceinline__ void put_rows(double* out, size_t stride, int kout, int m, double l0, double l1, double l2,
+                                         const int32_t (&ps)[NR], const double (&U0)[NR], const double (&U1)[NR],
+                                         const double (&U2)[NR]) {
+    const int lane = (int)(threadIdx.x & 63);
+    int rows = 0;
+#pragma unroll
+    for (int r = 0; r < NR; r++) rows += __popcll(__ballot(ps[r] >= 0));
+    double* const at = out + (size_t)kout * stride;
+    if (m <= rows) {
+#pragma nounroll
+        for (int j = 0; j < m; j++) {
+            const double a = readlane_f64(l0, j), b = readlane_f64(l1, j), c = readlane_f64(l2, j);
+#pragma unroll
+            for (int r = 0; r < NR; r++)
+                if (ps[r] >= 0)
+                    at[j * stride + ps[r]] = __builtin_fma(a, U0[r], __builtin_fma(b, U1[r], c * U2[r]));
+        }
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        unsigned long long todo = __ballot(ps[r] >= 0);
+#pragma nounroll
+        while (todo) {
+            const int j = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            const int p = __builtin_amdgcn_readlane(ps[r], j);
+            const double a = readlane_f64(U0[r], j), b = readlane_f64(U1[r], j), c = readlane_f64(U2[r], j);
+            if (lane < m) at[lane * stride + p] = __builtin_fma(l0, a, __builtin_fma(l1, b, l2 * c));
+        }
+    }
+}
+
 // Per-instance linear stamp values -> Glin, Clin in F positions.
 template <int NT>
 __device__ void dev_lin_setup(const DPlan* __restrict__ P, const double* __restrict__ p,

@@ -1100,14 +1100,20 @@ __device__ __forceinline__ void run_lds(Rec& rec, Hdr c, ConstPtr<LdsArgs> A, co
         double* const wave = A->wave ? A->wave + A->w_off[inst] : nullptr;
         int kout = 0;
         const int n_probe = P->n_probe;
-        int32_t ps[NR];
+        // a row's place in a sample, read where samples are written: kept, it
+        // would hold registers across the transient
+        auto places = [&](int32_t (&ps)[NR]) {
+            c = fresh(c);
 #pragma unroll
-        for (int r = 0; r < NR; r++) {
-            const int k = tid + W * r;
-            ps[r] = (wave && k < n) ? c->probe[k] : -1;
-        }
+            for (int r = 0; r < NR; r++) {
+                const int k = lane_id() + W * r;
+                ps[r] = k < c->n ? c->probe[k] : -1;
+            }
+        };
         if (wave) {
-            while (kout < A->o.n_out && t_start + kout * A->o.dt_out <= t_start + 1e-9 * A->o.dt_out) {
+            int32_t ps[NR];
+            places(ps);
+            while (kout < A->o.n_out && out_due(out_time(t_start, kout, A->o.dt_out), t_start, A->o.dt_out)) {
 #pragma unroll
                 for (int r = 0; r < NR; r++)
                     if (ps[r] >= 0) wave[(size_t)kout * n_probe + ps[r]] = Uh0[r];
@@ -1222,19 +1228,16 @@ __device__ __forceinline__ void run_lds(Rec& rec, Hdr c, ConstPtr<LdsArgs> A, co
             T2 = T1; T1 = T0; T0 = tn;
             if (npts < 3) npts++;
             steps++;
-            if (wave) {
-                while (kout < A->o.n_out) {
-                    const double tq = t_start + kout * A->o.dt_out;
-                    if (tq > tn + 1e-9 * A->o.dt_out) break;
-                    double l0, l1, l2;
-                    step_pred(npts, tq, T0, T1, T2, l0, l1, l2);
-#pragma unroll
-                    for (int r = 0; r < NR; r++)
-                        if (ps[r] >= 0)
-                            wave[(size_t)kout * n_probe + ps[r]] = __builtin_fma(l0, Uh0[r], __builtin_fma(l1, Uh1[r], l2 * Uh2[r]));
-                    kout++;
-                }
-            }
+            if (wave)
+                put_samples(kout, A->o.t_start, A->o.dt_out, A->o.n_out, tn,
+                            [&](double tq, double& l0, double& l1, double& l2) {
+                                step_pred(npts, tq, T0, T1, T2, l0, l1, l2);
+                            },
+                            [&](int k0, int m, double l0, double l1, double l2) {
+                                int32_t ps[NR];
+                                places(ps);
+                                put_rows<NR>(wave, n_probe, k0, m, l0, l1, l2, ps, Uh0, Uh1, Uh2);
+                            });
             t = tn;
             h = hh * fac;
             if (hit && srcbp) {

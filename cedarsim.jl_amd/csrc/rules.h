@@ -235,6 +235,17 @@ CEDAR_HD double clip_step(double t, double& hh, double tb, int& hit) {
     return tn;
 }
 
+// Output sample k lies at out_time and is due once the run has reached t.
+// Never fused: the host counts with them the samples that a kernel has written.
+CEDAR_HD double out_time(double t_start, int k, double dt_out) {
+#pragma clang fp contract(off)
+    return t_start + k * dt_out;
+}
+CEDAR_HD bool out_due(double tq, double t, double dt_out) {
+#pragma clang fp contract(off)
+    return tq <= t + 1e-9 * dt_out;
+}
+
 // step factor after an LTE test with error err (in tolerance units)
 CEDAR_HD double reject_factor(double err, int k) {
     double f = (err == err) ? 0.9 * pow(err, -1.0 / (double)(k + 1)) : 0.1;

@@ -140,7 +140,9 @@ __global__ __launch_bounds__(kSensThreads) void k_sens(SensArgs A) {
 // k_sens's solves at the DC point, at the initial point and at each accepted
 // step, on the instance's own LU in LDS.  Lane i holds unknown i's
 // sensitivity at the last three points.
+template <bool FineGrid>
 struct SensRec {
+    static constexpr bool kFineGrid = FineGrid;
     const SensRunArgs& A;
     const int j;
     double *sn, *d1, *d2;          // LDS: s at the new point; charge sensitivities one and two steps back
@@ -203,6 +205,10 @@ struct SensRec {
         const int sl = i < P->n ? P->probe_slot[i] : -1;
         if (sl >= 0) A.sens[((size_t)kout * A.n_sp + j) * A.n_probe + sl] = l0 * s0 + l1 * s1 + l2 * s2;
     }
+    __device__ void on_outputs(const int32_t (&ps)[1], int kout, int m, double l0, double l1, double l2) {
+        const double a[1] = {s0}, b[1] = {s1}, c[1] = {s2};
+        put_rows<1>(A.sens + (size_t)j * A.n_probe, (size_t)A.n_sp * A.n_probe, kout, m, l0, l1, l2, ps, a, b, c);
+    }
 };
 
 // One wavefront per parameter, each running the whole transient with its own
@@ -212,6 +218,7 @@ struct SensRec {
 // parameter costs nothing, while host step control cost a graph launch and a
 // round trip per Newton iteration and another of each per accepted step.
 // An inverter over 1 ns with six parameters: 82.5 -> 12.9 ms.
+template <bool FineGrid>
 __global__ __launch_bounds__(NT) void k_tran_sens(SensRunArgs A) {
     extern __shared__ double lds[];
     const int j = blockIdx.x;
@@ -224,7 +231,7 @@ __global__ __launch_bounds__(NT) void k_tran_sens(SensRunArgs A) {
     L.qx = L.x + A.n;
     L.st = L.qx + A.n;
     double* sn = L.st + A.n_stamp;
-    SensRec rec{A, j, sn, sn + A.n, sn + 2 * A.n};
+    SensRec<FineGrid> rec{A, j, sn, sn + A.n, sn + 2 * A.n};
     if ((int)threadIdx.x < A.n) rec.d1[threadIdx.x] = rec.d2[threadIdx.x] = 0.0;
     double* lin = A.ws + (size_t)j * A.ws_stride;
     run_instance<1>(rec, A.P, A.p, A.u0, A.wave, A.u_final, A.stats, A.o, L, lin + A.n_lin,
@@ -238,7 +245,11 @@ size_t tran_sens_lds(int32_t n, int32_t nnz, int32_t n_stamp) {
 }
 
 hipError_t launch_tran_sens(const SensRunArgs& a, hipStream_t s) {
-    hipLaunchKernelGGL(k_tran_sens, dim3(a.n_sp), dim3(NT), tran_sens_lds(a.n, a.nnz, a.n_stamp), s, a);
+    // 0.45 us a sample written one by one, 4 % of a run for the other form: an
+    // inverter's 13 ms, so the line lies where they cost the same
+    const size_t lds = tran_sens_lds(a.n, a.nnz, a.n_stamp);
+    if (a.o.n_out > 1024) hipLaunchKernelGGL(k_tran_sens<true>, dim3(a.n_sp), dim3(NT), lds, s, a);
+    else hipLaunchKernelGGL(k_tran_sens<false>, dim3(a.n_sp), dim3(NT), lds, s, a);
     return hipGetLastError();
 }
 

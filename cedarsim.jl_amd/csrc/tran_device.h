@@ -7,6 +7,8 @@
 // Rec is called at the points a forward sensitivity run needs (sens.hip): the
 // DC point and the initial point, each with its Jacobian just assembled in
 // L.F, every accepted step, and every output sample; the batch passes NoRec.
+// Rec::kFineGrid writes the samples of a step together (put_samples), for
+// output grids finer than the steps; it costs the run 4 % in registers.
 #pragma once
 #include "dcop_rules.h"
 #include "device.h"
@@ -21,6 +23,7 @@ struct Lds {
 };
 
 struct NoRec {
+    static constexpr bool kFineGrid = false;
     __device__ __forceinline__ void on_dc(const DPlan*, const double*, const Lds&, const double*) {}
     __device__ __forceinline__ void on_initial(const DPlan*, const double*, const Lds&, const double*, bool) {}
     __device__ __forceinline__ void on_step(const DPlan*, const double*, const Lds&, const double*, const double*,
@@ -142,7 +145,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
         int kout = 0;
         const int n_probe = P->n_probe;
         if (wave) {
-            while (kout < o.n_out && o.t_start + kout * o.dt_out <= o.t_start + 1e-9 * o.dt_out) {
+            while (kout < o.n_out && out_due(out_time(o.t_start, kout, o.dt_out), o.t_start, o.dt_out)) {
 #pragma unroll
                 for (int r = 0; r < NR; r++) {
                     const int i = tid + NT * r;
@@ -262,20 +265,35 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
             T2 = T1; T1 = T0; T0 = tn;
             if (npts < 3) npts++;
             steps++;
-            if (wave) {
+            auto weights = [&](double tq, double& l0, double& l1, double& l2) {
+                l2 = 0.0;
+                if (npts >= 3) {
+                    l0 = (tq - T1) * (tq - T2) / ((T0 - T1) * (T0 - T2));
+                    l1 = (tq - T0) * (tq - T2) / ((T1 - T0) * (T1 - T2));
+                    l2 = (tq - T0) * (tq - T1) / ((T2 - T0) * (T2 - T1));
+                } else {
+                    const double s = (tq - T1) / (T0 - T1);
+                    l0 = s;
+                    l1 = 1.0 - s;
+                }
+            };
+            if constexpr (Rec::kFineGrid) {
+                if (wave)
+                    put_samples(kout, o.t_start, o.dt_out, o.n_out, tn, weights,
+                                [&](int k0, int m, double l0, double l1, double l2) {
+                                    int32_t ps[NR];
+#pragma unroll
+                                    for (int r = 0; r < NR; r++)
+                                        ps[r] = tid + NT * r < n ? P->probe_slot[tid + NT * r] : -1;
+                                    put_rows<NR>(wave, n_probe, k0, m, l0, l1, l2, ps, Uh0, Uh1, Uh2);
+                                    rec.on_outputs(ps, k0, m, l0, l1, l2);
+                                });
+            } else if (wave) {
                 while (kout < o.n_out) {
-                    const double tq = o.t_start + kout * o.dt_out;
-                    if (tq > tn + 1e-9 * o.dt_out) break;
-                    double l0, l1, l2 = 0.0;
-                    if (npts >= 3) {
-                        l0 = (tq - T1) * (tq - T2) / ((T0 - T1) * (T0 - T2));
-                        l1 = (tq - T0) * (tq - T2) / ((T1 - T0) * (T1 - T2));
-                        l2 = (tq - T0) * (tq - T1) / ((T2 - T0) * (T2 - T1));
-                    } else {
-                        const double s = (tq - T1) / (T0 - T1);
-                        l0 = s;
-                        l1 = 1.0 - s;
-                    }
+                    const double tq = out_time(o.t_start, kout, o.dt_out);
+                    if (!out_due(tq, tn, o.dt_out)) break;
+                    double l0, l1, l2;
+                    weights(tq, l0, l1, l2);
 #pragma unroll
                     for (int r = 0; r < NR; r++) {
                         const int i = tid + NT * r;

@@ -222,3 +222,60 @@ def test_lds_bound_batch_is_resident_at_once(engine, n, count):
         b.close()
     assert set(r.retcodes) == {"Success"}
     assert ms <= 1.4e3 * max(st.busy_s for st in r.stats)
+
+
+@pytest.mark.parametrize("name,n_out,probes", [
+    ("inverter", 2, None), ("inverter", 65, None), ("inverter", 5001, None), ("inverter", 20001, ["out"]),
+    ("inverter", 3001, ["out", "VIN.I", "in"]), ("ring67", 4001, None), ("ring67", 30001, ["s66", "vdd", "s3", "s64"]),
+    ("ring149", 3001, ["s148", "s0", "s70"])])
+def test_fine_output_grids(engine, name, n_out, probes):
+    """Output grids finer than the steps: up to hundreds of samples are due at
+    one accepted point, written 64 at a time, lanes over the samples where
+    more are due than rows are probed and over the rows otherwise.  cs_tran
+    (AUTO and GLOBAL) and batches on both kernels against the oracle."""
+    print(f"[gpu] fine grid {name} {n_out} {probes}", flush=True)
+    rng = np.random.default_rng(n_out)
+    u0 = None
+    if name == "inverter":
+        flat, span = ch.lower(inverter()), 0.3e-9
+    else:
+        flat, span = ch.lower(ring_oscillator(int(name[4:]))), 2e-12
+        u0 = ring_initial_state(flat, rng)
+    kw = {"init": L.INIT_UIC} if u0 is not None else {}
+    p = flat.params()
+    w, _, st, rc = O.tran(flat, p, u0, ch.grid_options((0.0, span), n_out=n_out, **kw))
+    assert rc == 0
+    s = engine.load(flat, solver=L.SOLVER_LEVEL)
+    if probes:
+        s.set_probes(probes)
+        w = w[:, s.probes]
+    runs = []
+    for kern in (L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_GLOBAL, L.BATCH_KERNEL_LDS):
+        o = ch.grid_options((0.0, span), n_out=n_out, batch_kernel=kern, **kw)
+        r = s.tran(o, p, u0)
+        assert r.retcode == "Success" and r.stats.steps == st.steps
+        runs.append(r.wave)
+        if kern != L.BATCH_KERNEL_AUTO:
+            b = ch.Batch(engine, [s], [0, 0], [p, p], o, None if u0 is None else [u0, u0])
+            try:
+                b.run()
+                runs += b.results().wave
+            finally:
+                b.close()
+    for x in runs:
+        assert np.all(np.abs(x - w) <= 1e-6 * np.abs(w) + 1e-9)
+
+
+def test_samples_cost_less_than_the_run(engine):
+    """200,001 samples of an inverter's run do not double its time on the
+    device (one after the other they took ten times the run)."""
+    print("[gpu] cost of samples", flush=True)
+    s = engine.load(ch.lower(inverter()))
+    busy = {}
+    for n_out in (21, 200_001):
+        for _ in range(2):
+            r = s.tran(ch.grid_options((0.0, 1e-9), n_out=n_out, batch_kernel=L.BATCH_KERNEL_LDS))
+        assert r.retcode == "Success"
+        busy[n_out] = r.stats.busy_s
+    print(f"[gpu] busy {busy}", flush=True)
+    assert busy[200_001] <= 2.0 * busy[21]

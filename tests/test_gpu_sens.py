@@ -164,3 +164,23 @@ def test_one_launch_matches_host_step_control(engine, case):
         a, b = ga[:, j], gg[:, j]
         _say(f"{case} {names[j]}: max |s| {np.max(np.abs(b)):.3e}, difference {np.max(np.abs(a - b)):.2e}")
         assert np.all(np.abs(a - b) <= 1e-6 * np.abs(b) + 1e-9 * np.max(np.abs(b)) + 1e-300), names[j]
+
+
+@pytest.mark.parametrize("n_out,probes", [(65, None), (3001, None), (20001, ["out"])])
+def test_one_launch_fine_output_grid(engine, n_out, probes):
+    """More samples due at a step than unknowns are probed: the one launch
+    writes them lanes over the samples; waveform and sensitivities as with
+    host step control (the bars of test_one_launch_matches_host_step_control)."""
+    flat = ch.lower(inverter())
+    names = ["MN.vth", "MP.w", "CL"]
+    sys_ = engine.load(flat)
+    if probes:
+        sys_.set_probes(probes)
+    run = [sys_.tran_sens(ch.grid_options((0.0, 0.3e-9), n_out=n_out, batch_kernel=k), names)
+           for k in (L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_GLOBAL)]
+    (ra, ga), (rg, gg) = run
+    assert ra.retcode == rg.retcode == "Success" and ra.stats.steps == rg.stats.steps
+    assert np.all(np.abs(ra.wave - rg.wave) <= 1e-6 * np.abs(rg.wave) + 1e-9)
+    for j in range(len(names)):
+        a, b = ga[:, j], gg[:, j]
+        assert np.all(np.abs(a - b) <= 1e-6 * np.abs(b) + 1e-9 * np.max(np.abs(b)) + 1e-300), names[j]
