@@ -15,6 +15,7 @@
 #include <cstdio>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <numeric>
 #include <string>
 #include <vector>
@@ -52,15 +53,11 @@ struct Circuit {
     CPlan hcp{};                // device pointers, host copy
     void* cbuf = nullptr;
     const CPlan* d_cplan = nullptr;
-    // one instance on the LDS-resident kernel (cs_tran, cs_dcop): a device
-    // buffer and its pinned image, kept and grown from call to call
+    // one instance on the LDS-resident kernel (cs_tran, cs_dcop)
     int32_t lds_nr = 0;         // rows per lane, 0: does not fit
     std::string lds_why;
     bool lds_dyn = false;
     size_t lds_bytes = 0;
-    char* sbuf = nullptr;
-    char* h_sbuf = nullptr;
-    size_t sbuf_bytes = 0;
     // large circuits: the supernodal path (big.h) instead of all of the above
     BigCircuit* big = nullptr;
 };
@@ -118,6 +115,12 @@ struct cs_ctx {
     std::string err;
     std::vector<std::unique_ptr<Circuit>> circuits;
     std::vector<std::unique_ptr<Batch>> batches;
+    // one-launch runs of single circuits: a device buffer and a pinned image of
+    // its start, kept and grown from call to call; a call holds single_mu
+    std::mutex single_mu;
+    char* sbuf = nullptr;
+    char* h_sbuf = nullptr;
+    size_t sbuf_bytes = 0, h_sbuf_bytes = 0;
 };
 
 namespace {
@@ -495,10 +498,10 @@ int cs_destroy(cs_ctx* ctx) {
             if (c->h_norm) (void)hipHostFree(c->h_norm);
             if (c->h_stage) (void)hipHostFree(c->h_stage);
             if (c->cbuf) (void)hipFree(c->cbuf);
-            if (c->sbuf) (void)hipFree(c->sbuf);
-            if (c->h_sbuf) (void)hipHostFree(c->h_sbuf);
             if (c->big) big_destroy(c->big);
         }
+    if (ctx->sbuf) (void)hipFree(ctx->sbuf);
+    if (ctx->h_sbuf) (void)hipHostFree(ctx->h_sbuf);
     for (hipStream_t st : ctx->side) (void)hipStreamDestroy(st);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -1243,29 +1246,33 @@ static int tran_plain(cs_ctx* ctx, int32_t cid, const double* p, const double* u
 
 // ---- one instance on the LDS-resident kernel ------------------------------------------
 // The whole analysis in one launch, where the plain path takes a graph launch
-// and a host round trip per Newton iteration.  The circuit keeps the device
-// buffer and its pinned image: one copy up (arguments, parameters, initial
-// state), the kernel, one copy down (stats, final state, waveform).
+// and a host round trip per Newton iteration.  The context keeps a device
+// buffer and a pinned image of its start: one copy up (arguments, parameters,
+// initial state), the kernel, one copy down (stats, final state and samples
+// of up to kSinglePin bytes).  More samples go straight to the caller's array,
+// as far as the run came: an inverter's run with 100 MiB of them took 88 ms
+// through a pinned image of their size, 51 so, and the context pins no more
+// than the 1 MiB.
 struct SingleRun {
     LdsArgs* args;          // in the pinned image
     double *p, *u0;
     cs_tran_stats* st;      // results, in the pinned image
-    double *u, *wave;
-    char* d_args;
-    size_t up, down0, down; // bytes to copy up; the results' range
+    double *u, *wave;       // (wave null: the samples stay on the device)
+    char *d_args, *d_st;
+    double* d_wave;
+    size_t up, down;        // bytes to copy up; bytes of results to copy down
 };
 
-// The device buffer and its pinned image outlive the call up to kSingleKeep
-// bytes; a run whose samples need more than kSingleMax stays on the plain
-// path, which writes them straight to the caller's array.
-constexpr size_t kSingleKeep = (size_t)64 << 20, kSingleMax = (size_t)1 << 30;
+// The buffers outlive the call up to kSingleKeep bytes; a run whose samples
+// need more than kSingleMax stays on the plain path, which writes them
+// straight to the caller's array.
+constexpr size_t kSinglePin = (size_t)1 << 20, kSingleKeep = (size_t)64 << 20, kSingleMax = (size_t)1 << 30;
 
-static void single_trim(Circuit& C) {
-    if (C.sbuf_bytes <= kSingleKeep) return;
-    (void)hipFree(C.sbuf);
-    (void)hipHostFree(C.h_sbuf);
-    C.sbuf = C.h_sbuf = nullptr;
-    C.sbuf_bytes = 0;
+static void single_free(cs_ctx* ctx) {
+    if (ctx->sbuf) (void)hipFree(ctx->sbuf);
+    if (ctx->h_sbuf) (void)hipHostFree(ctx->h_sbuf);
+    ctx->sbuf = ctx->h_sbuf = nullptr;
+    ctx->sbuf_bytes = ctx->h_sbuf_bytes = 0;
 }
 
 // The samples a run on one launch has written: those up to the time it
@@ -1286,20 +1293,21 @@ static int single_buffers(cs_ctx* ctx, Circuit& C, const cs_tran_opts& o, bool w
     const size_t o_args = take(sizeof(LdsArgs)), o_z = take(64), o_segs = take(2 * sizeof(int4)),
                  o_p = take(sizeof(double) * P.lay.n_params), o_u0 = take(sizeof(double) * P.n);
     R.up = at;
-    const size_t o_st = take(sizeof(cs_tran_stats)), o_u = take(sizeof(double) * P.n), o_w = take(sizeof(double) * n_wave);
-    R.down0 = o_st;
-    R.down = at - o_st;
-    if (at > C.sbuf_bytes) {
-        if (C.sbuf) (void)hipFree(C.sbuf);
-        if (C.h_sbuf) (void)hipHostFree(C.h_sbuf);
-        C.sbuf = C.h_sbuf = nullptr;
-        C.sbuf_bytes = 0;
-        const size_t bytes = at + at / 4;
-        HIPCHK(ctx, hipMalloc((void**)&C.sbuf, bytes));
-        HIPCHK(ctx, hipHostMalloc((void**)&C.h_sbuf, bytes, hipHostMallocDefault));
-        C.sbuf_bytes = bytes;
+    const size_t o_st = take(sizeof(cs_tran_stats)), o_u = take(sizeof(double) * P.n);
+    size_t pinned = at;
+    const size_t o_w = take(sizeof(double) * n_wave);
+    const bool pin_wave = sizeof(double) * n_wave <= kSinglePin;
+    if (pin_wave) pinned = at;
+    R.down = pinned - o_st;
+    if (at > ctx->sbuf_bytes || pinned > ctx->h_sbuf_bytes) {
+        single_free(ctx);
+        const size_t bytes = at + at / 4, h_bytes = pinned + pinned / 4;
+        HIPCHK(ctx, hipMalloc((void**)&ctx->sbuf, bytes));
+        ctx->sbuf_bytes = bytes;
+        HIPCHK(ctx, hipHostMalloc((void**)&ctx->h_sbuf, h_bytes, hipHostMallocDefault));
+        ctx->h_sbuf_bytes = h_bytes;
     }
-    char *h = C.h_sbuf, *d = C.sbuf;
+    char *h = ctx->h_sbuf, *d = ctx->sbuf;
     std::memset(h, 0, o_p);
     // zeros at o_z: offsets, instance and circuit numbers; then the queue, and
     // the chunk's segment range (0, 1)
@@ -1313,8 +1321,10 @@ static int single_buffers(cs_ctx* ctx, Circuit& C, const cs_tran_opts& o, bool w
     R.u0 = (double*)(h + o_u0);
     R.st = (cs_tran_stats*)(h + o_st);
     R.u = (double*)(h + o_u);
-    R.wave = (double*)(h + o_w);
+    R.wave = pin_wave ? (double*)(h + o_w) : nullptr;
     R.d_args = d + o_args;
+    R.d_st = d + o_st;
+    R.d_wave = (double*)(d + o_w);
     LdsArgs& a = *R.args;
     a.cplans = C.d_cplan;
     a.plans = C.d_dplan;
@@ -1322,7 +1332,7 @@ static int single_buffers(cs_ctx* ctx, Circuit& C, const cs_tran_opts& o, bool w
     a.p_off = a.u_off = a.w_off = (const int64_t*)(d + o_z);
     a.params = (const double*)(d + o_p);
     a.u0 = with_u0 ? (const double*)(d + o_u0) : nullptr;
-    a.wave = n_wave ? (double*)(d + o_w) : nullptr;
+    a.wave = n_wave ? R.d_wave : nullptr;
     a.u_final = (double*)(d + o_u);
     a.stats = (cs_tran_stats*)(d + o_st);
     a.order = (const int32_t*)(d + o_z);
@@ -1345,6 +1355,7 @@ static int tran_single(cs_ctx* ctx, Circuit& C, const double* p, const double* u
     if (o->n_out > 0 && !(o->dt_out > 0)) return fail(ctx, CS_E_INVALID, "dt_out must be > 0");
     (void)hipSetDevice(ctx->device);
     const int32_t n_out = wave ? std::max(o->n_out, 0) : 0;
+    std::lock_guard<std::mutex> lock(ctx->single_mu);
     SingleRun R{};
     int rc = single_buffers(ctx, C, *o, u0 != nullptr, n_out, R);
     if (rc) return rc;
@@ -1354,17 +1365,18 @@ static int tran_single(cs_ctx* ctx, Circuit& C, const double* p, const double* u
     PackShape k;
     k.nr = C.lds_nr;
     k.dyn = C.lds_dyn;
-    HIPCHK(ctx, hipMemcpyAsync(C.sbuf, C.h_sbuf, R.up, hipMemcpyHostToDevice, s));
+    HIPCHK(ctx, hipMemcpyAsync(ctx->sbuf, ctx->h_sbuf, R.up, hipMemcpyHostToDevice, s));
     HIPCHK(ctx, launch_tran_pack(k, (const LdsArgs*)R.d_args, 1, C.lds_bytes, s));
-    HIPCHK(ctx, hipMemcpyAsync(C.h_sbuf + R.down0, C.sbuf + R.down0, R.down, hipMemcpyDeviceToHost, s));
+    HIPCHK(ctx, hipMemcpyAsync(R.st, R.d_st, R.down, hipMemcpyDeviceToHost, s));
     HIPCHK(ctx, hipStreamSynchronize(s));
-    const int32_t rows = samples_written(*o, n_out, *R.st);
-    if (rows) std::memcpy(wave, R.wave, sizeof(double) * (size_t)rows * P.probe.size());
+    const size_t got = sizeof(double) * (size_t)samples_written(*o, n_out, *R.st) * P.probe.size();
+    if (got && R.wave) std::memcpy(wave, R.wave, got);
+    else if (got) HIPCHK(ctx, hipMemcpy(wave, R.d_wave, got, hipMemcpyDeviceToHost));
     if (u_final) std::memcpy(u_final, R.u, sizeof(double) * P.n);
     R.st->busy_s /= ctx->clock_hz;
     if (st_out) *st_out = *R.st;
     rc = R.st->retcode;
-    single_trim(C);   // R's pointers end here
+    if (ctx->sbuf_bytes > kSingleKeep) single_free(ctx);   // R's pointers end here
     if (rc == CS_E_DTMIN) ctx->err = "transient: step size fell below dt_min";
     else if (rc == CS_E_NOCONV)
         ctx->err = std::string("transient: initial point did not converge") +
@@ -1377,14 +1389,15 @@ static int tran_single(cs_ctx* ctx, Circuit& C, const double* p, const double* u
 static int dcop_single(cs_ctx* ctx, Circuit& C, const double* p, const cs_tran_opts* o, double* u_out,
                        cs_tran_stats* st) {
     const Plan& P = C.plan;
+    std::lock_guard<std::mutex> lock(ctx->single_mu);
     SingleRun R{};
     int rc = single_buffers(ctx, C, *o, false, 0, R);
     if (rc) return rc;
     std::memcpy(R.p, p, sizeof(double) * P.lay.n_params);
     hipStream_t s = ctx->stream;
-    HIPCHK(ctx, hipMemcpyAsync(C.sbuf, C.h_sbuf, R.up, hipMemcpyHostToDevice, s));
+    HIPCHK(ctx, hipMemcpyAsync(ctx->sbuf, ctx->h_sbuf, R.up, hipMemcpyHostToDevice, s));
     HIPCHK(ctx, launch_lds_dcop(C.lds_nr, C.lds_dyn, (const LdsArgs*)R.d_args, C.lds_bytes, s));
-    HIPCHK(ctx, hipMemcpyAsync(C.h_sbuf + R.down0, C.sbuf + R.down0, R.down, hipMemcpyDeviceToHost, s));
+    HIPCHK(ctx, hipMemcpyAsync(R.st, R.d_st, R.down, hipMemcpyDeviceToHost, s));
     HIPCHK(ctx, hipStreamSynchronize(s));
     std::memcpy(u_out, R.u, sizeof(double) * P.n);
     rc = R.st->retcode;
@@ -1477,7 +1490,7 @@ static int sens_single(cs_ctx* ctx, Circuit& C, const double* p, const double* u
     a.o = *o;
     hipStream_t s = ctx->stream;
     cs_tran_stats st{};
-    std::vector<double> u(n), hw((size_t)n_out * np), hs((size_t)n_out * blk);
+    std::vector<double> u(n);
     auto run = [&]() -> int {
         HIPCHK(ctx, hipMemcpyAsync(d + o_sp, sp.data(), sizeof(SensParam) * n_sp, hipMemcpyHostToDevice, s));
         HIPCHK(ctx, hipMemcpyAsync(d + o_prow, P.prow.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, s));
@@ -1486,21 +1499,17 @@ static int sens_single(cs_ctx* ctx, Circuit& C, const double* p, const double* u
         HIPCHK(ctx, launch_tran_sens(a, s));
         HIPCHK(ctx, hipMemcpyAsync(&st, d + o_st, sizeof(st), hipMemcpyDeviceToHost, s));
         HIPCHK(ctx, hipMemcpyAsync(u.data(), d + o_u, sizeof(double) * n, hipMemcpyDeviceToHost, s));
-        if (a.wave) {
-            HIPCHK(ctx, hipMemcpyAsync(hw.data(), a.wave, sizeof(double) * hw.size(), hipMemcpyDeviceToHost, s));
-            HIPCHK(ctx, hipMemcpyAsync(hs.data(), a.sens, sizeof(double) * hs.size(), hipMemcpyDeviceToHost, s));
-        }
         HIPCHK(ctx, hipStreamSynchronize(s));
+        const size_t rows = a.wave ? samples_written(*o, n_out, st) : 0;
+        if (rows) {
+            HIPCHK(ctx, hipMemcpy(wave, a.wave, sizeof(double) * rows * np, hipMemcpyDeviceToHost));
+            HIPCHK(ctx, hipMemcpy(sens, a.sens, sizeof(double) * rows * blk, hipMemcpyDeviceToHost));
+        }
         return CS_OK;
     };
     rc = run();
     (void)hipFree(d);
     if (rc) return rc;
-    const int32_t rows = a.wave ? samples_written(*o, n_out, st) : 0;
-    if (rows) {
-        std::memcpy(wave, hw.data(), sizeof(double) * (size_t)rows * np);
-        std::memcpy(sens, hs.data(), sizeof(double) * (size_t)rows * blk);
-    }
     if (u_final) std::memcpy(u_final, u.data(), sizeof(double) * n);
     st.busy_s = 0.0;
     if (st_out) *st_out = st;

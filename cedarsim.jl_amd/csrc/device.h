@@ -111,7 +111,7 @@ __device__ __forceinline__ void put_samples(int& kout, double t_start, double dt
 // Written one by one a sample cost a whole pass of the wavefront, 225 ns:
 // cs_tran of an inverter (five rows, 1 ns, 786,000 samples) took 169 ms, of
 // which the run itself is 5; now 18.5, and six sensitivities of it at
-// 1,000,001 samples 557 ms, now 124.
+// 1,000,001 samples 557 ms, now 63.
 template <int NR>
 __device__ __forceinline__ void put_rows(double* out, size_t stride, int kout, int m, double l0, double l1, double l2,
                                          const int32_t (&ps)[NR], const double (&U0)[NR], const double (&U1)[NR],

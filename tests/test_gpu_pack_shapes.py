@@ -5,6 +5,9 @@ and driven sources, one, two and four rows per lane, and circuits whose solve
 has long tasks and updated diagonals (an RC mesh).  The step sequences are
 equal, so waveforms agree to reltol 1e-6 / abstol 1e-9 V as in the other
 parity tests."""
+import ctypes
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -117,20 +120,61 @@ def test_early_stop_leaves_later_samples(engine):
         assert np.all(r.wave[done, 0] > 1.0) and np.all(r.wave[~done] == 0.0)
 
 
-def test_large_sample_buffer_is_given_back(engine):
-    """More than 64 MiB of samples: the buffer kept per circuit is freed after
-    the call, and the next calls, large and small, give the same samples
-    (every 100,000th sample of the large run is one of the small run's)."""
-    print("[gpu] large sample buffer", flush=True)
+@pytest.mark.parametrize("kern", [L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_LDS])
+def test_large_sample_buffer_is_given_back(engine, kern):
+    """More than 64 MiB of samples: the context's buffer is freed after the
+    call, and the next calls, large and small, give the same samples (every
+    100,000th sample of the large run is one of the small run's)."""
+    print(f"[gpu] large sample buffer, kernel {kern}", flush=True)
     flat = ch.lower(inverter())
     s = engine.load(flat)
     m = 100_000
     n_out = 20 * m + 1
     assert n_out * len(s.probes) * 8 > 64 << 20
-    runs = [s.tran(ch.grid_options((0.0, 1e-9), n_out=k)) for k in (21, n_out, 21, n_out)]
+    runs = [s.tran(ch.grid_options((0.0, 1e-9), n_out=k, batch_kernel=kern)) for k in (21, n_out, 21, n_out)]
     assert all(r.retcode == "Success" for r in runs)
     assert np.array_equal(runs[0].wave, runs[2].wave) and np.array_equal(runs[1].wave, runs[3].wave)
     assert np.all(np.abs(runs[1].wave[::m] - runs[0].wave) <= 1e-9 * np.abs(runs[0].wave) + 1e-9)
+
+
+def _free_device_memory():
+    hip = ctypes.CDLL("libamdhip64.so.7")   # the runtime the library itself links
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_sample_buffers_do_not_add_up_over_circuits():
+    """Twelve circuits of one context, each run with 30 MiB of samples: the
+    context keeps one buffer for all of them (each had kept its own, and as
+    much pinned host memory)."""
+    print("[gpu] sample buffers over circuits", flush=True)
+    eng = ch.Engine(0)
+    try:
+        flat = ch.lower(inverter())
+        systems = [eng.load(flat) for _ in range(12)]
+        n_out = (30 << 20) // (8 * len(systems[0].probes))
+        free = []
+        for s in systems:
+            assert s.tran(ch.grid_options((0.0, 1e-10), n_out=n_out)).retcode == "Success"
+            free.append(_free_device_memory())
+        assert free[0] - free[-1] <= 16 << 20
+    finally:
+        eng.close()
+
+
+@pytest.mark.parametrize("kern", [L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_LDS])
+def test_two_threads_on_one_context(engine, kern):
+    """Two threads, each with a circuit of its own in the same context: every
+    run gives the samples it gives alone."""
+    print(f"[gpu] two threads, kernel {kern}", flush=True)
+    systems = [engine.load(ch.lower(inverter())), engine.load(ch.lower(inverter(cload=25e-15)))]
+    opts = [ch.grid_options((0.0, 3e-10), n_out=k, batch_kernel=kern) for k in (31, 60_001)]
+    alone = [[s.tran(o).wave for o in opts] for s in systems]
+    with ThreadPoolExecutor(2) as ex:
+        got = list(ex.map(lambda s: [s.tran(opts[q % 2]).wave for q in range(12)], systems))
+    for g, a in zip(got, alone):
+        assert all(np.array_equal(w, a[q % 2]) for q, w in enumerate(g))
 
 
 def test_infinite_tolerance_and_span(engine):
