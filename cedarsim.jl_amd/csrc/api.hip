@@ -880,7 +880,10 @@ int cs_dcop(cs_ctx* ctx, int32_t cid, const double* p, const cs_tran_opts* o, do
         if (rc) ctx->err = err;
         return rc;
     }
-    if (C->lds_nr && o->batch_kernel != CS_BATCH_KERNEL_GLOBAL) return dcop_single(ctx, *C, p, o, u_out, st);
+    if (C->lds_nr && o->batch_kernel != CS_BATCH_KERNEL_GLOBAL) {
+        rc = dcop_single(ctx, *C, p, o, u_out, st);
+        if (rc != CS_E_OOM || o->batch_kernel == CS_BATCH_KERNEL_LDS) return rc;
+    }
     if ((rc = ensure_workspace(ctx, *C)) || (rc = ensure_graph(ctx, *C))) return rc;
     const Plan& P = C->plan;
     HIPCHK(ctx, hipMemcpyAsync(C->w.p, p, sizeof(double) * P.lay.n_params, hipMemcpyHostToDevice, ctx->stream));
@@ -1302,9 +1305,13 @@ static int single_buffers(cs_ctx* ctx, Circuit& C, const cs_tran_opts& o, bool w
     if (at > ctx->sbuf_bytes || pinned > ctx->h_sbuf_bytes) {
         single_free(ctx);
         const size_t bytes = at + at / 4, h_bytes = pinned + pinned / 4;
-        HIPCHK(ctx, hipMalloc((void**)&ctx->sbuf, bytes));
+        if (hipMalloc((void**)&ctx->sbuf, bytes) != hipSuccess ||
+            hipHostMalloc((void**)&ctx->h_sbuf, h_bytes, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();   // later launches must not report it
+            single_free(ctx);
+            return fail(ctx, CS_E_OOM, "no memory for the run's parameters and samples");
+        }
         ctx->sbuf_bytes = bytes;
-        HIPCHK(ctx, hipHostMalloc((void**)&ctx->h_sbuf, h_bytes, hipHostMallocDefault));
         ctx->h_sbuf_bytes = h_bytes;
     }
     char *h = ctx->h_sbuf, *d = ctx->sbuf;
@@ -1433,8 +1440,10 @@ int cs_tran(cs_ctx* ctx, int32_t cid, const double* p, const double* u0, const c
     // a circuit takes the same kernel and the same bits either way.
     if (o && C && p && !C->big && C->lds_nr && o->batch_kernel == CS_BATCH_KERNEL_AUTO &&
         (!wave || sizeof(double) * std::max(o->n_out, 0) * C->plan.probe.size() <= kSingleMax) &&
-        (o->jac_reuse == 0 || (o->jac_reuse == 1 && C->plan.n_mos == 0)))
-        return tran_single(ctx, *C, p, u0, o, wave, u_final, st_out);
+        (o->jac_reuse == 0 || (o->jac_reuse == 1 && C->plan.n_mos == 0))) {
+        const int rc = tran_single(ctx, *C, p, u0, o, wave, u_final, st_out);
+        if (rc != CS_E_OOM) return rc;   // without memory for its samples: the plain path needs none
+    }
     return tran_plain(ctx, cid, p, u0, o, wave, u_final, st_out, nullptr);
 }
 
@@ -1475,7 +1484,10 @@ static int sens_single(cs_ctx* ctx, Circuit& C, const double* p, const double* u
                  o_u = take(sizeof(double) * n), o_w = take(sizeof(double) * (size_t)n_out * np),
                  o_s = take(sizeof(double) * (size_t)n_out * blk);
     char* d = nullptr;
-    HIPCHK(ctx, hipMalloc((void**)&d, at));
+    if (hipMalloc((void**)&d, at) != hipSuccess) {
+        (void)hipGetLastError();   // later launches must not report it
+        return fail(ctx, CS_E_OOM, "no memory for the run's samples");
+    }
     a.P = C.d_dplan;
     a.p = (const double*)(d + o_p);
     a.u0 = uic ? (const double*)(d + o_u0) : nullptr;
@@ -1540,7 +1552,10 @@ int cs_tran_sens(cs_ctx* ctx, int32_t cid, const double* p, const double* u0, co
         R.sp[j].val = p ? p[sp_idx[j]] : 0.0;
     }
     if (!p) return fail(ctx, CS_E_INVALID, "bad argument");
-    if (sens_fits(ctx, *C, *o, n_sp)) return sens_single(ctx, *C, p, u0, o, R.sp, wave, sens, u_final, st_out);
+    if (sens_fits(ctx, *C, *o, n_sp)) {
+        const int rs = sens_single(ctx, *C, p, u0, o, R.sp, wave, sens, u_final, st_out);
+        if (rs != CS_E_OOM) return rs;   // without memory for its samples: the host's step control needs none
+    }
     const int n = P.n, np = (int)P.probe.size();
     R.S.assign(3 * (size_t)n_sp * np, 0.0);
     R.s_nat.assign((size_t)n_sp * n, 0.0);
