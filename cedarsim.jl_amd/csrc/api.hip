@@ -1266,10 +1266,12 @@ struct SingleRun {
     size_t up, down;        // bytes to copy up; bytes of results to copy down
 };
 
-// The buffers outlive the call up to kSingleKeep bytes; a run whose samples
+// The buffers outlive the call up to kSingleKeep bytes.  A run whose samples
 // need more than kSingleMax stays on the plain path, which writes them
-// straight to the caller's array.
-constexpr size_t kSinglePin = (size_t)1 << 20, kSingleKeep = (size_t)64 << 20, kSingleMax = (size_t)1 << 30;
+// straight to the caller's array: 17 ns a sample of five values in one launch
+// against 8 there, so that an inverter's 1 ns takes 33 against 70 ms with 60
+// MiB of them and 145 against 122 with 300.
+constexpr size_t kSinglePin = (size_t)1 << 20, kSingleKeep = (size_t)96 << 20, kSingleMax = (size_t)64 << 20;
 
 static void single_free(cs_ctx* ctx) {
     if (ctx->sbuf) (void)hipFree(ctx->sbuf);
@@ -1450,14 +1452,16 @@ int cs_tran(cs_ctx* ctx, int32_t cid, const double* p, const double* u0, const c
 // A sensitivity run goes in one launch (k_tran_sens) where a wavefront holds
 // one unknown per lane, the factors fit the default LDS, and every
 // parameter's wavefront is resident at once (four per CU); its samples are
-// held on the device up to kSingleMax bytes.  Modified Newton,
+// held on the device up to kSensMax bytes (an inverter's 267 MiB: 63 ms
+// against 106 with the host's step control, which costs half as much a sample).  Modified Newton,
 // Verilog-A devices and larger circuits keep the host's step control, and
 // CS_BATCH_KERNEL_GLOBAL asks for it.
+constexpr size_t kSensMax = (size_t)512 << 20;
 static bool sens_fits(const cs_ctx* ctx, const Circuit& C, const cs_tran_opts& o, int32_t n_sp) {
     const Plan& P = C.plan;
     return o.batch_kernel == CS_BATCH_KERNEL_AUTO && o.jac_reuse == 0 && P.n_va == 0 && P.n <= kSensMaxN &&
            tran_sens_lds(P.n, P.nnz, P.n_stamp) <= 40 * 1024 && n_sp <= 4 * std::max(ctx->n_cu, 1) &&
-           sizeof(double) * std::max(o.n_out, 0) * P.probe.size() * (n_sp + 1) <= kSingleMax;
+           sizeof(double) * std::max(o.n_out, 0) * P.probe.size() * (n_sp + 1) <= kSensMax;
 }
 
 static int sens_single(cs_ctx* ctx, Circuit& C, const double* p, const double* u0, const cs_tran_opts* o,

@@ -320,8 +320,9 @@ int cs_dcop(cs_ctx* ctx, int32_t cid, const double* p, const cs_tran_opts* o,
 /* tran!(circ, tspan).  By default a circuit that fits runs its whole transient
  * in one launch of the LDS-resident kernel, as a batch of one; circuits that
  * do not fit (more than 256 unknowns or 512 devices, Verilog-A devices, 64 KiB
- * of LDS), supernodal ones, and modified Newton (jac_reuse) on a circuit with
- * nonlinear devices take the plain path: the host runs the BDF step control
+ * of LDS), supernodal ones, runs with more than 64 MiB of samples or no memory
+ * for them, and modified Newton (jac_reuse) on a circuit with nonlinear devices
+ * take the plain path: the host runs the BDF step control
  * and every Newton iteration is one launch of a captured hipGraph (device
  * eval -> assembly -> LU refactor -> solve -> norm).  Both follow the same
  * rules; results agree to rounding.  o->batch_kernel = CS_BATCH_KERNEL_LDS
@@ -438,7 +439,8 @@ int cs_bsimcmg_eval_noalloc(cs_ctx* ctx, int64_t n, const double* L, const doubl
  * operating point, the DC point's sensitivity pins them).  wave as cs_tran
  * (required); sens: n_out x n_sp x n_probe, interpolated like wave.
  * Circuits of up to 64 unknowns run in one launch; larger ones, jac_reuse,
- * Verilog-A devices and CS_BATCH_KERNEL_GLOBAL take the plain path.
+ * Verilog-A devices, more than 512 MiB of samples (or no memory for them) and
+ * CS_BATCH_KERNEL_GLOBAL take the plain path.
  * Circuits on the supernodal solver are refused. */
 int cs_tran_sens(cs_ctx* ctx, int32_t cid, const double* p, const double* u0, const cs_tran_opts* o,
                  int32_t n_sp, const int32_t* sp_idx, double* wave, double* sens, double* u_final,

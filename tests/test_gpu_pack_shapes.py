@@ -120,17 +120,20 @@ def test_early_stop_leaves_later_samples(engine):
         assert np.all(r.wave[done, 0] > 1.0) and np.all(r.wave[~done] == 0.0)
 
 
-@pytest.mark.parametrize("kern", [L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_LDS])
-def test_large_sample_buffer_is_given_back(engine, kern):
-    """More than 64 MiB of samples: the context's buffer is freed after the
-    call, and the next calls, large and small, give the same samples (every
-    100,000th sample of the large run is one of the small run's)."""
-    print(f"[gpu] large sample buffer, kernel {kern}", flush=True)
+@pytest.mark.parametrize("kern,m", [(L.BATCH_KERNEL_AUTO, 83_886), (L.BATCH_KERNEL_AUTO, 83_887),
+                                    (L.BATCH_KERNEL_AUTO, 100_000), (L.BATCH_KERNEL_LDS, 100_000),
+                                    (L.BATCH_KERNEL_LDS, 130_000)])
+def test_large_sample_buffer_is_given_back(engine, kern, m):
+    """64 MiB of samples, the most that AUTO takes on the one launch, and more:
+    on the plain path, and on the one launch when asked for, whose buffer is
+    kept or freed after the call.  The next calls, large and small, give the
+    same samples (every m-th sample of the large run is one of the small
+    run's)."""
+    print(f"[gpu] large sample buffer, kernel {kern}, 20 x {m}", flush=True)
     flat = ch.lower(inverter())
     s = engine.load(flat)
-    m = 100_000
     n_out = 20 * m + 1
-    assert n_out * len(s.probes) * 8 > 64 << 20
+    assert (n_out * len(s.probes) * 8 > 64 << 20) == (m > 83_886)
     runs = [s.tran(ch.grid_options((0.0, 1e-9), n_out=k, batch_kernel=kern)) for k in (21, n_out, 21, n_out)]
     assert all(r.retcode == "Success" for r in runs)
     assert np.array_equal(runs[0].wave, runs[2].wave) and np.array_equal(runs[1].wave, runs[3].wave)
