@@ -148,6 +148,7 @@ struct SensRec {
     double *sn, *d1, *d2;          // LDS: s at the new point; charge sensitivities one and two steps back
     double pin = 0.0, s0 = 0.0, s1 = 0.0, s2 = 0.0;
 
+    __device__ __forceinline__ bool writes() const { return j == 0; }
     // J s = -(dI/dp + a0 dQ/dp + a1 d1 + a2 d2) on the Jacobian assembled in L.F
     __device__ void solve(const DPlan* P, const double* p, const Lds& L, const double* Clin, int mode, bool pinned,
                           double a0, double a1, double a2) {
@@ -212,8 +213,8 @@ struct SensRec {
 };
 
 // One wavefront per parameter, each running the whole transient with its own
-// parameter's sensitivity: they take the same steps, so every one writes the
-// same waveform, state and statistics.  The run is a serial chain of small
+// parameter's sensitivity: they take the same steps, and the first one's
+// waveform, state and statistics stand for all.  The run is a serial chain of small
 // steps, and the chip is otherwise idle: repeating the transient per
 // parameter costs nothing, while host step control cost a graph launch and a
 // round trip per Newton iteration and another of each per accepted step.

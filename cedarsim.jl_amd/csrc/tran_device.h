@@ -9,6 +9,8 @@
 // L.F, every accepted step, and every output sample; the batch passes NoRec.
 // Rec::kFineGrid writes the samples of a step together (put_samples), for
 // output grids finer than the steps; it costs the run 4 % in registers.
+// Rec::writes is false for a workgroup that repeats another's run: waveform,
+// state and statistics are that one's to write.
 #pragma once
 #include "dcop_rules.h"
 #include "device.h"
@@ -24,6 +26,7 @@ struct Lds {
 
 struct NoRec {
     static constexpr bool kFineGrid = false;
+    __device__ __forceinline__ bool writes() const { return true; }
     __device__ __forceinline__ void on_dc(const DPlan*, const double*, const Lds&, const double*) {}
     __device__ __forceinline__ void on_initial(const DPlan*, const double*, const Lds&, const double*, bool) {}
     __device__ __forceinline__ void on_step(const DPlan*, const double*, const Lds&, const double*, const double*,
@@ -151,7 +154,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
                     const int i = tid + NT * r;
                     if (i < n) {
                         const int sl = P->probe_slot[i];
-                        if (sl >= 0) wave[(size_t)kout * n_probe + sl] = Uh0[r];
+                        if (sl >= 0 && rec.writes()) wave[(size_t)kout * n_probe + sl] = Uh0[r];
                     }
                 }
                 rec.on_output(P, kout, 1.0, 0.0, 0.0);
@@ -285,7 +288,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
 #pragma unroll
                                     for (int r = 0; r < NR; r++)
                                         ps[r] = tid + NT * r < n ? P->probe_slot[tid + NT * r] : -1;
-                                    put_rows<NR>(wave, n_probe, k0, m, l0, l1, l2, ps, Uh0, Uh1, Uh2);
+                                    if (rec.writes()) put_rows<NR>(wave, n_probe, k0, m, l0, l1, l2, ps, Uh0, Uh1, Uh2);
                                     rec.on_outputs(ps, k0, m, l0, l1, l2);
                                 });
             } else if (wave) {
@@ -299,7 +302,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
                         const int i = tid + NT * r;
                         if (i < n) {
                             const int sl = P->probe_slot[i];
-                            if (sl >= 0)
+                            if (sl >= 0 && rec.writes())
                                 wave[(size_t)kout * n_probe + sl] =
                                     l0 * Uh0[r] + l1 * Uh1[r] + l2 * Uh2[r];
                         }
@@ -317,6 +320,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
             }
         }
     }
+    if (!rec.writes()) return;
 #pragma unroll
     for (int r = 0; r < NR; r++) {
         const int i = tid + NT * r;

@@ -184,3 +184,22 @@ def test_one_launch_fine_output_grid(engine, n_out, probes):
     for j in range(len(names)):
         a, b = ga[:, j], gg[:, j]
         assert np.all(np.abs(a - b) <= 1e-6 * np.abs(b) + 1e-9 * np.max(np.abs(b)) + 1e-300), names[j]
+
+
+@pytest.mark.parametrize("n_out", [21, 3001])
+def test_one_launch_does_not_depend_on_the_parameters_beside(engine, n_out):
+    """A parameter's sensitivity, the waveform, the state and the statistics are
+    the same bits whichever parameters run beside it, in any order: the first
+    parameter's wavefront writes what is common to all."""
+    flat = ch.lower(inverter())
+    sys_ = engine.load(flat)
+    names = ["MN.vth", "MN.kp", "MP.w", "MP.l", "CL", "VDD.dc"]
+    o = ch.grid_options((0.0, 0.3e-9), n_out=n_out)
+    ref, gref = sys_.tran_sens(o, names)
+    assert ref.retcode == "Success"
+    for order in ([5], [2, 0], [3, 1, 4, 0, 5, 2]):
+        r, g = sys_.tran_sens(o, [names[k] for k in order])
+        assert np.array_equal(r.wave, ref.wave) and np.array_equal(r.u_final, ref.u_final)
+        assert r.stats.steps == ref.stats.steps and r.stats.newton_iters == ref.stats.newton_iters
+        for q, k in enumerate(order):
+            assert np.array_equal(g[:, q], gref[:, k]), names[k]
