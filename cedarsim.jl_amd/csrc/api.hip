@@ -81,6 +81,7 @@ struct Batch {
     std::vector<int64_t> p_off, u_off, w_off;
     int32_t n_inst = 0;
     int32_t nr = 1;
+    bool has_va = false;                       // some circuit has Verilog-A devices
     int32_t nblocks = 0;
     size_t lds = 0;
     BatchArgs args{};
@@ -298,6 +299,7 @@ int ensure_workspace(cs_ctx* ctx, Circuit& C) {
     C.w.st = take(std::max(P.n_stamp, 1));
     C.w.norm = take(NRM_SLOTS);
     C.w.sp = (StepDev*)take(sizeof(StepDev) / sizeof(double) + 1);
+    C.w.has_va = P.n_va > 0;
     HIPCHK(ctx, hipMemset(C.wbuf, 0, bytes));
     HIPCHK(ctx, hipHostMalloc((void**)&C.h_norm, NRM_SLOTS * sizeof(double), hipHostMallocDefault));
     HIPCHK(ctx, hipHostMalloc((void**)&C.h_stage, (3 * (size_t)P.n + sizeof(StepDev) / sizeof(double) + 1) *
@@ -1840,6 +1842,7 @@ int cs_batch_create(cs_ctx* ctx, int32_t n_inst, const int32_t* inst_cid, const 
         po += P.lay.n_params;
         uo += P.n;
         wo += (int64_t)o->n_out * (int64_t)P.probe.size();
+        B->has_va = B->has_va || P.n_va > 0;
         nnz_max = std::max(nnz_max, P.nnz);
         n_max = std::max(n_max, P.n);
         st_max = std::max(st_max, P.n_stamp);
@@ -1932,7 +1935,7 @@ int cs_batch_create(cs_ctx* ctx, int32_t n_inst, const int32_t* inst_cid, const 
     A.o = *o;
     if (B->kernel == CS_BATCH_KERNEL_GLOBAL) {
         B->lds = batch_lds_bytes(A);
-        int per_cu = batch_max_blocks(B->nr, B->lds);
+        int per_cu = batch_max_blocks(B->nr, B->has_va, B->lds);
         if (per_cu <= 0) return fail(ctx, CS_E_RANGE, "batched kernel does not fit: LDS per instance too large");
         B->nblocks = std::min<int64_t>(n_inst, (int64_t)per_cu * std::max(ctx->n_cu, 1));
         void *d_g, *d_c, *d_l;
@@ -1969,7 +1972,7 @@ int cs_batch_run(cs_ctx* ctx, int32_t bid, double* kernel_ms) {
     if (B->kernel == CS_BATCH_KERNEL_GLOBAL) {
         HIPCHK(ctx, hipMemsetAsync(B->args.queue, 0, sizeof(int32_t), s));
         HIPCHK(ctx, hipEventRecord(B->ev0, s));
-        HIPCHK(ctx, launch_tran_batch(B->nr, B->args, B->nblocks, B->lds, s));
+        HIPCHK(ctx, launch_tran_batch(B->nr, B->has_va, B->args, B->nblocks, B->lds, s));
         HIPCHK(ctx, hipEventRecord(B->ev1, s));
     } else {
         HIPCHK(ctx, hipMemsetAsync(B->pack_args.queue, 0, sizeof(int32_t), s));

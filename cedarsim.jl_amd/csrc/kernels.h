@@ -26,6 +26,7 @@ enum : int32_t { NRM_WRMS = 0, NRM_MAXD = 1, NRM_RES = 2, NRM_DONE = 3, NRM_SLOT
 struct InstDev {
     double *p, *linbuf, *Glin, *Clin, *F, *inv, *u, *x, *qx, *st, *u0, *norm;
     StepDev* sp;
+    bool has_va;             // the circuit has Verilog-A devices
 };
 
 struct BatchArgs {
@@ -217,8 +218,8 @@ void launch_charges(const DPlan* dp, const InstDev& w, const double* v, double* 
 
 // batched transient: LDS bytes per workgroup and launch
 size_t batch_lds_bytes(const BatchArgs& a);
-int batch_max_blocks(int nr, size_t lds);   // resident workgroups per CU
-hipError_t launch_tran_batch(int nr, const BatchArgs& a, int nblocks, size_t lds, hipStream_t s);
+int batch_max_blocks(int nr, bool va, size_t lds);   // resident workgroups per CU
+hipError_t launch_tran_batch(int nr, bool va, const BatchArgs& a, int nblocks, size_t lds, hipStream_t s);
 
 // LDS bytes of one instance beside its image
 size_t lds_kernel_bytes(int32_t dbl_max, int32_t words_max);

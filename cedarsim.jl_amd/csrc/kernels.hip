@@ -28,15 +28,16 @@ __global__ __launch_bounds__(kSingleThreads) void k_lin_setup(const DPlan* dp, I
 }
 
 // JAC = false: the residual only, F keeps the factors of an earlier
-// iteration (modified Newton)
-template <bool JAC>
+// iteration (modified Newton).  VA = false: no Verilog-A device, whose models
+// would hold registers and scratch memory
+template <bool JAC, bool VA>
 __global__ __launch_bounds__(kSingleThreads) void k_eval_assemble(const DPlan* dp, InstDev w) {
     __shared__ double red[kSingleThreads];
     const DPlan* P = dp;
     const StepDev sp = *w.sp;
     dev_sources<kSingleThreads>(P, w.p, sp.t, sp.mode, w.st);
     dev_mos<kSingleThreads>(P, w.p, w.u, w.st, w.p[P->p_gmin]);
-    if (P->n_va) dev_va<kSingleThreads>(P, w.p, w.u, w.st, w.p[P->p_gmin]);
+    if constexpr (VA) dev_va<kSingleThreads>(P, w.p, w.u, w.st, w.p[P->p_gmin]);
     __syncthreads();
     const double a0 = sp.kind == STEP_TRAN ? sp.a0 : 0.0;
     const double m = dev_assemble<kSingleThreads, JAC>(P, w.Glin, w.Clin, a0, w.u,
@@ -105,8 +106,9 @@ void launch_lin_setup(const DPlan* dp, const InstDev& w, hipStream_t s) {
     hipLaunchKernelGGL(k_lin_setup, dim3(1), dim3(kSingleThreads), 0, s, dp, w);
 }
 void launch_eval_assemble(const DPlan* dp, const InstDev& w, hipStream_t s, bool jac) {
-    if (jac) hipLaunchKernelGGL(k_eval_assemble<true>, dim3(1), dim3(kSingleThreads), 0, s, dp, w);
-    else hipLaunchKernelGGL(k_eval_assemble<false>, dim3(1), dim3(kSingleThreads), 0, s, dp, w);
+    auto* f = w.has_va ? (jac ? k_eval_assemble<true, true> : k_eval_assemble<false, true>)
+                       : (jac ? k_eval_assemble<true, false> : k_eval_assemble<false, false>);
+    hipLaunchKernelGGL(f, dim3(1), dim3(kSingleThreads), 0, s, dp, w);
 }
 void launch_lu(const DPlan* dp, const InstDev& w, hipStream_t s) {
     hipLaunchKernelGGL(k_lu, dim3(1), dim3(kSingleThreads), 0, s, dp, w);
@@ -134,7 +136,7 @@ namespace {
 // wavefronts per SIMD) the compiler spilled 74 of them, among them the ones
 // it keeps spilled scalar registers in, and in a build without Verilog-A
 // models the kernel's answers were wrong (runs ended with DtLessThanMin).
-template <int NR>
+template <int NR, bool VA>
 __global__ __launch_bounds__(NT) void k_tran_batch(BatchArgs A) {
     extern __shared__ double lds[];
     __shared__ int s_idx;
@@ -160,7 +162,7 @@ __global__ __launch_bounds__(NT) void k_tran_batch(BatchArgs A) {
         const int cid = __builtin_amdgcn_readfirstlane(A.inst_cid[inst]);
         const DPlan* P = A.plans + cid;
         NoRec rec;
-        run_instance<NR>(rec, P, A.params + A.p_off[inst], A.u0 ? A.u0 + A.u_off[inst] : nullptr,
+        run_instance<NR, VA>(rec, P, A.params + A.p_off[inst], A.u0 ? A.u0 + A.u_off[inst] : nullptr,
                          A.wave ? A.wave + A.w_off[inst] : nullptr, A.u_final + A.u_off[inst],
                          A.stats + inst, A.o, L, Glin, Clin, linbuf);
     }
@@ -172,30 +174,28 @@ size_t batch_lds_bytes(const BatchArgs& a) {
     return sizeof(double) * ((size_t)a.nnz_max + 4 * (size_t)a.n_max + a.stamp_max);
 }
 
-template <int NR>
-static int max_blocks_nr(size_t lds) {
+namespace {
+typedef void (*BatchKernel)(BatchArgs);
+template <bool VA>
+BatchKernel batch_kernel(int nr) {
+    switch (nr) {
+    case 1: return k_tran_batch<1, VA>;
+    case 2: return k_tran_batch<2, VA>;
+    case 4: return k_tran_batch<4, VA>;
+    default: return k_tran_batch<8, VA>;
+    }
+}
+BatchKernel batch_kernel(int nr, bool va) { return va ? batch_kernel<true>(nr) : batch_kernel<false>(nr); }
+}  // namespace
+
+int batch_max_blocks(int nr, bool va, size_t lds) {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_tran_batch<NR>, NT, lds) != hipSuccess)
-        return 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_kernel(nr, va), NT, lds) != hipSuccess) return 0;
     return nb;
 }
 
-int batch_max_blocks(int nr, size_t lds) {
-    switch (nr) {
-    case 1: return max_blocks_nr<1>(lds);
-    case 2: return max_blocks_nr<2>(lds);
-    case 4: return max_blocks_nr<4>(lds);
-    default: return max_blocks_nr<8>(lds);
-    }
-}
-
-hipError_t launch_tran_batch(int nr, const BatchArgs& a, int nblocks, size_t lds, hipStream_t s) {
-    switch (nr) {
-    case 1: hipLaunchKernelGGL(k_tran_batch<1>, dim3(nblocks), dim3(NT), lds, s, a); break;
-    case 2: hipLaunchKernelGGL(k_tran_batch<2>, dim3(nblocks), dim3(NT), lds, s, a); break;
-    case 4: hipLaunchKernelGGL(k_tran_batch<4>, dim3(nblocks), dim3(NT), lds, s, a); break;
-    default: hipLaunchKernelGGL(k_tran_batch<8>, dim3(nblocks), dim3(NT), lds, s, a); break;
-    }
+hipError_t launch_tran_batch(int nr, bool va, const BatchArgs& a, int nblocks, size_t lds, hipStream_t s) {
+    hipLaunchKernelGGL(batch_kernel(nr, va), dim3(nblocks), dim3(NT), lds, s, a);
     return hipGetLastError();
 }
 

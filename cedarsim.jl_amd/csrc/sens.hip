@@ -235,7 +235,7 @@ __global__ __launch_bounds__(NT) void k_tran_sens(SensRunArgs A) {
     SensRec<FineGrid> rec{A, j, sn, sn + A.n, sn + 2 * A.n};
     if ((int)threadIdx.x < A.n) rec.d1[threadIdx.x] = rec.d2[threadIdx.x] = 0.0;
     double* lin = A.ws + (size_t)j * A.ws_stride;
-    run_instance<1>(rec, A.P, A.p, A.u0, A.wave, A.u_final, A.stats, A.o, L, lin + A.n_lin,
+    run_instance<1, false>(rec, A.P, A.p, A.u0, A.wave, A.u_final, A.stats, A.o, L, lin + A.n_lin,
                     lin + A.n_lin + A.nnz, lin);
 }
 

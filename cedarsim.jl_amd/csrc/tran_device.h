@@ -4,7 +4,8 @@
 // wavefront) owns one circuit instance; lane l owns unknowns l, l+64, ...
 // (NR of them) and keeps their history in registers.
 //
-// Rec is called at the points a forward sensitivity run needs (sens.hip): the
+// VA: some circuit has Verilog-A devices; without, their models' code is left
+// out.  Rec is called at the points a forward sensitivity run needs (sens.hip): the
 // DC point and the initial point, each with its Jacobian just assembled in
 // L.F, every accepted step, and every output sample; the batch passes NoRec.
 // Rec::kFineGrid writes the samples of a step together (put_samples), for
@@ -34,7 +35,7 @@ struct NoRec {
     __device__ __forceinline__ void on_output(const DPlan*, int, double, double, double) {}
 };
 
-template <int NR, class Rec>
+template <int NR, bool VA, class Rec>
 __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double* __restrict__ p,
                              const double* __restrict__ u0, double* __restrict__ wave,
                              double* __restrict__ ufin, cs_tran_stats* __restrict__ stp,
@@ -76,7 +77,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
         bool ok = false;
         for (;;) {
             dev_mos<NT>(P, p, L.u, L.st, g);
-            if (P->n_va) dev_va<NT>(P, p, L.u, L.st, g);
+            if constexpr (VA) dev_va<NT>(P, p, L.u, L.st, g);
             __syncthreads();
             const double lm = dev_assemble<NT>(P, Glin, Clin, 0.0, L.u, nullptr, L.st, L.F, L.x, pin);
             const double fn = block_reduce<NT>(lm, nullptr, OpMax());
@@ -198,7 +199,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
             bool conv = false;
             for (int it = 0; it < o.newton_maxit; it++) {
                 dev_mos<NT>(P, p, L.u, L.st, gmin);
-                if (P->n_va) dev_va<NT>(P, p, L.u, L.st, gmin);
+                if constexpr (VA) dev_va<NT>(P, p, L.u, L.st, gmin);
                 __syncthreads();
                 dev_assemble<NT>(P, Glin, Clin, a0, L.u, L.qx, L.st, L.F, L.x, nullptr);
                 __syncthreads();
