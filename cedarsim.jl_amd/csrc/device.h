@@ -15,6 +15,7 @@
 #include "dplan.h"
 #include "rules.h"
 #include "va_registry.h"
+#include "wave_math.h"
 
 namespace cedar {
 
@@ -168,12 +169,15 @@ __device__ void dev_lin_setup(const DPlan* __restrict__ P, const double* __restr
     __syncthreads();
 }
 
-template <int NT>
+// Inline: by wave_math.h's source_at, for kernels that run whole transients
+template <int NT, bool Inline = false>
 __device__ void dev_sources(const DPlan* __restrict__ P, const double* __restrict__ p,
                                             double t, int mode, double* __restrict__ st) {
     for (int s = threadIdx.x; s < P->n_src; s += NT) {
         const int4 d = P->src[s];
-        const double val = source_value(d.x, p + d.y, d.z, p[d.w], t, mode);
+        double val;
+        if constexpr (Inline) val = source_at(d.x, p + d.y, d.z, p[d.w], t, mode);
+        else val = source_value(d.x, p + d.y, d.z, p[d.w], t, mode);
         st[4 * P->n_mos + s] = P->src_m ? val * P->src_m[s] : val;
     }
 }

@@ -132,12 +132,24 @@ void launch_charges(const DPlan* dp, const InstDev& w, const double* v, double* 
 // ---------------------------------------------------------------------------
 namespace {
 
-// No register limit beyond the wavefront's own: held to 128 VGPRs (four
-// wavefronts per SIMD) the compiler spilled 74 of them, among them the ones
-// it keeps spilled scalar registers in, and in a build without Verilog-A
-// models the kernel's answers were wrong (runs ended with DtLessThanMin).
+// Bound by the latency of one wavefront's chains through the caches and LDS, so
+// by how many wavefronts are resident once a batch fills the device: registers.
+// With the waveforms and step factors of wave_math.h they are 123, 126, 164
+// and 216 (1, 2, 4 and 8 rows per lane; four, four, three and two wavefronts
+// per SIMD) and none is spilled; with the library's sin, exp, fmod and pow
+// inlined 208 to 256. Those held to 128 (74 spilled, among them the ones that
+// keep spilled scalar registers) gave wrong answers in a build without
+// Verilog-A models, DtLessThanMin from the first steps; the source is not at
+// fault as far as a CPU build shows (address and undefined-behaviour sanitizers,
+// uninitialised variables filled with patterns, lanes in any order between
+// barriers: the oracle's steps, one set of bits). So no limit that spills.
+// 4096 rings over 2 ps: 33 stages 7.5 ms held to 128, 8.0 without a limit, 5.2
+// now; 67 stages 12.8, 14.9, 10.3; 4096 12 x 12 meshes over 20 ps 44.7, 41.7,
+// 41.5.  The Verilog-A models take 175 and more (two per SIMD): 2048 inverters
+// of them 36.5 ms held to 128 and 30.4 now, but 4096 of them 50.4 and 60.4.
 template <int NR, bool VA>
-__global__ __launch_bounds__(NT) void k_tran_batch(BatchArgs A) {
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NR <= 2 && !VA ? 4 : 1)))
+void k_tran_batch(BatchArgs A) {
     extern __shared__ double lds[];
     __shared__ int s_idx;
     Lds L;

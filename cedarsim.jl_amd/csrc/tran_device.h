@@ -67,7 +67,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
     // of the second step are kept in L.qx, free until the charges are set.
     const double gmin = p[P->p_gmin];
     {
-        dev_sources<NT>(P, p, o.t_start, uic ? CS_MODE_TRAN : CS_MODE_DCOP, L.st);
+        dev_sources<NT, true>(P, p, o.t_start, uic ? CS_MODE_TRAN : CS_MODE_DCOP, L.st);
         int phase = uic ? -1 : 0, stage = 0, it = 0;
         const double* pin = uic ? u0 : nullptr;
         double g = gmin;
@@ -95,7 +95,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
                 if (!dc_done) { ok = true; break; }
                 rec.on_dc(P, p, L, Clin);
                 for (int i = tid; i < n; i += NT) L.qx[i] = L.u[i];
-                dev_sources<NT>(P, p, o.t_start, CS_MODE_TRAN, L.st);
+                dev_sources<NT, true>(P, p, o.t_start, CS_MODE_TRAN, L.st);
                 pin = L.qx;
                 phase = -1;
                 g = gmin;
@@ -168,7 +168,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
             double lb = INFINITY;
             for (int s = tid; s < P->n_src; s += NT) {
                 const int4 d = P->src[s];
-                const double b = wave_next_bp(d.x, p + d.y, d.z, t);
+                const double b = next_bp(d.x, p + d.y, d.z, t);
                 if (b < lb) lb = b;
             }
             double tb = block_reduce<NT>(lb, nullptr, OpMin());
@@ -194,7 +194,7 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
                     L.qx[i] = a1 * Qh0[r] + (k == 2 ? a2 * Qh1[r] : 0.0);
                 }
             }
-            dev_sources<NT>(P, p, tn, CS_MODE_TRAN, L.st);
+            dev_sources<NT, true>(P, p, tn, CS_MODE_TRAN, L.st);
             __syncthreads();
             bool conv = false;
             for (int it = 0; it < o.newton_maxit; it++) {
@@ -245,14 +245,14 @@ __device__ void run_instance(Rec& rec, const DPlan* __restrict__ P, const double
                         ss += q * q;
                     }
                 }
-                const double err = sqrt(block_reduce<NT>(ss, nullptr, OpSum()) / n);
-                if (!(err <= 1.0)) {
+                const double err2 = block_reduce<NT>(ss, nullptr, OpSum()) / n;
+                if (!(err2 <= 1.0)) {
                     rej++;
-                    h = hh * reject_factor(err, k);
+                    h = hh * step_reject(err2, k);
                     if (h < sd.dt_min) { rc = CS_E_DTMIN; break; }
                     continue;
                 }
-                fac = accept_factor(err, k);
+                fac = step_accept(err2, k);
             }
             // accept
             rec.on_step(P, p, L, Glin, Clin, gmin, k, a0, a1, a2);

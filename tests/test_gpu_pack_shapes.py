@@ -326,3 +326,65 @@ def test_samples_cost_less_than_the_run(engine):
         busy[n_out] = r.stats.busy_s
     print(f"[gpu] busy {busy}", flush=True)
     assert busy[200_001] <= 2.0 * busy[21]
+
+
+def test_global_kernel_fills_the_device(engine):
+    """4096 instances of a small circuit on the global-plan kernel are resident
+    at once: they take little longer than 2048 (in two rounds, twice as
+    long for rings of 33 stages less what a fuller CU costs: half as long
+    again)."""
+    print("[gpu] residency of the global-plan kernel", flush=True)
+    flat = ch.lower(ring_oscillator(33))
+    u0 = ring_initial_state(flat, np.random.default_rng(7))
+    s = engine.load(flat)
+    ms = {}
+    for count in (2048, 4096):
+        b = ch.Batch(engine, [s], [0] * count, [flat.params()] * count,
+                     ch.TranOptions(t_stop=2e-12, init=L.INIT_UIC, batch_kernel=L.BATCH_KERNEL_GLOBAL), [u0] * count)
+        try:
+            ms[count] = min(b.run() for _ in range(3))
+            assert set(b.results().retcodes) == {"Success"}
+        finally:
+            b.close()
+    print(f"[gpu] kernel ms {ms}", flush=True)
+    assert ms[4096] <= 1.25 * ms[2048]
+
+
+@pytest.mark.parametrize("wave", ["damped_sine", "late_sine", "one_shot_pulse", "slow_pulse", "sine_cycles"])
+def test_waveforms_on_every_kernel(engine, wave):
+    """Sources whose values the batched and one-launch kernels compute by
+    wave_math.h (damped and phase-shifted sines, a delayed one, one that ends
+    after its cycles, a pulse with no period, one with a period the run passes
+    twice) against the plain path, which calls the library, and the oracle."""
+    from cedarhip.netlist import WAVE_PULSE, WAVE_SIN, Waveform
+    print(f"[gpu] waveform {wave}", flush=True)
+    w = {"damped_sine": (WAVE_SIN, [0.3, 1.2, 2.5e9, 1e-10, 1.5e9, 40.0, 1e30]),
+         "late_sine": (WAVE_SIN, [0.9, -0.7, 1e9, 7e-10, 0.0, -75.0, 1e30]),
+         "sine_cycles": (WAVE_SIN, [0.9, 0.8, 3e9, 0.0, 0.0, 200.0, 2.0]),
+         "one_shot_pulse": (WAVE_PULSE, [0.1, 1.7, 2e-10, 5e-11, 8e-11, 3e-10, np.inf]),
+         "slow_pulse": (WAVE_PULSE, [1.7, 0.1, 1e-10, 5e-11, 8e-11, 2e-10, 6e-10])}[wave]
+
+    def circuit():
+        vin, out, gnd = (ch.Named(ch.net, k)() for k in ("in", "out", "gnd"))
+        ch.Named(ch.VoltageSource(tran=Waveform(*w)), "VIN")(vin, gnd)
+        ch.Named(ch.R(1e3), "R")(vin, out)
+        ch.Named(ch.C(1e-13), "C")(out, gnd)
+        ch.Gnd()(gnd)
+
+    flat = ch.lower(circuit)
+    p = flat.params()
+    s = engine.load(flat)
+    ref, _, st, rc = O.tran(flat, p, None, ch.grid_options((0.0, 1.5e-9), n_out=61))
+    assert rc == 0
+    waves = []
+    for kern in (L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_GLOBAL):
+        o = ch.grid_options((0.0, 1.5e-9), n_out=61, batch_kernel=kern)
+        r = s.tran(o, p)
+        assert r.retcode == "Success" and r.stats.steps == st.steps
+        waves.append(r.wave)
+        b = ch.tran_batch([flat] * 2, [p, p], o, engine=engine)
+        assert b.retcodes == ["Success"] * 2 and b.stats[1].steps == st.steps
+        waves += b.wave
+        waves.append(s.tran_sens(o, ["R"], p)[0].wave)
+    for x in waves:
+        assert np.all(np.abs(x - ref) <= 1e-6 * np.abs(ref) + 1e-9)
