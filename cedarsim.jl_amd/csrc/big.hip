@@ -811,7 +811,10 @@ __device__ __forceinline__ void panel_stage(double (&a)[kNb], int& p, int nb, do
             a[i] = Col ? a[i + 1] - (o * ipc) * l : a[i + 1] - l * o;
         };
         // the next pivot first; the dependent operations of its reciprocal
-        // (1.0 / x, step by step) then alternate with the other updates
+        // then alternate with the other updates.  They are the sequence the
+        // CDNA instruction set documents for a 64-bit division (scale, estimate,
+        // two corrections, quotient, div_fmas, div_fixup), the one the
+        // compiler makes of 1.0 / x, written out so that it can be spread
         update(0);
         const double x = wave_bcast(a[0], p + 1);
         constexpr int G = (W - 2 + 8) / 9;

@@ -137,7 +137,8 @@ hipError_t launch_tran_sens(const SensRunArgs& a, hipStream_t s);
 
 struct CPlan;
 
-// LDS-resident batched transient (tran_lds.hip): one launch per size class.
+// Arguments of the LDS-resident kernels: the packed launch of a batch, a single
+// circuit's run or DC point (tran_lds.hip), an adjoint class (adj_lds.hip).
 struct LdsArgs {
     const CPlan* cplans;
     const DPlan* plans;
@@ -150,10 +151,10 @@ struct LdsArgs {
     double* wave;            // may be null
     double* u_final;
     cs_tran_stats* stats;
-    const int32_t* order;    // this class's instances, largest first
-    int32_t* queue;          // this class's queue head (zeroed before launch)
-    int32_t n_inst;          // instances in this class
-    int32_t dbl_max;         // LDS doubles before the plan image
+    const int32_t* order;    // the launch's instances, in its order
+    int32_t* queue;          // its queue's head (zeroed before launch)
+    int32_t n_inst;          // its instances
+    int32_t dbl_max;         // LDS doubles before the plan image (adjoint)
     cs_tran_opts o;
     // packed launch: a chunk is up to kPackSegs segments, each a run of
     // instances of one circuit, one wavefront each.  Segment j is segs[2j] =

@@ -9,7 +9,7 @@
 // DC point and the initial point, each with its Jacobian just assembled in
 // L.F, every accepted step, and every output sample; the batch passes NoRec.
 // Rec::kFineGrid writes the samples of a step together (put_samples), for
-// output grids finer than the steps; it costs the run 4 % in registers.
+// output grids finer than the steps; it costs the run 4 %.
 // Rec::writes is false for a workgroup that repeats another's run: waveform,
 // state and statistics are that one's to write.
 #pragma once

@@ -1,7 +1,7 @@
 // tran_lds.hip — the LDS-resident batched transient kernels.
 //
 // k_tran_pack (the batched transient): one launch for the whole batch.  A
-// persistent grid of workgroups of kPackWaves wavefronts walks a queue of
+// persistent grid of workgroups of up to kPackWaves wavefronts walks a queue of
 // chunks.  A chunk is up to kPackSegs segments, each a run of instances of
 // one circuit: the workgroup copies the segments' plan images into LDS and
 // each wavefront runs one instance's whole transient (lds_core.h) in its own

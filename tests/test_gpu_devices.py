@@ -125,12 +125,15 @@ def _check_reference(name, flat, o, w):
         assert np.max(np.abs(w[:, flat.index("vout")] - K.butterworth_exact(t))) < GOLD["butterworth"]["tol"]
 
 
+@pytest.mark.parametrize("kernel", [L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_GLOBAL])
 @pytest.mark.parametrize("case", TRAN_CASES, ids=[c[0] for c in TRAN_CASES])
-def test_tran_plain_reference_circuits(engine, case):
-    """tran! on the plain path (host step control, one hipGraph per Newton
-    iteration): identical steps to the oracle and the reference's answers."""
+def test_tran_plain_reference_circuits(engine, case, kernel):
+    """tran! in one launch (AUTO) and on the plain path (GLOBAL: host step
+    control, one hipGraph per Newton iteration): identical steps to the oracle
+    and the reference's answers."""
     name, flat, o, u0 = _tran_case(case)
-    _say(f"plain tran {name}")
+    o.batch_kernel = kernel
+    _say(f"plain tran {name}, kernel {kernel}")
     sol = engine.load(flat).tran(o, None, u0)
     w_ref, _, st_ref, rc = O.tran(flat, flat.params(), u0, o)
     assert sol.retcode == "Success" and rc == 0

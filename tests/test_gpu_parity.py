@@ -90,11 +90,13 @@ def test_dcop_inverter(engine):
     assert _rel_close(sol.u, u_ref, 1e-9, 1e-12)
 
 
-def test_tran_plain_inverter(engine):
-    """Config 0 over its whole span: the inverter, 0-20 ns, BDF2 at reltol 1e-6."""
-    _say("plain tran inverter 0-20ns")
+@pytest.mark.parametrize("kernel", [L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_GLOBAL])
+def test_tran_plain_inverter(engine, kernel):
+    """Config 0 over its whole span: the inverter, 0-20 ns, BDF2 at reltol 1e-6,
+    in one launch (AUTO) and on the plain path (GLOBAL)."""
+    _say(f"plain tran inverter 0-20ns, kernel {kernel}")
     flat = ch.lower(inverter())
-    opts = ch.grid_options((0.0, 20e-9), dt_out=10e-12)
+    opts = ch.grid_options((0.0, 20e-9), dt_out=10e-12, batch_kernel=kernel)
     sys = engine.load(flat)
     sol = sys.tran(opts)
     w_ref, uf_ref, st_ref, rc = O.tran(flat, flat.params(), None, opts)

@@ -61,13 +61,14 @@ def test_reuse_inverter_and_filter_plain(engine):
     fb = ch.lower(K.butterworth)
     sb = engine.load(fb, solver=L.SOLVER_LEVEL)
     u0 = np.zeros(fb.n)
-    ob = ch.grid_options((0.0, 4.0), n_out=41, init=L.INIT_UIC)
-    full = sb.tran(ob, u0=u0)
-    ob.jac_reuse = 1
-    mod = sb.tran(ob, u0=u0)
-    assert mod.retcode == "Success" and mod.stats.steps == full.stats.steps
-    assert mod.stats.newton_iters == full.stats.newton_iters
-    assert np.array_equal(np.asarray(mod.wave), np.asarray(full.wave))
+    for kernel in (L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_GLOBAL):   # the one launch, the plain path
+        ob = ch.grid_options((0.0, 4.0), n_out=41, init=L.INIT_UIC, batch_kernel=kernel)
+        full = sb.tran(ob, u0=u0)
+        ob.jac_reuse = 1
+        mod = sb.tran(ob, u0=u0)
+        assert mod.retcode == "Success" and mod.stats.steps == full.stats.steps
+        assert mod.stats.newton_iters == full.stats.newton_iters
+        assert np.array_equal(np.asarray(mod.wave), np.asarray(full.wave))
 
 
 def test_reuse_power_grid_supernodal(engine):

@@ -45,15 +45,17 @@ def test_spice_scopes_on_device(engine, name):
 def test_multimode_source_on_device(engine):
     """test/basic.jl:534-553: DC 5 with SIN(10 3 1k); the transient starts on
     the waveform (CedarDCOp's DC point, then the consistent start at t0) on
-    the plain path and both batched kernels."""
+    the one launch, the plain path and both batched kernels."""
     print("[gpu] spice multimode source", flush=True)
     flat = ch.lower(make_spice_circuit(DECKS["multimode_source"]["deck"]))
     o = ch.grid_options((0.0, 1e-3), n_out=21, reltol=1e-8, abstol=1e-10)
     w_ref, _, st_ref, rc = O.tran(flat, flat.params(), None, o)
     assert rc == 0 and w_ref[0, flat.index("node_vcc")] == pytest.approx(10.0)
-    sol = engine.load(flat).tran(o)
-    assert sol.retcode == "Success" and sol.stats.steps == st_ref.steps
-    assert np.allclose(sol.wave, w_ref, rtol=1e-6, atol=1e-9)
+    for kernel in (L.BATCH_KERNEL_AUTO, L.BATCH_KERNEL_GLOBAL):
+        o.batch_kernel = kernel
+        sol = engine.load(flat).tran(o)
+        assert sol.retcode == "Success" and sol.stats.steps == st_ref.steps
+        assert np.allclose(sol.wave, w_ref, rtol=1e-6, atol=1e-9)
     for kernel in (L.BATCH_KERNEL_LDS, L.BATCH_KERNEL_GLOBAL):
         o.batch_kernel = kernel
         r = ch.tran_batch([flat], [flat.params()], o, engine=engine)
