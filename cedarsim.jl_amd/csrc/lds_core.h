@@ -23,9 +23,9 @@
 // descriptors, pointers and index pairs took five), the next step's record
 // requested before the current step computes, and few register spills: with
 // the plan header's 44 words in scalar registers the packed kernel spilled
-// 233 scalar and 146 vector registers (now 133 and 0), and reloaded them
+// 233 scalar and 146 vector registers (now 147 and 0), and reloaded them
 // inside the iteration.  Instructions per iteration, averaged over that
-// batch, before and after: vector 1895 -> 995, scalar 1087 -> 470, LDS 359 ->
+// batch, before and after: vector 1895 -> 1093, scalar 1087 -> 531, LDS 359 ->
 // 218.
 //
 // Step control, predictor, local-error test and output interpolation follow
